@@ -621,6 +621,7 @@ struct fs_terrain {
     int32_t rows, cols, hbits;
     void *d_hq;            /* bilinear height quads */
     uint16_t *d_hp;        /* masked heights, one per texel */
+    uint32_t *d_hmax;      /* the largest of them, in parts (in d_hp's allocation) */
     uint32_t *d_color;     /* raw colour map */
     int32_t *h_alt;        /* host copy of the masked heights */
 };
@@ -681,7 +682,9 @@ static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_
     size_t n = (size_t)rows * (size_t)cols;
     size_t qbytes = n * (hbits == 8 ? 4 : 8);
     hipError_t e = hipMalloc(&t->d_hq, qbytes ? qbytes : 4);
-    if (e == hipSuccess) e = hipMalloc((void **)&t->d_hp, n ? n * 2 : 4);
+    const size_t hpbytes = (n * 2 + 15) & ~(size_t)15;
+    if (e == hipSuccess) e = hipMalloc((void **)&t->d_hp, hpbytes + FSK_HMAX_PARTS * 4);
+    t->d_hmax = (uint32_t *)((char *)t->d_hp + hpbytes);
     if (e == hipSuccess) e = hipMalloc((void **)&t->d_color, n ? n * 4 : 4);
     t->h_alt = (int32_t *)malloc(n ? n * 4 : 4);
     if (e != hipSuccess || !t->h_alt) {
@@ -692,7 +695,8 @@ static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_
     if (n) {
         e = hipMemcpyAsync(t->d_color, d_color_src, n * 4, hipMemcpyDeviceToDevice, ctx->stream);
         if (e == hipSuccess)
-            e = (hipError_t)fsk_height_quads(d_alt, rows, cols, hbits, t->d_hq, t->d_hp, ctx->stream);
+            e = (hipError_t)fsk_height_quads(d_alt, rows, cols, hbits, t->d_hq, t->d_hp,
+                                             t->d_hmax, ctx->stream);
         if (e == hipSuccess)
             e = hipMemcpyAsync(t->h_alt, d_alt, n * 4, hipMemcpyDeviceToHost, ctx->stream);
         if (e == hipSuccess)
@@ -747,8 +751,8 @@ static struct fs_shade *shade_new(struct futhark_context *ctx, const struct fs_t
         return NULL;
     }
     sun_vector(sun_height, sun_ang, s->sun);
-    e = (hipError_t)fsk_shade(t->d_hp, t->rows, t->cols, t->d_color, t->rows, t->cols,
-                              s->sun[0], s->sun[1], s->sun[2], size, s->d_shaded, ctx->stream);
+    e = (hipError_t)fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, t->d_color, s->sun, size,
+                              s->d_shaded, ctx->stream);
     if (e == hipSuccess)
         e = (hipError_t)fsk_color_quads(s->d_shaded, size, size, s->d_cq, ctx->stream);
     if (e != hipSuccess) {
@@ -1594,8 +1598,8 @@ int fsx_map_shade_factor(struct futhark_context *ctx, const struct fsx_map *map,
     const struct fs_terrain *t = map->t;
     const struct fs_shade *s = map->s;
     HIPCHECK(ctx, hipSetDevice(ctx->device));
-    HIPCHECK(ctx, fsk_shade_factor(t->d_hp, t->rows, t->cols, s->sun[0], s->sun[1], s->sun[2],
-                                   s->rows, dev_sf, ctx->stream));
+    HIPCHECK(ctx, fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, NULL, s->sun, s->rows, dev_sf,
+                            ctx->stream));
     return 0;
 }
 

@@ -116,13 +116,16 @@ int fsk_batch_run(const fsk_batch *b, hipStream_t s);
  * number of mismatching inputs to *d_bad. */
 int fsk_selftest(int which, unsigned long long *d_bad, hipStream_t s);
 
-/* Map preparation. */
+/* Map preparation.  fsk_height_quads also writes the map's largest masked
+ * height to d_hmax, as FSK_HMAX_PARTS values whose maximum it is.  fsk_shade evaluates the sun-ray counts of the size^2
+ * grid and writes the shaded colours of d_color (u32), or, with d_color
+ * NULL, the shade factors sqrt(1 / (4*count + 1)) (f32). */
+#define FSK_HMAX_PARTS 128
 int fsk_height_quads(const int32_t *d_alt, int32_t rows, int32_t cols, int32_t hbits,
-                     void *d_hq, uint16_t *d_hplain, hipStream_t s);
-int fsk_shade(const uint16_t *d_hplain, int32_t hrows, int32_t hcols,
-              const uint32_t *d_color, int32_t crows, int32_t ccols,
-              float sun0, float sun1, float sun2, int32_t size,
-              uint32_t *d_shaded, hipStream_t s);
+                     void *d_hq, uint16_t *d_hplain, uint32_t *d_hmax, hipStream_t s);
+int fsk_shade(const uint16_t *d_hplain, const uint32_t *d_hmax, int32_t rows, int32_t cols,
+              const uint32_t *d_color, const float sun[3], int32_t size, void *d_out,
+              hipStream_t s);
 int fsk_color_quads(const uint32_t *d_col, int32_t rows, int32_t cols, void *d_cq,
                     hipStream_t s);
 
@@ -173,8 +176,6 @@ int fsk_fill_u32(uint32_t *d_p, size_t n, uint32_t v, hipStream_t s);
  * to the scalar: no atomics on the scalar, reproducible results. */
 int fsk_l2_loss(const float *d_img, const float *d_tgt, size_t n, float *d_g, float *d_loss,
                 int32_t accumulate, float *d_partials, int32_t n_partials, hipStream_t s);
-int fsk_shade_factor(const uint16_t *d_hplain, int32_t hrows, int32_t hcols, float sun0,
-                     float sun1, float sun2, int32_t size, float *d_sf, hipStream_t s);
 
 #ifdef __cplusplus
 }

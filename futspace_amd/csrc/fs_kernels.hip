@@ -1339,28 +1339,76 @@ __global__ __launch_bounds__(256) void k_render2(Render2Args a)
 /* ------------------------------------------------------------------ */
 
 /* Ingest: `elem & mask` (fut/interactive.fut:189) and the bilinear quad
- * of each texel (right and lower neighbours wrap, as floor-mod does). */
+ * of each texel (right and lower neighbours wrap, as floor-mod does).  A
+ * thread holds kQuadRows rows of one column, so that a row's heights are
+ * read once and not again as the lower half of the row above, with all of
+ * its reads in flight together. */
+constexpr int kQuadRows = 4;
+
 template <int HBITS>
-__global__ void k_height_quads(const int32_t *__restrict__ alt, int32_t rows, int32_t cols,
-                               void *__restrict__ hq, uint16_t *__restrict__ hplain)
+__global__ __launch_bounds__(256) void k_height_quads(const int32_t *__restrict__ alt,
+                                                      int32_t rows, int32_t cols,
+                                                      void *__restrict__ hq,
+                                                      uint16_t *__restrict__ hplain)
 {
-    int32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t y = blockIdx.y;
+    const int32_t x = blockIdx.x * 256 + threadIdx.x;
+    const int32_t y0 = blockIdx.y * kQuadRows;
     if (x >= cols)
         return;
     const uint32_t mk = HBITS == 8 ? 0xFFu : 0xFFFFu;
-    int32_t x1 = x + 1 == cols ? 0 : x + 1;
-    int32_t y1 = y + 1 == rows ? 0 : y + 1;
-    uint32_t h00 = (uint32_t)alt[(size_t)y * cols + x] & mk;
-    uint32_t h01 = (uint32_t)alt[(size_t)y * cols + x1] & mk;
-    uint32_t h10 = (uint32_t)alt[(size_t)y1 * cols + x] & mk;
-    uint32_t h11 = (uint32_t)alt[(size_t)y1 * cols + x1] & mk;
-    size_t t = (size_t)y * cols + x;
-    if (HBITS == 8)
-        ((uint32_t *)hq)[t] = h00 | (h01 << 8) | (h10 << 16) | (h11 << 24);
-    else
-        ((uint2 *)hq)[t] = make_uint2(h00 | (h01 << 16), h10 | (h11 << 16));
-    hplain[t] = (uint16_t)h00;
+    const int32_t x1 = x + 1 == cols ? 0 : x + 1;
+    uint32_t h0[kQuadRows + 1], h1[kQuadRows + 1];
+#pragma unroll
+    for (int j = 0; j <= kQuadRows; j++) {
+        /* row `rows` is row 0; rows past it are not used */
+        const int32_t y = y0 + j < rows ? y0 + j : 0;
+        h0[j] = (uint32_t)alt[(size_t)y * cols + x] & mk;
+        h1[j] = (uint32_t)alt[(size_t)y * cols + x1] & mk;
+    }
+#pragma unroll
+    for (int j = 0; j < kQuadRows; j++) {
+        if (y0 + j >= rows)
+            break;
+        const size_t t = (size_t)(y0 + j) * cols + x;
+        if (HBITS == 8)
+            ((uint32_t *)hq)[t] = h0[j] | (h1[j] << 8) | (h0[j + 1] << 16) | (h1[j + 1] << 24);
+        else
+            ((uint2 *)hq)[t] = make_uint2(h0[j] | (h1[j] << 16), h0[j + 1] | (h1[j + 1] << 16));
+        hplain[t] = (uint16_t)h0[j];
+    }
+}
+
+/* The largest of n heights (16-byte aligned) as one value per workgroup in
+ * hmax[FSK_HMAX_PARTS]: a pass of its own, since one atomic maximum per
+ * workgroup of k_height_quads took longer than reading the heights again
+ * (2048^2: 12 against 4 us). */
+__global__ __launch_bounds__(1024) void k_height_max(const uint16_t *__restrict__ hp, size_t n,
+                                                     uint32_t *__restrict__ hmax)
+{
+    const size_t first = (size_t)blockIdx.x * 1024 + threadIdx.x;
+    const size_t stride = (size_t)gridDim.x * 1024, n8 = n / 8;
+    uint32_t top = 0u;
+    for (size_t i = first; i < n8; i += stride) {
+        const uint4 v = ((const uint4 *)hp)[i];
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            top = max(top, max(w[j] & 0xFFFFu, w[j] >> 16));
+    }
+    for (size_t i = n8 * 8 + first; i < n; i += stride)
+        top = max(top, (uint32_t)hp[i]);
+    __shared__ uint32_t wtop[16];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+        top = max(top, (uint32_t)__shfl_xor((int)top, off));
+    if ((threadIdx.x & 63) == 0)
+        wtop[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++)
+            top = max(top, wtop[w]);
+        hmax[blockIdx.x] = top;
+    }
 }
 
 __global__ void k_color_quads(const uint32_t *__restrict__ c, int32_t rows, int32_t cols,
@@ -1379,31 +1427,122 @@ __global__ void k_color_quads(const uint32_t *__restrict__ c, int32_t rows, int3
 /* generate_shadowmap_accumulated, fut/effects.fut:108-125: for each
  * texel of the size^2 grid count the 255 sun-ray steps that pass below
  * the terrain by more than half a unit (nearest `png_height`,
- * fut/render_functions.fut:63-64), then darken with argb.mix. */
-__global__ void k_shade(const uint16_t *__restrict__ hp, int32_t hrows, int32_t hcols,
-                        const uint32_t *__restrict__ col, int32_t crows, int32_t ccols,
-                        float s0, float s1, float s2, int32_t size, uint32_t *__restrict__ out)
+ * fut/render_functions.fut:63-64), then darken with argb.mix -- or, for the
+ * differentiable renderer, write the shade factor sqrt(1 / (4*count + 1)).
+ *
+ * The steps' offsets t * sun (t = 4 * dist) are the same for every texel:
+ * the host forms them once (the same f32 products) and they arrive as
+ * kernel arguments, i.e. in scalar registers.  A wave holds kShadeTexels
+ * runs of 64 texels of one row, so a step's map row is one scalar too, and
+ * a texel's step is nine vector instructions and a coalesced 2-byte load.
+ * Under a sun above the horizon the ray climbs: (height + t * s1) - probe is
+ * non-decreasing in t for a fixed probe, also in f32, so once it is at least
+ * -0.5 against the map's largest height no later step can count, and the
+ * wave leaves when that holds for its lowest texel (at sun height 0.1
+ * after at most 64 of the 255 steps on an 8-bit map).  Measured, sun height
+ * 0.1: 1024^2 grid 338 -> 25 us; 4096^2 grid, heights to 1024 (nearly every
+ * step) 4.79 -> 0.64 ms, where the vector instructions bound it; before,
+ * one texel per thread took every step with two general floor-mods. */
+constexpr int kShadeSteps = 256;      /* dist = 1 .. 255 */
+constexpr int kShadeTexels = 4;       /* texels per thread, 64 apart in x */
+constexpr int kShadeGroup = 5;        /* steps between exit tests; 255 = 51 * 5 */
+
+struct ShadeArgs {
+    const uint16_t *hp;
+    const uint32_t *hmax;             /* the map's largest height: k_height_max's parts */
+    const uint32_t *col;              /* raw colours (not read for the shade factor) */
+    void *out;
+    int32_t hrows, hcols, size;
+    float rrows, rcols;               /* 1 / hrows, 1 / hcols */
+    /* t * s0, t * s1, t * s2 of step dist at [dist] */
+    float dx[kShadeSteps], dh[kShadeSteps], dy[kShadeSteps];
+};
+static_assert(sizeof(ShadeArgs) <= 4096, "kernel argument size");
+
+/* Floor-mod of a map coordinate.  kWrapPow2: a mask.  kWrapSmall: any side
+ * m <= 2^16 and |v| < 2^22: v / m in f32 is within 2^-22 relative of the
+ * quotient, which is below 2^22, so its floor is the integer quotient or
+ * one off, and one correction either way gives the remainder.  kWrapX86:
+ * every i32. */
+enum { kWrapPow2 = 0, kWrapSmall = 1, kWrapX86 = 2 };
+
+template <int WRAP>
+__device__ __forceinline__ int32_t wrap_map(int32_t v, int32_t m, float rm)
 {
-    int32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t y = blockIdx.y;
-    if (x >= size)
+    if (WRAP == kWrapPow2)
+        return v & (m - 1);
+    if (WRAP == kWrapX86)
+        return fmod_i32(v, m);
+    int32_t r = v - (int32_t)floorf((float)v * rm) * m;
+    r = r < 0 ? r + m : r;
+    return r >= m ? r - m : r;
+}
+
+/* WRAP kWrapX86 is for sun vectors that are not finite, whose probes take
+ * the x86 cast's INT_MIN; a finite sun's offsets are at most 1020. */
+template <int WRAP, bool FACTOR>
+__global__ __launch_bounds__(256) void k_shade(ShadeArgs a)
+{
+    const int32_t lane = threadIdx.x & 63;
+    const int32_t y = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + (threadIdx.x >> 6));
+    const int32_t x0 = blockIdx.x * (64 * kShadeTexels) + lane;
+    if (y >= a.size)
         return;
-    const float step_size = 4.0f;
-    float fx = (float)x, fy = (float)y;
-    float height = (float)hp[(size_t)fmod_i32(y, hrows) * hcols + fmod_i32(x, hcols)];
-    int32_t count = 0;
-    for (int32_t dist = 1; dist < 256; dist++) {
-        float t = (float)dist * step_size;
-        float px = fx + (t * s0);
-        float py = fy + (t * s2);
-        int32_t ix = fmod_i32(i32_f32_x86(px), hcols);
-        int32_t iy = fmod_i32(i32_f32_x86(py), hrows);
-        float probe = (float)hp[(size_t)iy * hcols + ix];
-        count += (((height + (t * s1)) - probe) < -0.5f) ? 1 : 0;
+    const size_t row = (size_t)wrap_map<WRAP>(y, a.hrows, a.rrows) * (size_t)a.hcols;
+    static_assert(FSK_HMAX_PARTS == 128, "two parts per lane");
+    float hmax = (float)max(a.hmax[lane], a.hmax[lane + 64]);
+    const float fy = (float)y;
+    float fx[kShadeTexels], height[kShadeTexels], low = 65536.0f;
+    int32_t count[kShadeTexels];
+#pragma unroll
+    for (int u = 0; u < kShadeTexels; u++) {
+        const int32_t x = x0 + 64 * u;
+        fx[u] = (float)x;
+        height[u] = (float)a.hp[row + (size_t)wrap_map<WRAP>(x, a.hcols, a.rcols)];
+        low = fminf(low, x < a.size ? height[u] : low);
+        count[u] = 0;
     }
-    float amount = (float)count;
-    uint32_t c = col[(size_t)fmod_i32(y, crows) * ccols + fmod_i32(x, ccols)];
-    out[(size_t)y * size + x] = argb_mix(step_size * amount, 0xFF000000u, 1.0f, c);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        low = fminf(low, __shfl_xor(low, off));
+        hmax = fmaxf(hmax, __shfl_xor(hmax, off));
+    }
+    const bool rises = a.dh[1] >= 0.0f;
+    for (int32_t d0 = 1; d0 < kShadeSteps; d0 += kShadeGroup) {
+        /* uniform over the wave: low and the step's values are */
+        if (rises && ((low + a.dh[d0]) - hmax) >= -0.5f)
+            break;
+#pragma unroll
+        for (int j = 0; j < kShadeGroup; j++) {
+            const int32_t d = d0 + j;
+            auto texel = [](float v) { return WRAP == kWrapX86 ? i32_f32_x86(v) : (int32_t)v; };
+            const int32_t iy = __builtin_amdgcn_readfirstlane(
+                wrap_map<WRAP>(texel(fy + a.dy[d]), a.hrows, a.rrows));
+            const FS_GLOBAL char *hrow =
+                (const FS_GLOBAL char *)(a.hp + (size_t)iy * (size_t)a.hcols);
+#pragma unroll
+            for (int u = 0; u < kShadeTexels; u++) {
+                const uint32_t ix =
+                    (uint32_t)wrap_map<WRAP>(texel(fx[u] + a.dx[d]), a.hcols, a.rcols);
+                const float probe = (float)*(const FS_GLOBAL uint16_t *)(hrow + ix * 2u);
+                count[u] += (((height[u] + a.dh[d]) - probe) < -0.5f) ? 1 : 0;
+            }
+        }
+    }
+    const float step_size = 4.0f;
+#pragma unroll
+    for (int u = 0; u < kShadeTexels; u++) {
+        const int32_t x = x0 + 64 * u;
+        if (x >= a.size)
+            continue;
+        const float amount = (float)count[u];
+        const size_t t = (size_t)y * (size_t)a.size + (size_t)x;
+        if (FACTOR)
+            ((float *)a.out)[t] = __builtin_sqrtf(1.0f / ((step_size * amount) + 1.0f));
+        else
+            ((uint32_t *)a.out)[t] = argb_mix(step_size * amount, 0xFF000000u, 1.0f,
+                                              a.col[row + (size_t)wrap_map<WRAP>(x, a.hcols, a.rcols)]);
+    }
 }
 
 /* ------------------------------------------------------------------ */
@@ -2556,31 +2695,6 @@ __global__ void k_zero_f32(float *__restrict__ p, size_t n)
         p[i] = 0.0f;
 }
 
-/* Shade factor of the relaxation: the same sun-ray count as k_shade,
- * then sf = sqrt(1 / (4*count + 1)). */
-__global__ void k_shade_factor(const uint16_t *__restrict__ hp, int32_t hrows, int32_t hcols,
-                               float s0, float s1, float s2, int32_t size, float *__restrict__ sf)
-{
-    int32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t y = blockIdx.y;
-    if (x >= size)
-        return;
-    const float step_size = 4.0f;
-    float fx = (float)x, fy = (float)y;
-    float height = (float)hp[(size_t)fmod_i32(y, hrows) * hcols + fmod_i32(x, hcols)];
-    int32_t count = 0;
-    for (int32_t dist = 1; dist < 256; dist++) {
-        float t = (float)dist * step_size;
-        float px = fx + (t * s0);
-        float py = fy + (t * s2);
-        int32_t ix = fmod_i32(i32_f32_x86(px), hcols);
-        int32_t iy = fmod_i32(i32_f32_x86(py), hrows);
-        float probe = (float)hp[(size_t)iy * hcols + ix];
-        count += (((height + (t * s1)) - probe) < -0.5f) ? 1 : 0;
-    }
-    sf[(size_t)y * size + x] = __builtin_sqrtf(1.0f / ((step_size * (float)count) + 1.0f));
-}
-
 inline bool pow2(int32_t v)
 {
     return v > 0 && (v & (v - 1)) == 0;
@@ -2929,15 +3043,6 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
     return hipGetLastError();
 }
 
-int fsk_shade_factor(const uint16_t *d_hplain, int32_t hrows, int32_t hcols, float sun0,
-                     float sun1, float sun2, int32_t size, float *d_sf, hipStream_t s)
-{
-    dim3 grid((size + 255) / 256, size);
-    hipLaunchKernelGGL(k_shade_factor, grid, dim3(256), 0, s, d_hplain, hrows, hcols, sun0, sun1,
-                       sun2, size, d_sf);
-    return hipGetLastError();
-}
-
 int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const float *d_sn,
                 const uint32_t *d_color, int32_t n, uint32_t *d_out, int64_t pitch, hipStream_t s)
 {
@@ -3055,24 +3160,53 @@ int fsk_render(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t, uint32
 }
 
 int fsk_height_quads(const int32_t *d_alt, int32_t rows, int32_t cols, int32_t hbits,
-                     void *d_hq, uint16_t *d_hplain, hipStream_t s)
+                     void *d_hq, uint16_t *d_hplain, uint32_t *d_hmax, hipStream_t s)
 {
-    dim3 grid((cols + 255) / 256, rows);
-    if (hbits == 8)
-        hipLaunchKernelGGL(k_height_quads<8>, grid, dim3(256), 0, s, d_alt, rows, cols, d_hq, d_hplain);
-    else
-        hipLaunchKernelGGL(k_height_quads<16>, grid, dim3(256), 0, s, d_alt, rows, cols, d_hq, d_hplain);
+    dim3 grid((cols + 255) / 256, (rows + kQuadRows - 1) / kQuadRows);
+    void (*kern)(const int32_t *, int32_t, int32_t, void *, uint16_t *) =
+        hbits == 8 ? k_height_quads<8> : k_height_quads<16>;
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, d_alt, rows, cols, d_hq, d_hplain);
+    hipLaunchKernelGGL(k_height_max, dim3(FSK_HMAX_PARTS), dim3(1024), 0, s, d_hplain,
+                       (size_t)rows * (size_t)cols, d_hmax);
     return hipGetLastError();
 }
 
-int fsk_shade(const uint16_t *d_hplain, int32_t hrows, int32_t hcols,
-              const uint32_t *d_color, int32_t crows, int32_t ccols,
-              float sun0, float sun1, float sun2, int32_t size,
-              uint32_t *d_shaded, hipStream_t s)
+int fsk_shade(const uint16_t *d_hplain, const uint32_t *d_hmax, int32_t rows, int32_t cols,
+              const uint32_t *d_color, const float sun[3], int32_t size, void *d_out,
+              hipStream_t s)
 {
-    dim3 grid((size + 255) / 256, size);
-    hipLaunchKernelGGL(k_shade, grid, dim3(256), 0, s, d_hplain, hrows, hcols, d_color, crows,
-                       ccols, sun0, sun1, sun2, size, d_shaded);
+    ShadeArgs a;
+    a.hp = d_hplain;
+    a.hmax = d_hmax;
+    a.col = d_color;
+    a.out = d_out;
+    a.hrows = rows;
+    a.hcols = cols;
+    a.size = size;
+    a.rrows = 1.0f / (float)rows;
+    a.rcols = 1.0f / (float)cols;
+    const float step_size = 4.0f;
+    for (int32_t d = 0; d < kShadeSteps; d++) {
+        const float t = (float)d * step_size;
+        a.dx[d] = t * sun[0];
+        a.dh[d] = t * sun[1];
+        a.dy[d] = t * sun[2];
+    }
+    /* kWrapSmall's range: sides and grid up to 2^16 and offsets up to 1020 */
+    const bool finite = std::isfinite(sun[0]) && std::isfinite(sun[1]) && std::isfinite(sun[2]) &&
+                        std::fabs(sun[0]) <= 1.5f && std::fabs(sun[2]) <= 1.5f;
+    const bool small = rows <= 65536 && cols <= 65536 && size <= 65536;
+    const int w = !(finite && small) ? kWrapX86
+                  : pow2(rows) && pow2(cols) ? kWrapPow2 : kWrapSmall;
+    void (*kern)(ShadeArgs);
+    if (d_color)
+        kern = w == kWrapPow2 ? k_shade<kWrapPow2, false>
+               : w == kWrapSmall ? k_shade<kWrapSmall, false> : k_shade<kWrapX86, false>;
+    else
+        kern = w == kWrapPow2 ? k_shade<kWrapPow2, true>
+               : w == kWrapSmall ? k_shade<kWrapSmall, true> : k_shade<kWrapX86, true>;
+    dim3 grid((size + 64 * kShadeTexels - 1) / (64 * kShadeTexels), (size + 3) / 4);
+    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

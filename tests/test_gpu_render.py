@@ -267,3 +267,30 @@ def test_tuning_belongs_to_its_context(ctx):
     finally:
         c2.close()
     assert ctx.tuning() == base
+
+
+@pytest.mark.parametrize("rows,cols,size,bits,sun_h,sun_a", [
+    (1, 1, 65, 8, 0.1, 0.1),                     # one texel: every probe wraps to it
+    (3, 300, 257, 8, 1.5, 0.3),                  # a low sun over a few rows: every step
+    (257, 129, 300, 16, 1.2, -2.5),              # heights above 255, odd sides
+    (64, 256, 256, 16, 0.4, 3.0),                # powers of two, rows != columns
+    (100, 90, 1, 8, 2.5, 0.7),                   # one grid texel, the sun below
+    (128, 128, 130, 8, 0.3, float("inf")),       # probes with no place: the casts' INT_MIN
+    (100, 90, 130, 8, 0.3, float("nan")),
+])
+def test_shade_wraps_and_exits(ctx, rows, cols, size, bits, sun_h, sun_a):
+    """Shaded colours and shade factors at the edges of the shadow pass: map
+    sides against grid sides, steps that end early and that do not."""
+    import torch
+
+    from futspace_amd.diff import DiffRenderer
+    rng = np.random.default_rng(rows * 7 + cols)
+    col = rng.integers(0, 1 << 32, (rows, cols), dtype=np.uint32)
+    hts = rng.integers(0, 256 if bits == 8 else 700, (rows, cols)).astype(np.int32)
+    m = ctx.map(col, hts, height_bits=bits, shade_size=size, sun_height=sun_h, sun_ang=sun_a)
+    shaded, alt = O.update_map(col, hts, sun_h, sun_a, size=size, bits=bits)
+    _check(m.shaded(), shaded)
+    sf = DiffRenderer(ctx, m).sf
+    torch.cuda.synchronize()
+    want = O.shade_factor(O.shadow_counts(alt, O.sun(sun_h, sun_a), size))
+    assert np.array_equal(sf.cpu().numpy().view(np.uint32), want.view(np.uint32))
