@@ -374,9 +374,11 @@ constexpr uint32_t kQRowBits = 13;
 constexpr uint32_t kQRowMask = (1u << kQRowBits) - 1u;
 constexpr uint32_t kQColShift = 13, kQSliceShift = 17, kQGroupShift = 22;
 constexpr uint32_t kQLaneMask = (0xFFu << kQGroupShift) | (15u << kQColShift);  /* g and c */
-/* Frames up to kMaxRows rows: the row fields allow 8191, and a 4-column
- * tile of that height still fits in LDS. */
+/* Frames up to kMaxRows rows are rendered whole columns at a time: the row
+ * fields allow 8191, and a 4-column tile of that height still fits in LDS.
+ * Taller ones, up to kMaxFrameRows, are rendered in bands of rows. */
 constexpr int kMaxRows = 7680;
+constexpr int kMaxFrameRows = 1 << 22;
 constexpr int kChunkAlign = 4;                   /* chunks are multiples of SG * kChunkAlign */
 
 /* blockIdx -> column tile.  Workgroups are dispatched round-robin over
@@ -397,6 +399,7 @@ struct RenderArgs {
     int64_t pitch;
     int32_t ntiles;
     int32_t chunk_max;     /* slices per chunk, at most kChunk */
+    int32_t band_rows;     /* banded renders: rows per workgroup */
     /* slice mode: workgroups ntiles .. ntiles + nzero - 1 clear zero[zero_n4]
      * (the fused step's gradient) on CUs the tiles leave idle */
     float4 *zero;
@@ -719,14 +722,74 @@ __device__ __forceinline__ uint32_t nearest_index(const fsk_map &m, float x, flo
     return (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
 }
 
+/* What the fill shows at row `row0` of a column whose nearest sample at or
+ * above that row is transparent: the first opaque one beyond it, as a stripe
+ * value (0: none, sky).  The visible samples are the strict running minima
+ * of the projected rows over the whole depth range; a wave projects 64
+ * slices at a time.  Every lane of the wave must call it. */
+template <int HBITS, bool HP2, bool CP2, int MODE>
+__device__ uint32_t column_above(const fsk_map &m, const fsk_frame &f, int32_t col, int32_t row0,
+                                 const float *sq)
+{
+    const int32_t lane = threadIdx.x & 63;
+    const float Hf = (float)f.rows, fcol = (float)col;
+    int32_t run = f.rows;
+    for (int32_t base = 0; base < f.n && run > 0; base += 64) {
+        const int32_t k = base + lane;
+        const Slice sl = slice_params(f, min(k, f.n - 1));
+        const float x = sl.sx + (fcol * sl.dx);
+        const float y = sl.sy + (fcol * sl.dy);
+        float hgt;
+        if (MODE == kOutNearest)
+            hgt = (float)((const int32_t *)m.hq)[nearest_index<HP2>(m, x, y)];
+        else
+            hgt = height_interp<HBITS>(height_quad<HBITS, HP2>(m, x, y), x, y);
+        const float rel = ((f.cam_h - hgt) * sl.iz) + f.horizon;
+        const int32_t r = k < f.n ? screen_row_clamped(rel, Hf) : f.rows;
+        int32_t v = r;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int32_t o = __shfl_up(v, off);
+            if (lane >= off)
+                v = min(v, o);
+        }
+        const int32_t before = __shfl_up(v, 1);
+        const bool visible = r < (lane == 0 ? run : min(run, before));
+        uint32_t c = 0u;
+        if (visible && r <= row0) {
+            if (MODE == kOutColour)
+                c = color_of_quad(color_quad<CP2>(m, x, y), sq, x, y);
+            else if (MODE == kOutNearest)
+                c = ((const uint32_t *)m.cq)[nearest_index<HP2>(m, x, y)] ^ f.sky;
+            else
+                c = (floorf(x) == ceilf(x) || floorf(y) == ceilf(y)) ? 0u : (uint32_t)(k + 1);
+        }
+        const uint64_t opaque = __ballot(c != 0u);
+        if (opaque)
+            return (uint32_t)__builtin_amdgcn_readlane((int)c, __builtin_ctzll(opaque));
+        run = min(run, __builtin_amdgcn_readlane(v, 63));
+    }
+    return 0u;
+}
+
 /* chunk_max must be a multiple of NT/TC (the slice groups) and at most
- * CMAX; the LDS layout is sized for it. */
+ * CMAX; the LDS layout is sized for it.
+ *
+ * BAND: the tile covers rows row0 .. row0 + H - 1 of the frame only (out
+ * points at row0), H = min(band_rows, f.rows - row0).  Rows are then counted
+ * from row0 and clamped to [0, H]: a sample at or below the band is not
+ * visible in it, and of those above it only the nearest is, at row 0, from
+ * where it covers the band down to the next nearer one -- just what the
+ * whole column shows there.  Should that sample be transparent, the rows it
+ * covers show the next opaque one above, which column_above finds. */
 template <int TC, int NT, int CMAX, int HBITS, bool HP2, bool CP2, int MODE = kOutColour,
-          int GATHER = kGather, int CBATCH = kColourBatch, class Tables = NoTables>
+          int GATHER = kGather, int CBATCH = kColourBatch, class Tables = NoTables,
+          bool BAND = false>
 __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f, uint32_t *out,
                                             int64_t pitch, int32_t tile, int32_t chunk_max,
                                             uint32_t *lds, TileShared<TC> &sh,
-                                            const Tables &tables = Tables())
+                                            const Tables &tables = Tables(), int32_t row0 = 0,
+                                            int32_t band_rows = 0)
 {
     constexpr int NW = NT / 64;                  /* waves */
     constexpr int SG = NT / TC;                  /* slice groups */
@@ -737,7 +800,7 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
     const int32_t tabs = tab_stride(chunk_max);
     float4 *tl = (float4 *)lds;                                  /* [tabs] */
     float *tz = (float *)(lds + 4 * tabs);                       /* [tabs] */
-    const int32_t H = f.rows, n = f.n;
+    const int32_t H = BAND ? min(band_rows, f.rows - row0) : f.rows, n = f.n;
     const int32_t Hp = (H + 3) & ~3;
     uint32_t *stripe = lds + 5 * tabs;                           /* [TC][Hp] */
     const int32_t qcap = TC * min(H, chunk_max);                 /* visible rows differ */
@@ -751,7 +814,9 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
     const int32_t col = col0 + c;
     const bool colok = col < f.cols;
     const float fcol = (float)col;
-    const float Hf = (float)H;
+    /* the rows' clamp; frame rows are below 2^24, so exact */
+    const float topf = BAND ? (float)row0 : 0.0f;
+    const float Hf = BAND ? (float)(row0 + H) : (float)H;
 
     /* The stripe is not cleared: the spans of a column's visible samples
      * tile the rows from its final y-buffer down to H (transparent samples
@@ -852,8 +917,10 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                     float rel = ((f.cam_h - hgt) * izs[u]) + f.horizon;
                     /* a tame frame keeps |rel| < 2^30: the cast of the
                      * clamped value is the whole x86 semantics */
-                    int32_t r = TAME ? (int32_t)__builtin_amdgcn_fmed3f(rel, 0.0f, Hf)
-                                     : screen_row_clamped(rel, Hf);
+                    int32_t r = TAME || BAND ? (int32_t)__builtin_amdgcn_fmed3f(rel, topf, Hf)
+                                             : screen_row_clamped(rel, Hf);
+                    if (BAND)
+                        r = TAME || rel < 2147483648.0f ? r - row0 : 0;
                     if (j & 1)
                         ah[j / 2] |= (uint32_t)r << 16;
                     else
@@ -1109,6 +1176,7 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
     }
     uint32_t *wfill = (uint32_t *)&sh.wtot[0][0];      /* [NW][TC] */
     uint32_t *wfpre = (uint32_t *)&sh.wpre[0][0];
+    uint32_t *top = lds;                               /* [TC]; the slice table is done */
 #pragma unroll
     for (int j = 0; j < TC; j++) {
         uint32_t v = pre[j];
@@ -1140,10 +1208,25 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                 wfpre[(lane >> 2) * TC + cc] = lane < 4 ? 0u : ex;
         }
     }
+    if (BAND && row0 > 0) {
+        /* a column that a transparent sample above the band covers from its
+         * first row on: wave j finds what shows through in column j */
+        static_assert(TC <= NW, "a wave per column");
+        if (wave < TC && col0 + wave < f.cols && sh.carry[wave] == 0 && stripe[wave * Hp] == 0u) {
+            const uint32_t above =
+                column_above<HBITS, HP2, CP2, MODE>(m, f, col0 + wave, row0, sh.sq);
+            if (lane == 0)
+                top[wave] = above;
+        } else if (wave < TC && lane == 0) {
+            top[wave] = 0u;
+        }
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < TC; j++) {
         uint32_t p = wfpre[wave * TC + j];
+        if (BAND && row0 > 0)
+            p = p ? p : top[j];
         pre[j] = pre[j] ? pre[j] : p;
     }
     /* written twice for the same reason as the loop above */
@@ -1176,12 +1259,13 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
         rows(std::false_type{});
 }
 
-template <int TC, int NT, int CMAX, int HBITS, bool HP2, bool CP2, int WPE, int MODE>
+template <int TC, int NT, int CMAX, int HBITS, bool HP2, bool CP2, int WPE, int MODE,
+          bool BAND = false>
 __global__ __launch_bounds__(NT, WPE) void k_render(RenderArgs a)
 {
     extern __shared__ __align__(16) uint32_t lds[];  /* float4 slice table at its start */
     __shared__ TileShared<TC> sh;
-    if constexpr (MODE == kOutSlice) {
+    if constexpr (MODE == kOutSlice && !BAND) {
         if ((int32_t)blockIdx.x >= a.ntiles) {
             const size_t stride = (size_t)a.nzero * NT;
             for (size_t i = (size_t)(blockIdx.x - a.ntiles) * NT + threadIdx.x; i < a.zero_n4;
@@ -1190,90 +1274,18 @@ __global__ __launch_bounds__(NT, WPE) void k_render(RenderArgs a)
             return;
         }
     }
+    const int32_t tile = xcd_tile(blockIdx.x, a.ntiles);
+    const int32_t row0 = BAND ? (int32_t)blockIdx.y * a.band_rows : 0;
+    uint32_t *out = BAND ? a.out + (size_t)row0 * (size_t)a.pitch : a.out;
     if constexpr (MODE == kOutColour) {
         TileTables<TC, NT> tables;
         tables.load(threadIdx.x);
         render_tile<TC, NT, CMAX, HBITS, HP2, CP2, MODE, kGather, kColourBatch,
-                    TileTables<TC, NT>>(a.m, a.f, a.out, a.pitch, xcd_tile(blockIdx.x, a.ntiles),
-                                        a.chunk_max, lds, sh, tables);
+                    TileTables<TC, NT>, BAND>(a.m, a.f, out, a.pitch, tile, a.chunk_max, lds, sh,
+                                              tables, row0, a.band_rows);
     } else {
-        render_tile<TC, NT, CMAX, HBITS, HP2, CP2, MODE>(a.m, a.f, a.out, a.pitch,
-                                                         xcd_tile(blockIdx.x, a.ntiles),
-                                                         a.chunk_max, lds, sh);
-    }
-}
-
-/* Frames taller than the tile's kMaxRows: one thread per column walks the
- * slices front to back and paints each visible sample's span straight into
- * the frame (the reference's scan occlude, scatter and fill_vline,
- * fut/voxel_renderer.fut:231-249, seen from the sample's side, as the tile
- * does), then writes the sky above the final y-buffer and, if a
- * transparent sample occurred, fills the column top-down.  Slow -- one
- * thread per column, spans stored one cell at a time -- but without a row
- * limit.  Cells of transparent samples hold the mode's `empty` value until
- * the fill: 0 in colour mode (a frame colour is never 0), the sky in the
- * stateless program's mode (its fill's own test), 0xFFFFFFFE in slice
- * mode (a slice index or -1 otherwise). */
-constexpr int kMaxFrameRows = 1 << 22;
-
-template <int HBITS, bool HP2, bool CP2, int MODE>
-__global__ __launch_bounds__(64) void k_render_column(RenderArgs a)
-{
-    __shared__ float sq[256];
-    if (MODE == kOutColour) {
-        for (int32_t i = threadIdx.x; i < 256; i += 64)
-            fill_square_lut(sq, i);
-        __syncthreads();
-    }
-    const fsk_frame &f = a.f;
-    const fsk_map &m = a.m;
-    const int32_t col = blockIdx.x * 64 + threadIdx.x;
-    if (col >= f.cols)
-        return;
-    const int32_t H = f.rows;
-    const float Hf = (float)H, fcol = (float)col;
-    const uint32_t sky = MODE == kOutSlice ? 0xFFFFFFFFu : f.sky;
-    const uint32_t empty = MODE == kOutColour ? 0u : (MODE == kOutNearest ? f.sky : 0xFFFFFFFEu);
-    uint32_t *dst = a.out + col;
-    const size_t pitch = (size_t)a.pitch;
-    int32_t ybuf = H;
-    bool transp = false;
-    for (int32_t k = 0; k < f.n && ybuf > 0; k++) {
-        const Slice sl = slice_params(f, k);
-        const float x = sl.sx + (fcol * sl.dx);
-        const float y = sl.sy + (fcol * sl.dy);
-        float hgt;
-        if (MODE == kOutNearest)
-            hgt = (float)((const int32_t *)m.hq)[nearest_index<HP2>(m, x, y)];
-        else
-            hgt = height_interp<HBITS>(height_quad<HBITS, HP2>(m, x, y), x, y);
-        const float rel = ((f.cam_h - hgt) * sl.iz) + f.horizon;
-        const int32_t r = screen_row_clamped(rel, Hf);
-        if (r >= ybuf)
-            continue;
-        uint32_t v;
-        if (MODE == kOutColour)
-            v = color_of_quad(color_quad<CP2>(m, x, y), sq, x, y);
-        else if (MODE == kOutNearest)
-            v = ((const uint32_t *)m.cq)[nearest_index<HP2>(m, x, y)];
-        else
-            v = (floorf(x) == ceilf(x) || floorf(y) == ceilf(y)) ? empty : (uint32_t)k;
-        transp = transp || v == empty;
-        for (int32_t rr = r; rr < ybuf; rr++)
-            dst[(size_t)rr * pitch] = v;
-        ybuf = r;
-    }
-    for (int32_t rr = 0; rr < ybuf; rr++)
-        dst[(size_t)rr * pitch] = sky;
-    if (transp) {
-        uint32_t last = sky;
-        for (int32_t rr = 0; rr < H; rr++) {
-            const uint32_t v = dst[(size_t)rr * pitch];
-            if (v == empty)
-                dst[(size_t)rr * pitch] = last;
-            else
-                last = v;
-        }
+        render_tile<TC, NT, CMAX, HBITS, HP2, CP2, MODE, kGather, kColourBatch, NoTables, BAND>(
+            a.m, a.f, out, a.pitch, tile, a.chunk_max, lds, sh, NoTables(), row0, a.band_rows);
     }
 }
 
@@ -1785,19 +1797,52 @@ inline Shape resolve_shape(int32_t rows, const fsk_tuning &t)
     return s;
 }
 
+/* Frames of more than kMaxRows rows: 8-column tiles over bands of rows, each
+ * as tall as its stripe fits in LDS beside chunks of at most kBandChunk
+ * slices (half the whole-column tile's, for 1000 more rows a band).  A band
+ * repeats its columns' projection, about 8 us per tile, and stores its rows
+ * at the tile kernel's rate.  Measured on the stateless program's 800-column
+ * frames: 10^4 rows 306 -> 23 us, 10^5 rows 3.04 -> 0.13 ms (2.4 TB/s of
+ * stores), 10^6 rows 30.3 -> 1.39 ms, against one thread per column walking
+ * the slices and storing its spans cell by cell. */
+constexpr int kBandChunk = 1024;
+
+template <int HBITS, bool HP2, bool CP2, int MODE>
+hipError_t launch_bands(RenderArgs a, hipStream_t s)
+{
+    constexpr int TC = 8, NT = 1024, kGroups = NT / TC * kChunkAlign;
+    if (a.f.rows > kMaxFrameRows)
+        return hipErrorInvalidValue;
+    auto kern = k_render<TC, NT, kBandChunk, HBITS, HP2, CP2, 4, MODE, true>;
+    static std::atomic<int> dyn_cache[kMaxDevices];
+    hipError_t e = hipSuccess;
+    const int dyn_max = dyn_lds_max((const void *)kern, dyn_cache, &e);
+    if (!dyn_max)
+        return e;
+    a.chunk_max = std::min(kBandChunk, std::max(1, (a.f.n + kGroups - 1) / kGroups) * kGroups);
+    int32_t most = 64;
+    while (most + 64 <= kMaxRows &&
+           render_lds_bytes(TC, NT, most + 64, a.chunk_max) <= (size_t)dyn_max)
+        most += 64;
+    const int32_t bands = (a.f.rows + most - 1) / most;
+    a.band_rows = ((a.f.rows + bands - 1) / bands + 63) & ~63;
+    a.ntiles = (a.f.cols + TC - 1) / TC;
+    const size_t need = render_lds_bytes(TC, NT, a.band_rows, a.chunk_max);
+    if (need > (size_t)dyn_max)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, dim3(a.ntiles, (a.f.rows + a.band_rows - 1) / a.band_rows), dim3(NT),
+                       need, s, a);
+    return hipGetLastError();
+}
+
 template <int HBITS, bool HP2, bool CP2, int MODE = kOutColour>
 hipError_t launch_render(RenderArgs a, const fsk_tuning &tune, hipStream_t s,
                          int32_t *nzero = nullptr)
 {
     if (a.f.rows > kMaxRows) {
-        /* taller than a tile: the column kernel (no gradient clear) */
         if (nzero)
-            *nzero = 0;
-        if (a.f.rows > kMaxFrameRows)
-            return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_render_column<HBITS, HP2, CP2, MODE>), dim3((a.f.cols + 63) / 64),
-                           dim3(64), 0, s, a);
-        return hipGetLastError();
+            *nzero = 0;         /* no gradient clear */
+        return launch_bands<HBITS, HP2, CP2, MODE>(a, s);
     }
     Shape sh = resolve_shape(a.f.rows, tune);
     a.chunk_max = sh.chunk;
@@ -2832,6 +2877,7 @@ int fsk_render_slices_clear(const fsk_map *m, const fsk_frame *f, const fsk_tuni
     a.pitch = pitch;
     a.ntiles = 0;
     a.chunk_max = kChunk;
+    a.band_rows = 0;
     a.zero = nullptr;
     a.zero_n4 = 0;
     a.nzero = 0;
@@ -2898,6 +2944,7 @@ int fsk_render_nearest(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t
     a.pitch = pitch;
     a.ntiles = 0;
     a.chunk_max = kChunk;
+    a.band_rows = 0;
     a.zero = nullptr;
     a.zero_n4 = 0;
     a.nzero = 0;
@@ -3139,6 +3186,7 @@ int fsk_render(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t, uint32
     a.pitch = pitch;
     a.ntiles = 0;
     a.chunk_max = kChunk;
+    a.band_rows = 0;
     a.zero = nullptr;
     a.zero_n4 = 0;
     a.nzero = 0;

@@ -127,8 +127,8 @@ int futhark_entry_update_map(struct futhark_context *ctx, struct futhark_opaque_
  * (invz_param2, :103), scale (magic_number, :217; <= 0 means f32(w/2)),
  * n_slices (<= 0 means get_zs' count from distance, :28-34; a render
  * refuses more than 2^24 slices, and frames of more than 2^22 rows;
- * frames of more than 7680 rows take a slower one-thread-per-column
- * kernel, and a batched view has at most 7680 rows).
+ * frames of more than 7680 rows are rendered in bands of rows, and a
+ * batched view has at most 7680 rows).
  * `map` indexes the map list of a batched render. */
 struct fsx_view {
     float x, y, height, angle, horizon, distance, fov;

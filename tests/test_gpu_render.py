@@ -294,3 +294,33 @@ def test_shade_wraps_and_exits(ctx, rows, cols, size, bits, sun_h, sun_a):
     torch.cuda.synchronize()
     want = O.shade_factor(O.shadow_counts(alt, O.sun(sun_h, sun_a), size))
     assert np.array_equal(sf.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("h,w,n,bits", [(7681, 8, 300, 8), (9000, 17, 1025, 16),
+                                        (16000, 3, 2500, 8)])
+def test_bands_of_rows(ctx, h, w, n, bits):
+    """Frames rendered in bands of rows over one and several depth chunks,
+    with blocks of colour-0 texels (transparent samples, also where a band
+    begins) and a camera on an integral column: bit-exact, also into a
+    wider pitch."""
+    import torch
+    col, hts = scene.scene_maps(11, 128, 255 if bits == 8 else 900)
+    col = np.array(col, copy=True)
+    block = np.random.default_rng(n).random((16, 16)) < 0.5
+    col[np.kron(block, np.ones((8, 8), bool))] = 0
+    m = ctx.map(col, hts, height_bits=bits, shade_size=128)
+    shaded, alt = O.update_map(col, hts, size=128, bits=bits)
+    d, z0 = scene.depth_for(n, 400.0)
+    for x, angle, horizon in ((40.3, 1.3, 0.4 * h), (40.0, 0.0, 0.9 * h), (90.7, 4.0, -300.0)):
+        v = View(x=x, y=90.6, height=3.0 * hts.max() / 2, angle=angle, horizon=horizon,
+                 distance=400.0, fov=1.2, sky_color=sky_color(0.1), h=h, w=w, d=d, z0=z0,
+                 scale=h / 3.0, n_slices=n)
+        want = O.render_off(v, shaded, alt)
+        _check(ctx.render(m, v), want)
+        out = torch.full((h, w + 5), -1, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.render(m, v, out)
+        ctx.sync()
+        got = out.cpu().numpy()
+        _check(got[:, :w].view(np.uint32), want)
+        assert (got[:, w:] == -1).all()

@@ -100,3 +100,20 @@ def test_frames_taller_than_a_tile(ctx):
     v = View(x=40.0, y=-30.0, height=260.0, angle=0.7, horizon=3000.0, distance=300.0, fov=1.1,
              sky_color=0xFF9090E0, h=9000, w=11)
     assert np.array_equal(ctx.render_stateless(colour, height, v), _oracle(v, colour, height))
+
+
+@pytest.mark.parametrize("h,w,q,r,clear", [
+    (7681, 1, 64, 64, 0.5), (7681, 8, 48, 100, 0.97), (9001, 17, 128, 128, 0.5),
+    (20003, 9, 100, 48, 0.9), (20003, 24, 64, 64, 0.0),
+])
+def test_bands_of_rows(ctx, h, w, q, r, clear):
+    """Frames rendered in bands of rows, with a share of sky-coloured
+    (transparent) texels: a band whose first rows lie behind a transparent
+    sample from above it shows what the whole column shows there."""
+    colour, height = _maps(h + w, q, r)
+    gone = np.random.default_rng(h).random((q, r)) < clear
+    colour = np.where(gone, np.uint32(0xFF9090E0).view(np.int32), colour).astype(np.int32)
+    for horizon, alt in ((h * 0.5, 300.0), (h * 1.1, 150.0), (-200.0, 400.0)):
+        v = View(x=40.3, y=-30.2, height=alt, angle=0.7, horizon=horizon, distance=500.0,
+                 fov=1.1, sky_color=0xFF9090E0, h=h, w=w)
+        assert np.array_equal(ctx.render_stateless(colour, height, v), _oracle(v, colour, height))
