@@ -1274,30 +1274,43 @@ __global__ __launch_bounds__(NT, WPE) void k_render(RenderArgs a)
             return;
         }
     }
-    const int32_t tile = xcd_tile(blockIdx.x, a.ntiles);
     const int32_t row0 = BAND ? (int32_t)blockIdx.y * a.band_rows : 0;
     uint32_t *out = BAND ? a.out + (size_t)row0 * (size_t)a.pitch : a.out;
     if constexpr (MODE == kOutColour) {
+        /* the table loads go first: the tile's index arithmetic before them
+         * had cost the 1080p frame 0.2 us */
         TileTables<TC, NT> tables;
         tables.load(threadIdx.x);
         render_tile<TC, NT, CMAX, HBITS, HP2, CP2, MODE, kGather, kColourBatch,
-                    TileTables<TC, NT>, BAND>(a.m, a.f, out, a.pitch, tile, a.chunk_max, lds, sh,
-                                              tables, row0, a.band_rows);
+                    TileTables<TC, NT>, BAND>(a.m, a.f, out, a.pitch,
+                                              xcd_tile(blockIdx.x, a.ntiles), a.chunk_max, lds,
+                                              sh, tables, row0, a.band_rows);
     } else {
         render_tile<TC, NT, CMAX, HBITS, HP2, CP2, MODE, kGather, kColourBatch, NoTables, BAND>(
-            a.m, a.f, out, a.pitch, tile, a.chunk_max, lds, sh, NoTables(), row0, a.band_rows);
+            a.m, a.f, out, a.pitch, xcd_tile(blockIdx.x, a.ntiles), a.chunk_max, lds, sh,
+            NoTables(), row0, a.band_rows);
     }
 }
 
 /* render2 (fut/voxel_renderer.fut:257-305), the reference's ray-march
- * renderer, one thread per pixel.  The reference evaluates every
- * dist = 0 ... n and keeps the hit with the smallest dist (redstuff,
- * :254-255); dists grow along the ray, so that is the first hit, and the
- * march stops there (hits are the only elements that can win while the
+ * renderer.  The reference evaluates every dist = 0 ... n and keeps the hit
+ * with the smallest dist (redstuff, :254-255); dists grow along the ray, so
+ * that is the first hit (hits are the only elements that can win while the
  * miss distance i32(distance + 1) exceeds n, which the host checks).  The
  * colour is bilinear over the map's unshaded colours, evaluated for the
  * hit only.  cs/sn hold cos and sin of angle + horz_ang per column,
- * computed on the host with the C library as `futhark c` does. */
+ * computed on the host with the C library as `futhark c` does.
+ *
+ * The terrain height under a ray point does not depend on the pixel's row:
+ * a workgroup evaluates the heights of its 64 columns once for its
+ * kR2Rows rows, kR2Chunk dists at a time, into LDS.  A pixel then searches
+ * them: along dist the line of sight cam_h - dist * vert_ang is monotone,
+ * also in f32, so if its lower end over a group of 16 dists is not below the
+ * group's highest terrain, none of them hits.  Wave w of the 16 evaluates
+ * group w of a chunk, and so has the group's maximum in registers.  800 x 600
+ * pixels, 200 steps: 15 us, against 98 us with one thread per pixel marching
+ * through the map; bound by the latency of its two phases on 247
+ * workgroups. */
 struct Render2Args {
     fsk_map m;
     const uint32_t *color;     /* unshaded colours [hrows][hcols] */
@@ -1320,30 +1333,99 @@ __device__ __forceinline__ uint4 raw_color_quad(const uint32_t *col, int32_t row
     return make_uint4(col[fy * w + fx], col[fy * w + cx], col[cy * w + fx], col[cy * w + cx]);
 }
 
+constexpr int kR2Group = 16;                      /* dists per group */
+constexpr int kR2Chunk = 16 * kR2Group;           /* a group per wave */
+constexpr int kR2Rows = 32;                       /* frame rows per workgroup */
+
 template <int HBITS, bool HP2>
-__global__ __launch_bounds__(256) void k_render2(Render2Args a)
+__global__ __launch_bounds__(1024) void k_render2(Render2Args a)
 {
     __shared__ float sq[256];
+    __shared__ float hs[kR2Chunk][64], top[kR2Chunk / kR2Group][64];
+    const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t x = blockIdx.x * 64 + lane;
+    const float ca = a.cs[min(x, a.cols - 1)], sa = a.sn[min(x, a.cols - 1)];
     fill_square_lut(sq, threadIdx.x);
-    __syncthreads();
-    const int32_t x = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int32_t y = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (x >= a.cols || y >= a.rows)
-        return;
-    const float vert_ang = (a.horizon / 50.0f) + (((float)y / ((float)a.rows - 0.0f)) * (1.5f - 1.0f));
-    const float ca = a.cs[x], sa = a.sn[x];
-    uint32_t c = 0u;
-    for (int32_t dist = 0; dist <= a.n; dist++) {
-        const float fd = (float)dist;
-        const float px = a.cam_x + (fd * ca), py = a.cam_y + (fd * sa);
-        const float hgt = height_interp<HBITS>(height_quad<HBITS, HP2>(a.m, px, py), px, py);
-        if ((a.cam_h - (fd * vert_ang)) < hgt) {
+    constexpr int PX = kR2Rows / 16;
+    float vert_ang[PX];
+    int32_t hit[PX];
+#pragma unroll
+    for (int u = 0; u < PX; u++) {
+        const int32_t y = blockIdx.y * kR2Rows + u * 16 + wave;
+        vert_ang[u] = (a.horizon / 50.0f) + (((float)y / ((float)a.rows - 0.0f)) * (1.5f - 1.0f));
+        hit[u] = -1;
+    }
+    for (int32_t base = 0; base <= a.n; base += kR2Chunk) {
+        const int32_t d0 = base + wave * kR2Group;
+        float high = -INFINITY;
+#pragma unroll
+        for (int j0 = 0; j0 < kR2Group; j0 += 8) {
+            if (d0 + j0 > a.n) {
+                /* past the march: nothing is below the lowest height */
+#pragma unroll
+                for (int j = j0; j < j0 + 8; j++)
+                    hs[wave * kR2Group + j][lane] = -INFINITY;
+                continue;
+            }
+            float px[8], py[8];
+            uint2 q[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float fd = (float)(d0 + j0 + j);
+                px[j] = a.cam_x + (fd * ca);
+                py[j] = a.cam_y + (fd * sa);
+                q[j] = height_quad<HBITS, HP2>(a.m, px[j], py[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                float h = height_interp<HBITS>(q[j], px[j], py[j]);
+                h = d0 + j0 + j <= a.n ? h : -INFINITY;
+                hs[wave * kR2Group + j0 + j][lane] = h;
+                high = fmaxf(high, h);
+            }
+        }
+        top[wave][lane] = high;
+        __syncthreads();
+        const int32_t groups = min(kR2Chunk, a.n + 1 - base + kR2Group - 1) / kR2Group;
+        bool pending = false;
+#pragma unroll
+        for (int u = 0; u < PX; u++) {
+            for (int32_t g = 0; g < groups && hit[u] < 0; g++) {
+                const float f0 = (float)(base + g * kR2Group);
+                const float t0 = a.cam_h - (f0 * vert_ang[u]);
+                const float t1 = a.cam_h - ((f0 + (float)(kR2Group - 1)) * vert_ang[u]);
+                if (!(fminf(t0, t1) < top[g][lane]))
+                    continue;
+                uint32_t below = 0u;
+#pragma unroll
+                for (int j = 0; j < kR2Group; j++)
+                    below |= (a.cam_h - ((f0 + (float)j) * vert_ang[u])) <
+                                     hs[g * kR2Group + j][lane] ? 1u << j : 0u;
+                if (below)
+                    hit[u] = base + g * kR2Group + __builtin_ctz(below);
+            }
+            pending = pending || hit[u] < 0;
+        }
+        /* also keeps the next chunk's heights from those still being read */
+        if (!__syncthreads_or(pending))
+            break;
+    }
+    if (a.n < 0)
+        __syncthreads();                          /* the squares */
+#pragma unroll
+    for (int u = 0; u < PX; u++) {
+        const int32_t y = blockIdx.y * kR2Rows + u * 16 + wave;
+        if (x >= a.cols || y >= a.rows)
+            continue;
+        uint32_t c = 0u;
+        if (hit[u] >= 0) {
+            const float fd = (float)hit[u];
+            const float px = a.cam_x + (fd * ca), py = a.cam_y + (fd * sa);
             c = color_of_quad(raw_color_quad<HP2>(a.color, a.m.hrows, a.m.hcols, px, py), sq, px,
                               py);
-            break;
         }
+        a.out[(size_t)y * (size_t)a.pitch + (size_t)x] = c;
     }
-    a.out[(size_t)y * (size_t)a.pitch + (size_t)x] = c;
 }
 
 /* ------------------------------------------------------------------ */
@@ -3109,11 +3191,11 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
     a.n = n;
     a.rows = f->rows;
     a.cols = f->cols;
-    dim3 grid((f->cols + 63) / 64, (f->rows + 3) / 4);
+    dim3 grid((f->cols + 63) / 64, (f->rows + kR2Rows - 1) / kR2Rows);
     const bool p2 = pow2(m->hrows) && pow2(m->hcols);
     void (*kern)(Render2Args) = m->hbits == 8 ? (p2 ? k_render2<8, true> : k_render2<8, false>)
                                               : (p2 ? k_render2<16, true> : k_render2<16, false>);
-    hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(kern, grid, dim3(1024), 0, s, a);
     return hipGetLastError();
 }
 

@@ -68,3 +68,27 @@ def test_render2_rejects_unbounded_march(ctx):
     v = View(x=1.0, y=1.0, height=100.0, angle=0.0, horizon=0.0, distance=1e8, fov=1.2, h=4, w=4)
     with pytest.raises(RuntimeError):
         ctx.render2(m, v)
+
+
+@pytest.mark.parametrize("distance,h,w,horizon,bits", [
+    (-8.0, 5, 7, 3.0, 8),                                    # no step at all
+    (3.0, 33, 65, 8.0, 8),                                   # one step
+    (60.0, 32, 64, 30.0, 8), (64.0, 31, 63, 30.0, 16),       # one group of steps, and one more
+    (1020.0, 65, 129, 2.0, 8), (1024.0, 40, 66, 1.0, 8),     # one chunk of steps, and one more
+    (2100.0, 34, 70, -0.5, 16),                              # looking up and down
+    (400.0, 33, 65, float("inf"), 8), (400.0, 20, 30, float("-inf"), 8),
+])
+def test_render2_steps_and_tiles(ctx, distance, h, w, horizon, bits):
+    """Marches and frames at the edges of the kernel's groups, chunks and
+    workgroups, over a map that misses in places."""
+    hts = scene.heightmap(27, 128, 0.6, 255 if bits == 8 else 900)
+    hts = np.ascontiguousarray(hts[:, :96])
+    col = scene.colormap(27, hts, 255 if bits == 8 else 900)
+    m = ctx.map(col, hts, height_bits=bits)
+    for x, height in ((40.2, 1.2 * hts.max()), (90.7, 0.5 * hts.max())):
+        v = View(x=x, y=77.9, height=float(height), angle=2.2, horizon=horizon,
+                 distance=distance, h=h, w=w)
+        want = O.render2(v, col, np.asarray(hts, np.int32) & (255 if bits == 8 else 0xFFFF))
+        got = ctx.render2(m, v)
+        bad = int(np.count_nonzero(got != want))
+        assert bad == 0, f"{bad} of {got.size} pixels differ"
