@@ -1818,8 +1818,52 @@ struct Shape {
 
 constexpr size_t kStaticLds = 12288;  /* headroom for the kernels' static shared memory */
 
-inline Shape resolve_shape(int32_t rows, const fsk_tuning &t)
+/* Slices from which on a lane of a 1024-thread tile holds more than
+ * kHalfChunk / (slice groups) of them: up to there the kernels of half the
+ * chunk waste no registers and no passes on slices that are not there
+ * (1100 x 400, 1024 slices). */
+constexpr int kHalfChunk = 1024;
+
+/* The automatic shape of one frame: what was measured best over widths of
+ * 64 to 8192, 240 to 1240 rows and 64 to 4096 slices (us, 8x1 / 4x1 /
+ * 8x2 = columns x workgroups per CU).
+ *  - narrow: 4-column tiles still find a CU each, and a tile's time is its
+ *    latency chain and its share of the work (640 x 480, 2048 slices: 12.9 /
+ *    9.4 / 18.7);
+ *  - one chunk of the 512-thread tile, whose barriers and phases are the
+ *    shortest: up to 256 slices (64 x 240, 200: 7.2 / 7.4 / 6.4), or 512
+ *    where there are more tiles than CUs (3840 x 1080, 500: 17.8 / 32.4 /
+ *    13.5);
+ *  - more tiles than CUs: two tiles on a CU instead of one after the other
+ *    (2560 x 400, 1024: 16.8 / 19.2 / 13.8), unless the 1024-thread tile's
+ *    last 2048-slice chunk is more than three quarters full, where it is as
+ *    fast or faster (2560 x 1080, 2048: 26.2 / 27.4 / 27.1; 3000: 38.6 / 46.4
+ *    / 35.6) but for frames of many rounds (8192 x 1080, 2048: 52.4 / 72.1 /
+ *    49.8).
+ * spare: the caller would use kMinZeroBlocks idle CUs, which 4-column tiles
+ * may not leave. */
+inline fsk_tuning frame_shape(int32_t rows, int32_t cols, int32_t n, bool spare)
 {
+    fsk_tuning t = {0, 0, 0};
+    const int32_t cus = cu_count(), tiles4 = (cols + 3) / 4, tiles8 = (cols + 7) / 8;
+    const bool two = 2 * (render_lds_bytes(8, 512, rows, 512) + kStaticLds) <= lds_per_cu();
+    const bool narrow = tiles4 <= cus && !(spare && cus - tiles4 < kMinZeroBlocks);
+    if (two && n <= (tiles8 > cus ? 512 : 256))
+        t.wg_per_cu = 2;
+    else if (narrow)
+        t.tc = 4;
+    else if (two && tiles8 > cus && (tiles8 > 3 * cus || (n - 1) % kChunk < 3 * kChunk / 4))
+        t.wg_per_cu = 2;
+    return t;
+}
+
+/* The shape of a frame of `rows` rows under tuning `tune`; with cols > 0 a
+ * tuning left automatic follows frame_shape. */
+inline Shape resolve_shape(int32_t rows, const fsk_tuning &tune, int32_t cols = 0, int32_t n = 0,
+                           bool spare = false)
+{
+    const bool automatic = cols > 0 && !tune.tc && !tune.wg_per_cu && !tune.chunk;
+    const fsk_tuning t = automatic ? frame_shape(rows, cols, n, spare) : tune;
     Shape s;
     s.cmax = kChunk;
     int chunk = (t.chunk >= 256 && t.chunk <= kChunk) ? t.chunk : 0;
@@ -1876,6 +1920,12 @@ inline Shape resolve_shape(int32_t rows, const fsk_tuning &t)
         s.wg = 1;
         fit();
     }
+    if (s.nt == 1024) {
+        if (automatic && n <= kHalfChunk && s.chunk > kHalfChunk)
+            s.chunk = kHalfChunk;
+        if (s.chunk <= kHalfChunk)
+            s.cmax = kHalfChunk;
+    }
     return s;
 }
 
@@ -1926,7 +1976,8 @@ hipError_t launch_render(RenderArgs a, const fsk_tuning &tune, hipStream_t s,
             *nzero = 0;         /* no gradient clear */
         return launch_bands<HBITS, HP2, CP2, MODE>(a, s);
     }
-    Shape sh = resolve_shape(a.f.rows, tune);
+    Shape sh = resolve_shape(a.f.rows, tune, a.f.cols, a.f.n,
+                             MODE == kOutSlice && a.zero && a.zero_n4);
     a.chunk_max = sh.chunk;
     a.ntiles = (a.f.cols + sh.tc - 1) / sh.tc;
     /* slice mode: the workgroup slots the tiles leave free clear the
@@ -1935,12 +1986,17 @@ hipError_t launch_render(RenderArgs a, const fsk_tuning &tune, hipStream_t s,
     a.nzero = (MODE == kOutSlice && a.zero && a.zero_n4 && spare >= kMinZeroBlocks) ? spare : 0;
     if (nzero)
         *nzero = a.nzero;
+    const bool half = sh.cmax == kHalfChunk;
     if (sh.tc == 8) {
-        return sh.nt == 512 ? launch_render_cfg<8, 512, 512, HBITS, HP2, CP2, 4, MODE>(a, s)
-                            : launch_render_cfg<8, 1024, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s);
+        if (sh.nt == 512)
+            return launch_render_cfg<8, 512, 512, HBITS, HP2, CP2, 4, MODE>(a, s);
+        return half ? launch_render_cfg<8, 1024, kHalfChunk, HBITS, HP2, CP2, 4, MODE>(a, s)
+                    : launch_render_cfg<8, 1024, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s);
     }
-    return sh.nt == 512 ? launch_render_cfg<4, 512, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s)
-                        : launch_render_cfg<4, 1024, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s);
+    if (sh.nt == 512)
+        return launch_render_cfg<4, 512, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s);
+    return half ? launch_render_cfg<4, 1024, kHalfChunk, HBITS, HP2, CP2, 4, MODE>(a, s)
+                : launch_render_cfg<4, 1024, kChunk, HBITS, HP2, CP2, 4, MODE>(a, s);
 }
 
 /* ------------------------------------------------------------------ */

@@ -324,3 +324,20 @@ def test_bands_of_rows(ctx, h, w, n, bits):
         got = out.cpu().numpy()
         _check(got[:, :w].view(np.uint32), want)
         assert (got[:, w:] == -1).all()
+
+
+@pytest.mark.parametrize("w,h,n", [
+    (9, 33, 256), (9, 33, 257), (1024, 21, 1024), (1024, 21, 1025), (1025, 21, 300),
+    (2048, 20, 513), (2049, 20, 512), (2049, 20, 513), (2060, 20, 1536), (2060, 20, 1537),
+    (2060, 20, 2100), (6145, 9, 1700), (1030, 1249, 700), (1030, 1250, 200), (30, 2000, 3000),
+])
+def test_automatic_shapes(ctx, small_scene, w, h, n):
+    """Frames on both sides of the lines between the automatic tile shapes
+    (columns, workgroups per CU, chunk), one column or slice apart."""
+    col, hts = small_scene
+    m = ctx.map(col, hts, shade_size=128)
+    shaded, alt = O.update_map(col, hts, size=128)
+    d, z0 = scene.depth_for(n, 500.0)
+    v = View(x=70.3, y=20.6, height=280.0, angle=2.3, horizon=h * 0.3, distance=500.0, fov=1.2,
+             sky_color=sky_color(0.1), h=h, w=w, d=d, z0=z0, scale=h / 2.0, n_slices=n)
+    _check(ctx.render(m, v), O.render_painter_mt(v, shaded, alt, 8))
