@@ -1852,7 +1852,7 @@ int fsx_l2_loss(struct futhark_context *ctx, const float *dev_img, const float *
 
 struct fsx_batch {
     fsk_batch b;
-    void *d_mem;                   /* views | items | qmeta | counters */
+    void *d_mem;                   /* views | items | qmeta | padding | counters */
     int32_t n_views, n_maps;
     struct fs_terrain **terrains;  /* references held while the batch lives */
     struct fs_shade **shades;
@@ -1986,6 +1986,12 @@ int fsx_batch_new(struct futhark_context *ctx, const struct fsx_map *const *maps
         return 1;
     }
     bt->b.tune = ctx->tune;
+    int64_t tiles4 = 0, tiles8 = 0;
+    for (int32_t i = 0; i < n_views; i++) {
+        tiles4 += (views[i].w + 3) / 4;
+        tiles8 += (views[i].w + 7) / 8;
+    }
+    fsk_batch_shape(max_rows, tiles4, tiles8, &bt->b.tune);
     int32_t tc = fsk_tile_columns(max_rows, &bt->b.tune);
     int64_t n_items = 0;
     for (int32_t i = 0; i < n_views; i++) {
@@ -2014,27 +2020,33 @@ int fsx_batch_new(struct futhark_context *ctx, const struct fsx_map *const *maps
     size_t vb = sizeof(fsk_batch_view) * (size_t)n_views;
     size_t ib = sizeof(uint32_t) * (size_t)n_items;
     size_t mb = sizeof(uint32_t) * 2 * FS_QUEUES;
-    size_t cb = sizeof(uint32_t) * FS_QUEUES;
-    uint32_t *hitems = (uint32_t *)malloc(ib + mb);
+    /* the counters start on a line of their own */
+    const size_t cpad = (256 - (vb + ib + mb) % 256) % 256;
+    size_t cb = sizeof(uint32_t) * FSK_BATCH_COUNTERS(FS_QUEUES);
+    uint32_t *hitems = (uint32_t *)calloc(1, ib + mb + cpad + cb);
+    int32_t grid = fsk_batch_grid(max_rows, &bt->b.tune);
+    if (grid > n_items)
+        grid = (int32_t)n_items;
     int rc = 1;
     if (hitems && hipSetDevice(ctx->device) == hipSuccess &&
-        hipMalloc(&bt->d_mem, vb + ib + mb + cb) == hipSuccess) {
+        hipMalloc(&bt->d_mem, vb + ib + mb + cpad + cb) == hipSuccess) {
         deal_items(hv, n_views, hitems, hitems + n_items);
+        fsk_batch_counters_init((uint32_t *)((char *)hitems + ib + mb + cpad), grid, FS_QUEUES);
         char *base = (char *)bt->d_mem;
         hipError_t e = hipMemcpy(base, hv, vb, hipMemcpyHostToDevice);
         if (e == hipSuccess)
-            e = hipMemcpy(base + vb, hitems, ib + mb, hipMemcpyHostToDevice);
+            e = hipMemcpy(base + vb, hitems, ib + mb + cpad + cb, hipMemcpyHostToDevice);
         if (e == hipSuccess) {
             bt->b.views = (const fsk_batch_view *)base;
             bt->b.items = (const uint32_t *)(base + vb);
             bt->b.qmeta = (const uint32_t *)(base + vb + ib);
-            bt->b.counters = (uint32_t *)(base + vb + ib + mb);
+            bt->b.counters = (uint32_t *)(base + vb + ib + mb + cpad);
             bt->b.out = dev_out;
             bt->b.nqueues = FS_QUEUES;
             bt->b.max_rows = max_rows;
             bt->b.hbits = hbits;
             bt->b.pow2 = pow2;
-            bt->b.grid = fsk_batch_grid(max_rows, &bt->b.tune);
+            bt->b.grid = grid;
             rc = 0;
         } else {
             set_error(ctx, "fsx_batch_new: upload failed: %s", hipGetErrorString(e));

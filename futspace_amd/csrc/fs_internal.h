@@ -98,18 +98,28 @@ typedef struct {
     const fsk_batch_view *views;   /* device */
     const uint32_t *items;         /* device: view << 16 | tile, grouped by queue */
     const uint32_t *qmeta;         /* device: qstart[nqueues], qlen[nqueues] */
-    uint32_t *counters;            /* device: nqueues claim counters */
+    uint32_t *counters;            /* device: FSK_BATCH_COUNTERS(nqueues) claim counters */
     uint32_t *out;
     int32_t nqueues, max_rows, hbits, pow2;
     int32_t grid;                  /* persistent workgroups */
     fsk_tuning tune;
 } fsk_batch;
 
+/* Sets a tuning left automatic to the shape of a batch with views of up to
+ * max_rows rows, of tiles4 tiles of 4 columns or tiles8 of 8 in all. */
+void fsk_batch_shape(int32_t max_rows, int64_t tiles4, int64_t tiles8, fsk_tuning *t);
 /* Columns per tile the kernels use for frames of max_rows rows. */
 int32_t fsk_tile_columns(int32_t max_rows, const fsk_tuning *t);
 /* Persistent workgroups for a batch (CUs x workgroups per CU). */
 int32_t fsk_batch_grid(int32_t max_rows, const fsk_tuning *t);
-/* Reset the claim counters and run the persistent batched render. */
+/* The claim counters of a batch: one per queue and one of ended workgroups,
+ * FSK_COUNTER_STRIDE words apart so that each has a cache line of its own.
+ * fsk_batch_counters_init fills the host image that is uploaded with the
+ * batch; every launch leaves them in that state again. */
+#define FSK_COUNTER_STRIDE 64
+#define FSK_BATCH_COUNTERS(nqueues) (((nqueues) + 1) * FSK_COUNTER_STRIDE)
+void fsk_batch_counters_init(uint32_t *counters, int32_t grid, int32_t nqueues);
+/* Run the persistent batched render. */
 int fsk_batch_run(const fsk_batch *b, hipStream_t s);
 
 /* Device self-test `which` (0-7) of the arithmetic shortcuts; adds the

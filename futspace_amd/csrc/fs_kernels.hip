@@ -669,6 +669,11 @@ struct TileTables {
     }
 };
 
+/* Nothing to do before a tile's rows are written. */
+struct NoHook {
+    __device__ __forceinline__ void operator()() const {}
+};
+
 /* No colour tables (tile modes without the argb colour path). */
 struct NoTables {
     template <int TC>
@@ -784,12 +789,12 @@ __device__ uint32_t column_above(const fsk_map &m, const fsk_frame &f, int32_t c
  * covers show the next opaque one above, which column_above finds. */
 template <int TC, int NT, int CMAX, int HBITS, bool HP2, bool CP2, int MODE = kOutColour,
           int GATHER = kGather, int CBATCH = kColourBatch, class Tables = NoTables,
-          bool BAND = false>
+          bool BAND = false, class Hook = NoHook>
 __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f, uint32_t *out,
                                             int64_t pitch, int32_t tile, int32_t chunk_max,
                                             uint32_t *lds, TileShared<TC> &sh,
                                             const Tables &tables = Tables(), int32_t row0 = 0,
-                                            int32_t band_rows = 0)
+                                            int32_t band_rows = 0, Hook &&before_write = Hook())
 {
     constexpr int NW = NT / 64;                  /* waves */
     constexpr int SG = NT / TC;                  /* slice groups */
@@ -1112,6 +1117,7 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
     if (nl)
         __syncthreads();
 
+    before_write();
     const bool vec = (col0 + TC <= f.cols) && ((pitch & 3) == 0) &&
                      ((((uintptr_t)out) & 15u) == 0);
     /* a cell above its column's final y-buffer was never painted: 0 */
@@ -2012,24 +2018,29 @@ struct BatchArgs {
     int32_t nqueues, chunk_max;
 };
 
-/* XCD this wave runs on (hardware register XCC_ID). */
-__device__ __forceinline__ uint32_t xcc_id()
-{
-    return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & 0xFu;
-}
-
-__global__ void k_batch_reset(uint32_t *counters, int32_t n)
-{
-    int32_t i = threadIdx.x;
-    if (i < n)
-        counters[i] = 0u;
-}
-
-/* Persistent workgroups claim (view, tile) items from per-XCD queues: the
+/* Persistent workgroups take (view, tile) items from per-XCD queues: the
  * host deals each view's tiles out to the queues in contiguous blocks, so
- * neighbouring tiles of a view stay on one L2; a workgroup whose own queue
- * is drained takes from the next queues.  Every workgroup exits once all
- * queues report exhausted, after at most nqueues claims. */
+ * neighbouring tiles of a view stay on one L2 (workgroup i runs on XCD
+ * i mod 8).  Workgroup i takes item i / nqueues of queue i mod nqueues
+ * first, and then what the queues' counters hand out, from the next queues
+ * when its own is drained; it ends when all are.
+ *
+ * A claim is an atomic on memory all XCDs share, and those on one line go
+ * one after the other: each counter has a line of its own, the first item
+ * needs no claim, and a drained queue is told by reading its counter.  With
+ * the eight counters in one line, and an atomic on each of them for every
+ * workgroup that ran dry, the claims took longer than the tiles of a small
+ * batch (4 views: 157 us).
+ *
+ * The counters are as fsk_batch_counters_init left them before the first
+ * launch; the last workgroup to end leaves them so for the next one, so that
+ * no launch has to reset them first.  Every claim of a workgroup has
+ * returned before it counts itself as ended. */
+__host__ __device__ constexpr uint32_t batch_first_claim(uint32_t grid, uint32_t q, uint32_t nq)
+{
+    return (grid + nq - 1u - q) / nq;      /* workgroups that start on queue q */
+}
+
 template <int TC, int NT, int CMAX, int HBITS, bool HP2, bool CP2, int WPE>
 __global__ __launch_bounds__(NT, WPE) void k_render_batch(BatchArgs b)
 {
@@ -2041,19 +2052,28 @@ __global__ __launch_bounds__(NT, WPE) void k_render_batch(BatchArgs b)
         tables.load(threadIdx.x);
         tables.store(sh, threadIdx.x);    /* the claim loop's barrier publishes them */
     }
-    uint32_t q = xcc_id() % (uint32_t)b.nqueues;
-    int32_t tried = 0;
+    const uint32_t nq = (uint32_t)b.nqueues;
+    uint32_t q = blockIdx.x % nq, tried = 0u;
+    uint32_t len = b.qmeta[nq + q], next = blockIdx.x / nq;
+    bool claimed = true;                  /* next is this workgroup's */
     for (;;) {
         if (threadIdx.x == 0) {
             uint32_t v = 0xFFFFFFFFu;
-            while (tried < b.nqueues) {
-                uint32_t k = atomicAdd(&b.counters[q], 1u);
-                if (k < b.qmeta[b.nqueues + q]) {
-                    v = b.items[b.qmeta[q] + k];
+            while (tried < nq) {
+                uint32_t *count = b.counters + q * FSK_COUNTER_STRIDE;
+                if (!claimed && __hip_atomic_load(count, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT) < len) {
+                    next = atomicAdd(count, 1u);
+                    claimed = true;
+                }
+                if (claimed && next < len) {
+                    v = b.items[b.qmeta[q] + next];
                     break;
                 }
+                claimed = false;
                 tried++;
-                q = (q + 1u) % (uint32_t)b.nqueues;
+                q = q + 1u == nq ? 0u : q + 1u;
+                len = b.qmeta[nq + q];
             }
             cur = v;
         }
@@ -2063,8 +2083,29 @@ __global__ __launch_bounds__(NT, WPE) void k_render_batch(BatchArgs b)
         if (it == 0xFFFFFFFFu)
             break;
         const fsk_batch_view &bv = b.views[it >> 16];
-        render_tile<TC, NT, CMAX, HBITS, HP2, CP2, kOutColour>(
-            bv.m, bv.f, b.out + bv.offset, bv.f.cols, it & 0xFFFFu, b.chunk_max, lds, sh);
+        /* while a queue is far from its end the next claim is made before
+         * the tile's rows are written, and its round trip passes under
+         * them; near the end an item claimed early would wait for this
+         * workgroup while others run dry */
+        auto claim = [&]() {
+            if (threadIdx.x == 0) {
+                claimed = next + gridDim.x / nq < len;
+                if (claimed)
+                    next = atomicAdd(b.counters + q * FSK_COUNTER_STRIDE, 1u);
+            }
+        };
+        render_tile<TC, NT, CMAX, HBITS, HP2, CP2, kOutColour, kGather, kColourBatch, NoTables,
+                    false, decltype(claim) &>(bv.m, bv.f, b.out + bv.offset, bv.f.cols,
+                                              it & 0xFFFFu, b.chunk_max, lds, sh, NoTables(), 0,
+                                              0, claim);
+    }
+    if (threadIdx.x == 0) {
+        uint32_t *ended = b.counters + nq * FSK_COUNTER_STRIDE;
+        if (atomicAdd(ended, 1u) == gridDim.x - 1u) {
+            for (uint32_t i = 0; i < nq; i++)
+                b.counters[i * FSK_COUNTER_STRIDE] = batch_first_claim(gridDim.x, i, nq);
+            *ended = 0u;
+        }
     }
 }
 
@@ -2088,7 +2129,6 @@ hipError_t launch_batch_cfg(const fsk_batch *fb, int chunk, hipStream_t s)
     b.out = fb->out;
     b.nqueues = fb->nqueues;
     b.chunk_max = chunk;
-    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, fb->counters, fb->nqueues);
     hipLaunchKernelGGL(kern, dim3(fb->grid), dim3(NT), need, s, b);
     return hipGetLastError();
 }
@@ -2967,6 +3007,22 @@ float *fsk_scratch(int32_t device, int64_t *n_floats)
     return g_init_done[device] ? g_scratch_ptr[device] : nullptr;
 }
 
+/* The automatic shape of a batch, by the tiles it would have (us per batch
+ * of views of 320 x 240 to 1920 x 1080, 1024 to 4096 slices, as 8x1 / 4x1 /
+ * 8x2): 4-column tiles while each finds a CU (2 views: 30 / 27 / 34), else
+ * two 512-thread tiles per CU, whose stalls overlap (4 views: 76 / 93 / 70;
+ * 40: 442 / 621 / 340; 256: 2690 / 3805 / 2180), where two fit in LDS. */
+void fsk_batch_shape(int32_t max_rows, int64_t tiles4, int64_t tiles8, fsk_tuning *t)
+{
+    if (t->tc || t->wg_per_cu || t->chunk)
+        return;
+    if (tiles4 <= cu_count())
+        t->tc = 4;
+    else if (tiles8 > cu_count() &&
+             2 * (render_lds_bytes(8, 512, max_rows, 512) + kStaticLds) <= lds_per_cu())
+        t->wg_per_cu = 2;
+}
+
 int32_t fsk_tile_columns(int32_t max_rows, const fsk_tuning *t)
 {
     return resolve_shape(max_rows, *t).tc;
@@ -2986,6 +3042,14 @@ void fsk_default_tuning(fsk_tuning *t)
     t->wg_per_cu = e ? atoi(e) : 0;
     e = getenv("FSX_RENDER_CHUNK");
     t->chunk = e ? atoi(e) : 0;
+}
+
+void fsk_batch_counters_init(uint32_t *counters, int32_t grid, int32_t nqueues)
+{
+    for (int32_t q = 0; q < nqueues; q++)
+        counters[q * FSK_COUNTER_STRIDE] =
+            batch_first_claim((uint32_t)grid, (uint32_t)q, (uint32_t)nqueues);
+    counters[nqueues * FSK_COUNTER_STRIDE] = 0u;
 }
 
 int fsk_batch_run(const fsk_batch *b, hipStream_t s)

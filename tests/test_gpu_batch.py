@@ -177,3 +177,30 @@ def test_batch_refuses_views_taller_than_a_tile(ctx, pow2_maps):
     out = torch.empty(v.h * v.w, dtype=torch.int32, device="cuda")
     with pytest.raises(RuntimeError):
         ctx.batch(maps, [v], out, np.array([0], dtype=np.int64))
+
+
+@pytest.mark.parametrize("widths", [(3,), (9, 1), (40, 333, 8), (1024, 1025), (2048, 900, 17, 512)])
+def test_small_batches_replayed(ctx, widths):
+    """Batches of fewer and of more tiles than workgroups, whose queues are
+    uneven or empty: every run of the same batch renders every view (the
+    claim counters are whole again after each)."""
+    col, hts = scene.scene_maps(31, 128)
+    m = ctx.map(col, hts, shade_size=128)
+    shaded, alt = O.update_map(col, hts, size=128)
+    views = [View(x=10.0 * i + 5.3, y=40.6, height=270.0, angle=0.7 * i, horizon=20.0,
+                  distance=400.0, fov=1.2, sky_color=sky_color(0.1), h=24 + i, w=w, d=0.004,
+                  z0=0.5, scale=60.0) for i, w in enumerate(widths)]
+    want = [O.render_painter_mt(v, shaded, alt, 8) for v in views]
+    offs = np.cumsum([0] + [v.h * v.w for v in views]).astype(np.int64)
+    out = torch.empty(int(offs[-1]), dtype=torch.int32, device="cuda")
+    b = ctx.batch([m], views, out, offs[:-1])
+    b.capture()
+    for run in (b.run, b.replay, b.run, b.replay, b.replay):
+        out.fill_(-1)
+        torch.cuda.synchronize()
+        run()
+        ctx.sync()
+        got = out.cpu().numpy().view(np.uint32)
+        for v, o, w in zip(views, offs, want):
+            assert np.array_equal(got[o:o + v.h * v.w].reshape(v.h, v.w), w)
+    b.close()
