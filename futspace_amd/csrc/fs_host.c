@@ -55,19 +55,18 @@ struct futhark_context {
     int prof_on;              /* bracket render kernels with events */
     int prof_n;
     hipEvent_t *prof_ev;      /* FS_PROF_MAX pairs */
-    float *d_partials;        /* per-workgroup partial sums of the reductions */
+    double *d_partials;       /* per-workgroup partial sums of the reductions */
     float *d_trig;            /* render2's per-column cos / sin */
     size_t trig_cap;          /* floats in d_trig */
 };
 
-#define FS_PARTIALS 32768     /* floats in d_partials */
-#define FS_STEP_BLOCK_COLS 64 /* pixel blocks of the adjoint (and of the fused step) */
+#define FS_STEP_BLOCK_COLS 64 /* pixel blocks of the differentiable passes' limits */
 
 /* Pixel blocks of a w x h frame in the differentiable passes (64 columns
- * by fsk_grad_block_rows rows): one partial sum per block. */
+ * by fsk_limit_block_rows rows), which their limits count. */
 static int64_t step_blocks(int32_t w, int32_t h)
 {
-    const int32_t br = fsk_grad_block_rows(w, h);
+    const int32_t br = fsk_limit_block_rows(w, h);
     return (int64_t)((w + FS_STEP_BLOCK_COLS - 1) / FS_STEP_BLOCK_COLS) *
            (int64_t)((h + br - 1) / br);
 }
@@ -1605,10 +1604,10 @@ int fsx_map_shade_factor(struct futhark_context *ctx, const struct fsx_map *map,
 
 /* The context's scratch for per-workgroup partial sums (allocated once;
  * stream-ordered reuse). */
-static int partials(struct futhark_context *ctx, float **p)
+static int partials(struct futhark_context *ctx, double **p)
 {
     if (!ctx->d_partials) {
-        hipError_t e = hipMalloc((void **)&ctx->d_partials, sizeof(float) * FS_PARTIALS);
+        hipError_t e = hipMalloc((void **)&ctx->d_partials, sizeof(double) * FSK_PARTIALS);
         if (e != hipSuccess) {
             ctx->d_partials = NULL;
             set_error(ctx, "scratch allocation failed: %s", hipGetErrorString(e));
@@ -1679,14 +1678,14 @@ int fsx_render_f32_vjp(struct futhark_context *ctx, const struct fsx_view *view,
         set_error(ctx, "fsx_render_f32_vjp: null buffer");
         return 1;
     }
-    if (step_blocks(view->w, view->h) > FS_PARTIALS) {
+    if (step_blocks(view->w, view->h) > FSK_LIMIT_BLOCKS) {
         set_error(ctx, "fsx_render_f32_vjp: a %d x %d frame has %lld blocks of %d x %d pixels, "
                   "more than the %d partial sums of the adjoint", view->w, view->h,
                   (long long)step_blocks(view->w, view->h), FS_STEP_BLOCK_COLS,
-                  fsk_grad_block_rows(view->w, view->h), FS_PARTIALS);
+                  fsk_limit_block_rows(view->w, view->h), FSK_LIMIT_BLOCKS);
         return 1;
     }
-    float *part;
+    double *part;
     if (partials(ctx, &part))
         return 1;
     HIPCHECK(ctx, hipSetDevice(ctx->device));
@@ -1695,7 +1694,7 @@ int fsx_render_f32_vjp(struct futhark_context *ctx, const struct fsx_view *view,
         HIPCHECK(ctx, fsk_zero_f32(dev_gplanes, (size_t)3 * (size_t)hc * (size_t)wc, ctx->stream));
     if (view->h > 0 && view->w > 0)
         HIPCHECK(ctx, fsk_diff_grad(&f, dev_planes, dev_sf, hc, wc, dev_src, dev_gimg,
-                                    dev_gplanes, dev_gsky, accumulate != 0, part, FS_PARTIALS,
+                                    dev_gplanes, dev_gsky, accumulate != 0, part, FSK_PARTIALS,
                                     ctx->stream));
     else if (!accumulate)
         HIPCHECK(ctx, fsk_zero_f32(dev_gsky, 1, ctx->stream));
@@ -1724,20 +1723,19 @@ static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
     }
     const size_t nplanes = (size_t)3 * (size_t)hc * (size_t)wc;
     /* the loss and sky partials take half of the scratch each */
-    if (step_blocks(view->w, view->h) > FS_PARTIALS / 2) {
+    if (step_blocks(view->w, view->h) > FSK_LIMIT_BLOCKS / 2) {
         set_error(ctx, "%s: a %d x %d frame has %lld blocks of %d x %d pixels, more than the "
                   "%d loss partial sums of the fused step", what, view->w, view->h,
                   (long long)step_blocks(view->w, view->h), FS_STEP_BLOCK_COLS,
-                  fsk_grad_block_rows(view->w, view->h), FS_PARTIALS / 2);
+                  fsk_limit_block_rows(view->w, view->h), FSK_LIMIT_BLOCKS / 2);
         return 1;
     }
-    float *part = NULL;
+    double *part = NULL;
     if (noalloc) {
-        int64_t cap = 0;
-        part = fsk_scratch(ctx->device, &cap);
-        if (!part || cap < FS_PARTIALS) {
-            set_error(ctx, "%s: the device scratch of %lld floats is not set up", what,
-                      (long long)cap);
+        part = fsk_scratch(ctx->device);
+        if (!part) {
+            set_error(ctx, "%s: the device scratch of %d doubles is not set up", what,
+                      FSK_PARTIALS);
             return 1;
         }
     }
@@ -1773,7 +1771,7 @@ static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
         HIPCHECK(ctx, fsk_zero_f32(dev_gplanes, nplanes, ctx->stream));
     /* colour, loss terms and adjoint in one launch; the loss and sky
      * partials take the scratch's two halves */
-    const int32_t q = FS_PARTIALS / 2;
+    const int32_t q = FSK_PARTIALS / 2;
     HIPCHECK(ctx, fsk_diff_step_l2(&f, dev_planes, dev_sf, hc, wc, sky_scale, dev_src, dev_target,
                                    dev_img, dev_gimg, dev_gplanes, dev_gsky, accumulate != 0,
                                    dev_loss, accumulate != 0, part, part + q, q, ctx->stream));
@@ -1836,11 +1834,11 @@ int fsx_l2_loss(struct futhark_context *ctx, const float *dev_img, const float *
         return 1;
     }
     HIPCHECK(ctx, hipSetDevice(ctx->device));
-    float *part;
+    double *part;
     if (partials(ctx, &part))
         return 1;
     HIPCHECK(ctx, fsk_l2_loss(dev_img, dev_target, (size_t)n, dev_grad, dev_loss, accumulate, part,
-                              FS_PARTIALS, ctx->stream));
+                              FSK_PARTIALS, ctx->stream));
     return 0;
 }
 

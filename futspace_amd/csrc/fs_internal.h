@@ -50,10 +50,10 @@ int32_t fsk_frame_tame(const fsk_frame *f);
  * later calls on the same device return at once. */
 int fsk_device_init(void);
 
-/* The device address of `device`'s fixed scratch array (set up by
- * fsk_device_init; NULL before) and its size in floats.  Shared by every
- * caller on that device. */
-float *fsk_scratch(int32_t device, int64_t *n_floats);
+/* The device address of `device`'s fixed scratch array of FSK_PARTIALS
+ * doubles (set up by fsk_device_init; NULL before).  Shared by every caller
+ * on that device. */
+double *fsk_scratch(int32_t device);
 
 /* render2 (ray march) of one frame into out[rows][pitch]: d_cs/d_sn[cols]
  * the host's cos / sin of angle + horz_ang per column, d_color the map's
@@ -81,9 +81,13 @@ int fsk_render(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t, uint32
  * in bands of rows), and the rows of a batched view. */
 int32_t fsk_render_max_rows(void);
 int32_t fsk_batch_max_rows(void);
-/* Pixel rows of one adjoint workgroup's 64-column block in a w x h frame
- * (16, or 32 in frames of 2^22 pixels or more); one partial sum per block. */
-int32_t fsk_grad_block_rows(int32_t w, int32_t h);
+/* The differentiable passes' limit on frames counts blocks of 64 columns by
+ * this many rows (16, or 32 in frames of 2^22 pixels or more).  The adjoint's
+ * own workgroups cover half as many rows each or more, and leave one partial
+ * sum each: FSK_PARTIALS holds two for every block of the largest frame. */
+int32_t fsk_limit_block_rows(int32_t w, int32_t h);
+#define FSK_LIMIT_BLOCKS 32768
+#define FSK_PARTIALS (2 * FSK_LIMIT_BLOCKS)
 
 /* One view of a batched render, as the persistent kernel reads it. */
 typedef struct {
@@ -161,7 +165,7 @@ int fsk_diff_color(const fsk_frame *f, const float *d_cp, const float *d_sf, int
                    int32_t wc, float sky_scale, const int32_t *d_src, float *d_img, hipStream_t s);
 int fsk_diff_grad(const fsk_frame *f, const float *d_cp, const float *d_sf, int32_t hc,
                   int32_t wc, const int32_t *d_src, const float *d_gimg, float *d_gcp,
-                  float *d_gsky, int32_t sky_accumulate, float *d_partials, int32_t n_partials,
+                  float *d_gsky, int32_t sky_accumulate, double *d_partials, int32_t n_partials,
                   hipStream_t s);
 /* The fused L2 step after the slice render: for each pixel the colour px
  * (written to d_img if not null), g = 2 (px - d_tgt) (written to d_g if not
@@ -173,7 +177,7 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
                      int32_t wc, float sky_scale, const int32_t *d_src, const float *d_tgt,
                      float *d_img, float *d_g, float *d_gcp, float *d_gsky,
                      int32_t sky_accumulate, float *d_loss, int32_t loss_accumulate,
-                     float *d_loss_part, float *d_sky_part, int32_t n_partials, hipStream_t s);
+                     double *d_loss_part, double *d_sky_part, int32_t n_partials, hipStream_t s);
 int fsk_zero_f32(float *d_p, size_t n, hipStream_t s);
 /* One bias-corrected Adam step (step t >= 1) on d_p[n] with gradient d_g
  * and moments d_m, d_v, then d_p clamped to [lo, hi]. */
@@ -185,7 +189,7 @@ int fsk_fill_u32(uint32_t *d_p, size_t n, uint32_t v, hipStream_t s);
  * n_partials) and a one-workgroup pass adds their sum, in a fixed order,
  * to the scalar: no atomics on the scalar, reproducible results. */
 int fsk_l2_loss(const float *d_img, const float *d_tgt, size_t n, float *d_g, float *d_loss,
-                int32_t accumulate, float *d_partials, int32_t n_partials, hipStream_t s);
+                int32_t accumulate, double *d_partials, int32_t n_partials, hipStream_t s);
 
 #ifdef __cplusplus
 }

@@ -476,11 +476,10 @@ __device__ __forceinline__ uint32_t mix_channel_exact(float m1, float s1, float 
  * checked against the sqrt sequence for every f32 in [0, 1] by the device
  * self-test. */
 /* Scratch of the allocation-free fused step (fsx_render_f32_l2_step_noalloc):
- * per-workgroup partial sums, kScratchFloats floats per device, held until
+ * per-workgroup partial sums, FSK_PARTIALS doubles per device, held until
  * the process ends.  Host code reaches it only through the address
  * hipGetSymbolAddress returns for the current device (fsk_scratch). */
-constexpr int kScratchFloats = 32768;
-static __device__ __align__(256) float scratch[kScratchFloats];
+static __device__ __align__(256) double scratch[FSK_PARTIALS];
 
 constexpr uint32_t kQLo = 0x37810000u;           /* below sqrt(t) * 255 >= 1 */
 constexpr int kQBuckets = 2048;                  /* (bits(1.0f) - kQLo) >> 16 = 2047 */
@@ -2160,23 +2159,23 @@ hipError_t launch_batch(const fsk_batch *fb, hipStream_t s)
  * (argb.scale of 0xFF9090e0, fut/interactive.fut:163). */
 
 
-/* Sum of n per-workgroup partials in a fixed order by one workgroup of NT
- * threads, stored into *dst or added to it: thread t adds part[t],
- * part[t + NT], ... in that order (eight loads issued before the first
- * add), then the wave totals are added in wave order.  Every thread of the
- * workgroup must call it. */
-template <int NT>
-__device__ __forceinline__ void block_sum_partials(const float *__restrict__ part, int32_t n,
+/* Sum of n per-workgroup partials (f32 or f64) in f64 and in a fixed order
+ * by one workgroup of NT threads, stored into *dst or added to it: thread t
+ * adds part[t], part[t + NT], ... in that order (eight loads issued before
+ * the first add), then the wave totals are added in wave order.  Every
+ * thread of the workgroup must call it. */
+template <int NT, typename T>
+__device__ __forceinline__ void block_sum_partials(const T *__restrict__ part, int32_t n,
                                                    float *__restrict__ dst, int32_t accumulate)
 {
-    __shared__ float wsum[NT / 64];
-    float acc = 0.0f;
+    __shared__ double wsum[NT / 64];
+    double acc = 0.0;
     for (int32_t base = 0; base < n; base += 8 * NT) {
-        float v[8];
+        T v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int32_t i = base + u * NT + (int32_t)threadIdx.x;
-            v[u] = i < n ? part[i] : 0.0f;
+            v[u] = i < n ? part[i] : (T)0;
         }
 #pragma unroll
         for (int u = 0; u < 8; u++)
@@ -2189,10 +2188,10 @@ __device__ __forceinline__ void block_sum_partials(const float *__restrict__ par
         wsum[threadIdx.x >> 6] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
-        float t = 0.0f;
+        double t = 0.0;
         for (int w = 0; w < NT / 64; w++)
             t += wsum[w];
-        *dst = accumulate ? *dst + t : t;
+        *dst = accumulate ? *dst + (float)t : (float)t;
     }
 }
 
@@ -2207,10 +2206,10 @@ struct DiffArgs {
     float *img;            /* forward output [3][rows][cols] */
     float *gcp;            /* backward: dL/dcp accumulated [3][hc][wc] */
     float *gsky;           /* backward: dL/dsky_scale accumulated */
-    float *partials;       /* per-workgroup partial sums (loss or sky) */
+    double *partials;      /* per-workgroup partial sums (loss or sky) */
     const float *tgt;      /* fused step: the target frame [3][rows][cols] */
     float *gout;           /* fused step: dL/dimg written out (may be null) */
-    float *sky_part;       /* fused step: per-workgroup sky terms */
+    double *sky_part;      /* fused step: per-workgroup sky terms */
 };
 
 /* The relaxed argb.mix channel: sqrt(m1' a^2 + m2' b^2) with weights
@@ -2466,12 +2465,20 @@ __device__ __forceinline__ bool segment_sum_quad(const uint32_t key[4], float (&
         for (int c = 0; c < 3; c++)
             v[t * 3 + c] = val[t][c];
     int32_t f = same_prev ? 0 : 1;
+    /* once every lane's range holds its segment's first lane the later
+     * steps change nothing: most segments are two or three lanes long */
     segment_step<0x111, 0xf>(v, f);            /* row_shr:1 */
-    segment_step<0x112, 0xf>(v, f);            /* row_shr:2 */
-    segment_step<0x114, 0xf>(v, f);            /* row_shr:4 */
-    segment_step<0x118, 0xf>(v, f);            /* row_shr:8 */
-    segment_step<0x142, 0xa>(v, f);            /* row_bcast:15 */
-    segment_step<0x143, 0xc>(v, f);            /* row_bcast:31 */
+    if (__ballot(!f)) {
+        segment_step<0x112, 0xf>(v, f);        /* row_shr:2 */
+        if (__ballot(!f)) {
+            segment_step<0x114, 0xf>(v, f);    /* row_shr:4 */
+            if (__ballot(!f)) {
+                segment_step<0x118, 0xf>(v, f);    /* row_shr:8 */
+                segment_step<0x142, 0xa>(v, f);    /* row_bcast:15 */
+                segment_step<0x143, 0xc>(v, f);    /* row_bcast:31 */
+            }
+        }
+    }
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -2480,39 +2487,50 @@ __device__ __forceinline__ bool segment_sum_quad(const uint32_t key[4], float (&
     return !same_next;
 }
 
-constexpr int kGradThreads = 512;
+/* Workgroups of the adjoint: 64 columns by 4 waves, with a table of 1024
+ * texels each (28 KiB), so that five of them share a CU.  512 threads with
+ * 2048 texels: two per CU, 1900 x 1000 98 against 89 us per fused step; 128
+ * with 512: 94 us. */
+constexpr int kGradThreads = 256;
 /* Rows per thread in the adjoint: 2, or 4 in frames of kGradTallPixels
  * pixels or more.  A run of equal src down a thread's rows is merged in
  * registers, so more rows mean fewer texel inserts per pixel, which pays
- * where the adjoint is bound by its VALU work (3840 x 2160: 16.3 against
- * 18.2 ms per fitting step), while smaller frames need the waves of the
- * shorter blocks to hide their gathers' latency (1280 x 720: 78 against
- * 91 us per fused step). */
+ * where there are many workgroups per CU (3840 x 2160: 213 against 222 us
+ * per fused step), while smaller frames need the waves (1280 x 720: 72
+ * against 86 us). */
 constexpr int64_t kGradTallPixels = (int64_t)1 << 22;
-constexpr int kGradCapLog = 12;
+constexpr int kGradCapLog = 10;
 constexpr int kGradCap = 1 << kGradCapLog;   /* texel slots of a workgroup's LDS table */
-constexpr int kGradProbes = 2;
+constexpr int kGradFill = kGradCap / 8 * 7;  /* slots taken before new texels go past it */
+constexpr int kGradProbes = 4;
+constexpr int kGradRunLog = 4;               /* texels of a row that hash to adjacent slots */
 
-/* Add v[0..2] to texel `key` of the workgroup's LDS table (open addressing,
- * linear probing); returns whether this call took a new slot.  A texel that
- * finds no slot within kGradProbes, or any texel once half of the table
- * is taken (far-range blocks, where every sample has texels of its own),
- * goes straight to the global gradient.  The global f32 atomics are what
- * bounds the adjoint at 1280 x 720: stopping at a quarter of the table
- * had the fused step at 74 against 68 us. */
-template <int CAPLOG = kGradCapLog, int FILL_LIMIT = kGradCap / 2, int PROBES = kGradProbes>
-__device__ __forceinline__ bool table_add(uint32_t *keys, float *vals, const uint32_t *fill,
+/* Add v[0..2] to texel `key` of the workgroup's LDS table (open addressing);
+ * returns whether this call took a new slot.  A texel that finds no slot
+ * within kGradProbes, or any new texel once kGradFill slots are taken, goes
+ * straight to the global gradient.
+ *
+ * The sums are f64: an LDS f32 add takes 3 cycles per lane on this chip
+ * (193 per wave, whatever the addresses), an f64 one 9 per wave.  With f32
+ * sums the adds had bound the adjoint (72 of 98 us of a 1900 x 1000 step).
+ *
+ * The hash keeps runs of 2^kGradRunLog texels of a row together: adjacent
+ * slots, which adjacent lanes flush, are then adjacent in memory, and a
+ * wave's global atomics come as a few lines instead of one per lane
+ * (1280 x 720: 94 -> 81 us per fused step; the flush no longer shows). */
+__device__ __forceinline__ bool table_add(uint32_t *keys, double *vals, const uint32_t *fill,
                                           float *gcp, size_t plane, uint32_t key, const float v[3])
 {
-    constexpr int kCap = 1 << CAPLOG;
-    uint32_t h = (key * 2654435761u) >> (32 - CAPLOG);
+    constexpr uint32_t kRun = 1u << kGradRunLog;
+    uint32_t h = (((key >> kGradRunLog) * 2654435761u) >> (32 - kGradCapLog + kGradRunLog)) * kRun +
+                 (key & (kRun - 1u));
     /* a relaxed atomic load, which becomes an LDS read: a volatile read
      * through this generic pointer was a flat load that waited for every
      * global atomic of the wave still in flight */
     const bool open = __hip_atomic_load(fill, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <
-                      (uint32_t)FILL_LIMIT;
+                      (uint32_t)kGradFill;
 #pragma unroll 1
-    for (int p = 0; open && p < PROBES; p++) {
+    for (int p = 0; open && p < kGradProbes; p++) {
         uint32_t k = keys[h];
         bool mine = false;
         if (k == kNoKey) {
@@ -2523,10 +2541,11 @@ __device__ __forceinline__ bool table_add(uint32_t *keys, float *vals, const uin
 #pragma unroll
             for (int ch = 0; ch < 3; ch++)
                 if (v[ch] != 0.0f)
-                    atomicAdd(&vals[ch * kCap + h], v[ch]);
+                    __hip_atomic_fetch_add(&vals[ch * kGradCap + h], (double)v[ch],
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             return mine;
         }
-        h = (h + 1) & (kCap - 1);
+        h = (h + kRun) & (kGradCap - 1);
     }
 #pragma unroll
     for (int ch = 0; ch < 3; ch++)
@@ -2592,8 +2611,8 @@ __device__ __forceinline__ void sample_terms(const DiffArgs &a, int32_t k, int32
     sample_grad(a, e, run, key, val);
 }
 
-/* Adjoint.  A workgroup covers 64 adjacent columns x 16 rows; each thread
- * holds kGradRows rows of one column.  A run of equal src down the column
+/* Adjoint.  A workgroup covers 64 adjacent columns x 4 kGradRows rows; each
+ * thread holds kGradRows rows of one column.  A run of equal src down the column
  * is one visible sample: its incoming gradient is summed in registers and
  * pushed through the three mixes once.  For px = mix(wy0, X1, wy1, X2),
  * X1 = mix(wx0, s0, wx1, s1): d px / d s0 = wy0' * wx0' * s0 / px (X1
@@ -2603,7 +2622,7 @@ __device__ __forceinline__ void sample_terms(const DiffArgs &a, int32_t k, int32
  * columns magnifying one near texel) are merged by a segmented reduction
  * across the wave, so that the LDS table below sees distinct texels per
  * instruction; then an LDS hash table sums the terms per texel over the
- * whole 64 x 16 block (neighbouring samples share texels: a block touches
+ * whole block (neighbouring samples share texels: a block touches
  * several times fewer texels than it has sample-texel terms).  Short
  * per-thread row runs keep many waves in flight for the gathers.  Each
  * table entry is then added into the global f32 gradient with one atomic
@@ -2622,13 +2641,13 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
 {
     constexpr int kGradBlockRows = (kGradThreads / 64) * kGradRows;
     __shared__ uint32_t keys[kGradCap];
-    __shared__ float vals[3 * kGradCap];
+    __shared__ double vals[3 * kGradCap];
     __shared__ uint32_t fill;
     for (int32_t i = threadIdx.x; i < kGradCap; i += kGradThreads) {
         keys[i] = kNoKey;
-        vals[i] = 0.0f;
-        vals[kGradCap + i] = 0.0f;
-        vals[2 * kGradCap + i] = 0.0f;
+        vals[i] = 0.0;
+        vals[kGradCap + i] = 0.0;
+        vals[2 * kGradCap + i] = 0.0;
     }
     if (threadIdx.x == 0)
         fill = 0u;
@@ -2654,7 +2673,10 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
             g[ch][j] = in ? gin[ch * fplane + p] : 0.0f;
     }
     __syncthreads();
-    float sky_acc = 0.0f, loss_acc = 0.0f;
+    /* the sky term cancels where gradients of both signs meet: f64 keeps its
+     * sum as exact as the gradients */
+    double sky_acc = 0.0;
+    float loss_acc = 0.0f;
     float run[3] = {0.0f, 0.0f, 0.0f};
     SampleEval e;              /* FWD: the current run's sample */
 #pragma unroll
@@ -2691,10 +2713,10 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
         for (int ch = 0; ch < 3; ch++)
             run[ch] += g[ch][j];
         const bool ends = (j == kGradRows - 1 || src[j + 1] != k) && k != INT32_MIN;
-        if (ends && k < 0) {
+        if (k < 0 && k != INT32_MIN) {
 #pragma unroll
             for (int ch = 0; ch < 3; ch++)
-                sky_acc += run[ch] * sky_base(ch);
+                sky_acc += (double)g[ch][j] * (double)sky_base(ch);
         }
         const bool flush = ends && k >= 0;
         if (__ballot(flush)) {
@@ -2727,7 +2749,8 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
         }
     }
     /* per-workgroup partials, summed in a fixed order by the next launch */
-    __shared__ float wsky[kGradThreads / 64], wloss[kGradThreads / 64];
+    __shared__ double wsky[kGradThreads / 64];
+    __shared__ float wloss[kGradThreads / 64];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         sky_acc += __shfl_xor(sky_acc, off);
@@ -2742,7 +2765,7 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
     __syncthreads();
     if (threadIdx.x == 0) {
         const int32_t blk = blockIdx.y * gridDim.x + blockIdx.x;
-        float t = 0.0f, tl = 0.0f;
+        double t = 0.0, tl = 0.0;
         for (int w = 0; w < kGradThreads / 64; w++) {
             t += wsky[w];
             if (FWD)
@@ -2761,7 +2784,7 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
             continue;
 #pragma unroll
         for (int ch = 0; ch < 3; ch++) {
-            const float v = vals[ch * kGradCap + i];
+            const float v = (float)vals[ch * kGradCap + i];
             if (v != 0.0f)
                 unsafeAtomicAdd(&a.gcp[ch * plane + key], v);
         }
@@ -2772,21 +2795,21 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
  * partials into *gsky (= or +=), each in block_sum_partials' order (so
  * bit-identical to two calls of it), the two arrays' loads, shuffles and
  * final adds interleaved so that their latencies overlap. */
-__global__ __launch_bounds__(1024) void k_sum_step(const float *__restrict__ loss_part,
-                                                   const float *__restrict__ sky_part, int32_t n,
+__global__ __launch_bounds__(1024) void k_sum_step(const double *__restrict__ loss_part,
+                                                   const double *__restrict__ sky_part, int32_t n,
                                                    float *__restrict__ loss, int32_t loss_acc,
                                                    float *__restrict__ gsky, int32_t sky_acc)
 {
     constexpr int NT = 1024;
-    __shared__ float wsum[2][NT / 64];
-    float a = 0.0f, b = 0.0f;
+    __shared__ double wsum[2][NT / 64];
+    double a = 0.0, b = 0.0;
     for (int32_t base = 0; base < n; base += 8 * NT) {
-        float va[8], vb[8];
+        double va[8], vb[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             const int32_t i = base + u * NT + (int32_t)threadIdx.x;
-            va[u] = i < n ? loss_part[i] : 0.0f;
-            vb[u] = i < n ? sky_part[i] : 0.0f;
+            va[u] = i < n ? loss_part[i] : 0.0;
+            vb[u] = i < n ? sky_part[i] : 0.0;
         }
 #pragma unroll
         for (int u = 0; u < 8; u++) {
@@ -2806,11 +2829,11 @@ __global__ __launch_bounds__(1024) void k_sum_step(const float *__restrict__ los
     __syncthreads();
     if (threadIdx.x == 0 || threadIdx.x == 64) {
         const int k = threadIdx.x >> 6;
-        float t = 0.0f;
+        double t = 0.0;
         for (int w = 0; w < NT / 64; w++)
             t += wsum[k][w];
         float *dst = k ? gsky : loss;
-        *dst = (k ? sky_acc : loss_acc) ? *dst + t : t;
+        *dst = (k ? sky_acc : loss_acc) ? *dst + (float)t : (float)t;
     }
 }
 
@@ -2896,7 +2919,8 @@ __global__ __launch_bounds__(256) void k_adam(float *__restrict__ p, const float
     }
 }
 
-__global__ __launch_bounds__(1024) void k_sum_partials(const float *__restrict__ part, int32_t n,
+template <typename T>
+__global__ __launch_bounds__(1024) void k_sum_partials(const T *__restrict__ part, int32_t n,
                                                        float *__restrict__ dst, int32_t accumulate)
 {
     block_sum_partials<1024>(part, n, dst, accumulate);
@@ -2959,7 +2983,7 @@ void qtab_build(uint32_t *qt)
 
 std::mutex g_init_mu;
 bool g_init_done[64];
-float *g_scratch_ptr[64];    /* device address of `scratch` on each device */
+double *g_scratch_ptr[64];   /* device address of `scratch` on each device */
 
 }  // namespace
 
@@ -2991,16 +3015,14 @@ int fsk_device_init(void)
         e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess)
             return e;
-        g_scratch_ptr[dev] = (float *)p;
+        g_scratch_ptr[dev] = (double *)p;
         g_init_done[dev] = true;
     }
     return hipSuccess;
 }
 
-float *fsk_scratch(int32_t device, int64_t *n_floats)
+double *fsk_scratch(int32_t device)
 {
-    if (n_floats)
-        *n_floats = kScratchFloats;
     if (device < 0 || device >= 64)
         return nullptr;
     std::lock_guard<std::mutex> lock(g_init_mu);
@@ -3108,6 +3130,12 @@ int fsk_render_slices(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t,
     return fsk_render_slices_clear(m, f, t, d_src, pitch, nullptr, 0, nullptr, s);
 }
 
+/* Rows per thread of the adjoint on a w x h frame. */
+static int32_t grad_rows(int32_t w, int32_t h)
+{
+    return (int64_t)w * (int64_t)h >= kGradTallPixels ? 4 : 2;
+}
+
 static DiffArgs diff_args(const fsk_frame *f, const float *cp, const float *sf, int32_t hc,
                           int32_t wc, const int32_t *src)
 {
@@ -3171,8 +3199,10 @@ int fsk_diff_color(const fsk_frame *f, const float *d_cp, const float *d_sf, int
 }
 
 int fsk_l2_loss(const float *d_img, const float *d_tgt, size_t n, float *d_g, float *d_loss,
-                int32_t accumulate, float *d_partials, int32_t n_partials, hipStream_t s)
+                int32_t accumulate, double *d_partials, int32_t n_partials, hipStream_t s)
 {
+    /* one f32 per workgroup */
+    float *part = (float *)d_partials;
     size_t blocks = (n / 4 + 255) / 256;
     if (blocks > 4096)
         blocks = 4096;
@@ -3181,8 +3211,8 @@ int fsk_l2_loss(const float *d_img, const float *d_tgt, size_t n, float *d_g, fl
     if ((int64_t)blocks > n_partials)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_l2_loss, dim3((unsigned)blocks), dim3(256), 0, s, d_img, d_tgt, n, d_g,
-                       d_partials);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, d_partials, (int32_t)blocks,
+                       part);
+    hipLaunchKernelGGL(k_sum_partials<float>, dim3(1), dim3(1024), 0, s, part, (int32_t)blocks,
                        d_loss, accumulate);
     return hipGetLastError();
 }
@@ -3238,7 +3268,7 @@ int fsk_zero_f32(float *d_p, size_t n, hipStream_t s)
 
 int fsk_diff_grad(const fsk_frame *f, const float *d_cp, const float *d_sf, int32_t hc,
                   int32_t wc, const int32_t *d_src, const float *d_gimg, float *d_gcp,
-                  float *d_gsky, int32_t sky_accumulate, float *d_partials, int32_t n_partials,
+                  float *d_gsky, int32_t sky_accumulate, double *d_partials, int32_t n_partials,
                   hipStream_t s)
 {
     if (f->rows <= 0 || f->cols <= 0)
@@ -3248,15 +3278,15 @@ int fsk_diff_grad(const fsk_frame *f, const float *d_cp, const float *d_sf, int3
     a.gcp = d_gcp;
     a.gsky = d_gsky;
     a.partials = d_partials;
-    const int32_t br = fsk_grad_block_rows(f->cols, f->rows);
+    const int32_t rows = grad_rows(f->cols, f->rows), br = kGradThreads / 64 * rows;
     dim3 grid((f->cols + 63) / 64, (f->rows + br - 1) / br);
     if ((int64_t)grid.x * grid.y > n_partials)
         return hipErrorInvalidValue;
-    const bool p2 = pow2(hc) && pow2(wc), tall = br > 16;
+    const bool p2 = pow2(hc) && pow2(wc), tall = rows == 4;
     void (*kern)(DiffArgs) = p2 ? (tall ? k_diff_grad<true, false, 4> : k_diff_grad<true, false, 2>)
                                 : (tall ? k_diff_grad<false, false, 4> : k_diff_grad<false, false, 2>);
     hipLaunchKernelGGL(kern, grid, dim3(kGradThreads), 0, s, a);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(1024), 0, s, d_partials,
+    hipLaunchKernelGGL(k_sum_partials<double>, dim3(1), dim3(1024), 0, s, d_partials,
                        (int32_t)(grid.x * grid.y), d_gsky, sky_accumulate);
     return hipGetLastError();
 }
@@ -3265,7 +3295,7 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
                      int32_t wc, float sky_scale, const int32_t *d_src, const float *d_tgt,
                      float *d_img, float *d_g, float *d_gcp, float *d_gsky,
                      int32_t sky_accumulate, float *d_loss, int32_t loss_accumulate,
-                     float *d_loss_part, float *d_sky_part, int32_t n_partials, hipStream_t s)
+                     double *d_loss_part, double *d_sky_part, int32_t n_partials, hipStream_t s)
 {
     if (f->rows <= 0 || f->cols <= 0)
         return hipSuccess;
@@ -3278,12 +3308,12 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
     a.gsky = d_gsky;
     a.partials = d_loss_part;
     a.sky_part = d_sky_part;
-    const int32_t br = fsk_grad_block_rows(f->cols, f->rows);
+    const int32_t rows = grad_rows(f->cols, f->rows), br = kGradThreads / 64 * rows;
     dim3 grid((f->cols + 63) / 64, (f->rows + br - 1) / br);
     const int64_t nb = (int64_t)grid.x * grid.y;
     if (nb > n_partials)
         return hipErrorInvalidValue;
-    const bool p2 = pow2(hc) && pow2(wc), tall = br > 16;
+    const bool p2 = pow2(hc) && pow2(wc), tall = rows == 4;
     void (*kern)(DiffArgs) = p2 ? (tall ? k_diff_grad<true, true, 4> : k_diff_grad<true, true, 2>)
                                 : (tall ? k_diff_grad<false, true, 4> : k_diff_grad<false, true, 2>);
     hipLaunchKernelGGL(kern, grid, dim3(kGradThreads), 0, s, a);
@@ -3360,9 +3390,9 @@ int32_t fsk_batch_max_rows(void)
     return kMaxRows;
 }
 
-int32_t fsk_grad_block_rows(int32_t w, int32_t h)
+int32_t fsk_limit_block_rows(int32_t w, int32_t h)
 {
-    return (kGradThreads / 64) * ((int64_t)w * (int64_t)h >= kGradTallPixels ? 4 : 2);
+    return (int64_t)w * (int64_t)h >= kGradTallPixels ? 32 : 16;
 }
 
 int fsk_selftest(int which, unsigned long long *d_bad, hipStream_t s)

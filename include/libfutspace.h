@@ -229,7 +229,7 @@ int fsx_render_stateless(struct futhark_context *ctx, const int32_t *dev_color,
  * the forward pass; accumulate = 0 clears both first.  f32 atomics: the
  * summation order, hence the last bits, varies from run to run.  Its
  * per-workgroup partial sums limit the frame to ceil(w/64) * ceil(h/b)
- * <= 32768 blocks, b = 16 rows, or 32 in frames of 2^22 pixels or more
+ * <= 32768 blocks of pixels, b = 16 rows, or 32 in frames of 2^22 pixels or more
  * (every frame up to 8192 x 8192); larger frames are refused before
  * anything is enqueued.
  *
@@ -275,9 +275,9 @@ int fsx_adam_step(struct futhark_context *ctx, float *dev_param, const float *de
  * one-workgroup sum of the loss and sky partials.  The loss is summed per
  * workgroup in a fixed order, so the loss of a step is reproducible; the
  * gradients carry the f32-atomic summation order of fsx_render_f32_vjp.
- * The loss and sky partial sums (one each per block of 64 columns by
- * b = 16 rows, or 32 in frames of 2^22 pixels or more) limit the frame to
- * ceil(w/64) * ceil(h/b) <= 16384 blocks (every frame up to 8192 x 4096);
+ * The loss and sky partial sums limit the frame to ceil(w/64) * ceil(h/b)
+ * <= 16384 blocks of pixels, b = 16 rows, or 32 in frames of 2^22 pixels
+ * or more (every frame up to 8192 x 4096);
  * larger frames are refused before anything is enqueued.  Asynchronous
  * on the context stream. */
 int fsx_render_f32_l2_step(struct futhark_context *ctx, const struct fsx_map *map,
@@ -291,8 +291,8 @@ int fsx_render_f32_l2_step(struct futhark_context *ctx, const struct fsx_map *ma
  * reference; it is for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving or training loops).  Same
  * arguments, results and frame limit (16384 blocks, 8192 x 4096);
- * the per-workgroup partial sums live in a fixed scratch array of 32768
- * floats (128 KiB) per device, set up when the first context on the
+ * the per-workgroup partial sums live in a fixed scratch array of 65536
+ * doubles (512 KiB) per device, set up when the first context on the
  * device is created and held until the process ends, instead of the
  * context buffer fsx_render_f32_l2_step allocates on first use.  Every
  * call on a device shares that device's array, so calls that overlap on

@@ -490,3 +490,40 @@ def test_adam_step_matches_torch_adam(ctx):
         r.adam_step(p, grads[0] * 1e4, m, v, 1.0, 4, lo=0.25, hi=0.75)
         torch.cuda.synchronize()
         assert float(p.min()) >= 0.25 and float(p.max()) <= 0.75
+
+
+@pytest.mark.parametrize("h,w,size,zoom", [
+    (7, 1, 128, 1.0), (8, 64, 128, 1.0), (9, 65, 96, 1.0),       # edges of the workgroups
+    (200, 300, 128, 0.02),                                       # every pixel on a few texels
+    (200, 300, 512, 40.0),                                       # every sample on its own texels
+])
+def test_adjoint_table_and_blocks(ctx, h, w, size, zoom):
+    """Gradients of both adjoints against the oracle where a workgroup's
+    texel table holds a few texels, and where it overflows."""
+    col, hts = scene.scene_maps(29, 128)
+    m = ctx.map(col, hts, shade_size=size)
+    r = DiffRenderer(ctx, m)
+    alt = np.asarray(hts, np.int32) & 255
+    sf = O.shade_factor(O.shadow_counts(alt, O.sun(0.1, 0.1), size))
+    rng = np.random.default_rng(h + w + size)
+    planes = rng.random((3, size, size), dtype=np.float32)
+    d, z0 = scene.depth_for(300, 100.0 * zoom)
+    v = View(x=50.3, y=20.7, height=290.0, angle=0.9, horizon=0.1 * h, distance=100.0 * zoom,
+             fov=1.2, h=h, w=w, d=d, z0=z0, scale=h * zoom * 0.3, n_slices=300)
+    tp = torch.from_numpy(planes).cuda()
+    target = torch.from_numpy(rng.random((3, h, w), dtype=np.float32)).cuda()
+    img, src, gp, gs, loss = r.l2_step(tp, 0.4, v, target)
+    gimg = torch.from_numpy(rng.standard_normal((3, h, w)).astype(np.float32)).cuda()
+    gp2, gs2 = r.vjp_raw(tp, src, gimg, v)
+    torch.cuda.synchronize()
+    want_img, want_src = O.render_f32(v, planes, sf, alt, 0.4)
+    assert (want_src >= 0).sum() > h * w // 20
+    assert np.array_equal(img.cpu().numpy().view(np.uint32), want_img.view(np.uint32))
+    g = 2.0 * (want_img - target.cpu().numpy())
+    for got, sky, gi in ((gp, gs, g.astype(np.float32)), (gp2, gs2, gimg.cpu().numpy())):
+        want, want_sky = O.render_f32_vjp(v, planes, sf, want_src, gi)
+        assert _rel_err(got.cpu().numpy(), want) <= 1e-5
+        mass = np.abs(gi[:, want_src < 0]).sum() + 1e-3
+        assert abs(float(sky[0]) - float(want_sky)) <= 1e-5 * mass
+    want_loss = float(((want_img.astype(np.float64) - target.cpu().numpy()) ** 2).sum())
+    assert abs(float(loss[0]) - want_loss) <= 1e-5 * want_loss
