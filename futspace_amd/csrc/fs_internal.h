@@ -23,6 +23,7 @@ typedef struct {
     int32_t hrows, hcols, hbits;
     const void *cq;
     int32_t crows, ccols;
+    float rhrows, rhcols, rcrows, rccols;   /* fsk_map_recips; set by the launchers */
 } fsk_map;
 
 /* Per-frame scalars, computed on the host exactly as `futhark c` does:
@@ -36,14 +37,22 @@ typedef struct {
     float rfw;           /* 1 / fw, correctly rounded (the host's f32 division) */
     int32_t n, rows, cols;
     uint32_t sky;
-    int32_t tame;        /* fsk_frame_tame(this); set by the launchers */
+    int32_t tame;        /* fsk_frame_tame; set by the launchers */
 } fsk_frame;
 
-/* 1 when every sample of the frame stays where the render kernel may skip
- * the out-of-range branches of the x86 casts: finite scalars, slice depths
- * increasing from z0 > 0, every sample coordinate below 2^22 and every
- * projected row below 2^30 in magnitude for any 16-bit height. */
-int32_t fsk_frame_tame(const fsk_frame *f);
+/* FSK_TAME when every sample of the frame stays where the render kernel may
+ * skip the out-of-range branches of the x86 casts: finite scalars, slice
+ * depths increasing from z0 > 0, every sample coordinate below 2^22 and every
+ * projected row below 2^30 in magnitude for any 16-bit height.
+ * FSK_TAME_MOD when besides the coordinates are below 2^21 and max_side, the
+ * longest side of the sampled maps, is at most 2^20, so that sides that are
+ * no powers of two may be wrapped by reciprocals.  Else 0. */
+#define FSK_TAME 1
+#define FSK_TAME_MOD 2
+int32_t fsk_frame_tame(const fsk_frame *f, int32_t max_side);
+/* A reciprocal of m a little below 1 / m, for such wraps; a map's four. */
+float fsk_wrap_recip(int32_t m);
+void fsk_map_recips(fsk_map *m);
 
 /* Once per device, before its first render: uploads the kernels' constant
  * tables (the byte quantisation table of the colour path).  Thread-safe;
@@ -126,7 +135,7 @@ void fsk_batch_counters_init(uint32_t *counters, int32_t grid, int32_t nqueues);
 /* Run the persistent batched render. */
 int fsk_batch_run(const fsk_batch *b, hipStream_t s);
 
-/* Device self-test `which` (0-7) of the arithmetic shortcuts; adds the
+/* Device self-test `which` (0-8) of the arithmetic shortcuts; adds the
  * number of mismatching inputs to *d_bad. */
 int fsk_selftest(int which, unsigned long long *d_bad, hipStream_t s);
 

@@ -82,6 +82,20 @@ __device__ __forceinline__ int32_t wrap(int32_t v, int32_t m)
     return POW2 ? (v & (m - 1)) : fmod_i32(v, m);
 }
 
+/* Floor-mod of an integral f32 v, |v| < 2^21, by a side m <= 2^20 that is not
+ * a power of two, with rm a little below 1 / m (fsk_wrap_recip).  v * rm is
+ * then below the quotient, or at it, by less than 2^-21.4 of it, which is less
+ * than 1 / m: its floor is the quotient's floor, or one less where m divides
+ * v.  The remainder, exact in one FMA, is in [0, 2m), and the smaller of it
+ * and it less m (as unsigned) is the result.  Six vector instructions where
+ * the integer modulo takes some thirty; device self-test 8 compares the two. */
+__device__ __forceinline__ int32_t wrap_tame(float v, int32_t m, float rm)
+{
+    const float q = floorf(v * rm);
+    const uint32_t r = (uint32_t)(int32_t)__builtin_fmaf(-q, (float)m, v);
+    return (int32_t)min(r, r - (uint32_t)m);
+}
+
 /* ------------------------------------------------------------------ */
 /* matte argb, as restated for the reference (Gloss mixColors)         */
 /* ------------------------------------------------------------------ */
@@ -190,13 +204,21 @@ typedef uint32_t fs_u32x4 __attribute__((ext_vector_type(4)));
 template <int HBITS, bool HP2, bool TAME = false>
 __device__ __forceinline__ uint2 height_quad(const fsk_map &m, float x, float y)
 {
-    /* TAME: |x|, |y| < 2^22, so floor converts exactly without a clamp */
-    int32_t ix = wrap<HP2>(TAME ? (int32_t)floorf(x) : idx_of(floorf(x)), m.hcols);
-    int32_t iy = wrap<HP2>(TAME ? (int32_t)floorf(y) : idx_of(floorf(y)), m.hrows);
+    /* TAME: |x|, |y| < 2^22 (2^21 where the sides are no powers of two), so
+     * floor converts exactly without a clamp */
+    int32_t ix, iy;
+    if (TAME && !HP2) {
+        ix = wrap_tame(floorf(x), m.hcols, m.rhcols);
+        iy = wrap_tame(floorf(y), m.hrows, m.rhrows);
+    } else {
+        ix = wrap<HP2>(TAME ? (int32_t)floorf(x) : idx_of(floorf(x)), m.hcols);
+        iy = wrap<HP2>(TAME ? (int32_t)floorf(y) : idx_of(floorf(y)), m.hrows);
+    }
     /* maps are at most 2^28 texels (host-checked), so 32-bit offsets; the
      * wrapped index is always inside the map, whatever x and y are */
     uint32_t t = HP2 ? ((uint32_t)iy << __builtin_ctz((uint32_t)m.hcols)) + (uint32_t)ix
-                     : (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
+                 : TAME ? __umul24((uint32_t)iy, (uint32_t)m.hcols) + (uint32_t)ix
+                        : (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
     const FS_GLOBAL char *hq = (const FS_GLOBAL char *)m.hq;
     if (HBITS == 8)
         return make_uint2(*(const FS_GLOBAL uint32_t *)(hq + t * 4u), 0u);
@@ -540,10 +562,17 @@ __device__ __forceinline__ uint32_t color_fast(uint4 q, const float *sq, float w
  * another sum (a coordinate within 1 of the map origin); such waves, and
  * waves with translucent texels, take the general path below. */
 template <bool CP2>
-__device__ __forceinline__ uint4 color_quad(const fsk_map &m, float x, float y)
+__device__ __forceinline__ uint4 color_quad(const fsk_map &m, float x, float y,
+                                            int32_t tame = 0)
 {
-    int32_t ix = wrap<CP2>(idx_of(floorf(x)), m.ccols);
-    int32_t iy = wrap<CP2>(idx_of(floorf(y)), m.crows);
+    int32_t ix, iy;
+    if (!CP2 && tame >= FSK_TAME_MOD) {
+        ix = wrap_tame(floorf(x), m.ccols, m.rccols);
+        iy = wrap_tame(floorf(y), m.crows, m.rcrows);
+    } else {
+        ix = wrap<CP2>(idx_of(floorf(x)), m.ccols);
+        iy = wrap<CP2>(idx_of(floorf(y)), m.crows);
+    }
     /* colour maps have at most 65536^2 texels (host-checked), so the quad
      * index fits 32 bits; the byte offset is formed in 64 */
     uint32_t t = CP2 ? ((uint32_t)iy << __builtin_ctz((uint32_t)m.ccols)) + (uint32_t)ix
@@ -717,10 +746,17 @@ __device__ __forceinline__ uint32_t painted_value(uint32_t v, bool sky_cell, uin
 }
 
 /* Texel index of the stateless program's sample at (x, y): i32.f32 of
- * each coordinate (x86 truncation), floor-mod by the map size. */
-template <bool P2>
+ * each coordinate (x86 truncation), floor-mod by the map size.  TAME as in
+ * height_quad. */
+template <bool P2, bool TAME = false>
 __device__ __forceinline__ uint32_t nearest_index(const fsk_map &m, float x, float y)
 {
+    if (TAME && P2)
+        return (uint32_t)wrap<P2>((int32_t)y, m.hrows) * (uint32_t)m.hcols +
+               (uint32_t)wrap<P2>((int32_t)x, m.hcols);
+    if (TAME)
+        return __umul24((uint32_t)wrap_tame(truncf(y), m.hrows, m.rhrows), (uint32_t)m.hcols) +
+               (uint32_t)wrap_tame(truncf(x), m.hcols, m.rhcols);
     int32_t ix = wrap<P2>(i32_f32_x86(x), m.hcols);
     int32_t iy = wrap<P2>(i32_f32_x86(y), m.hrows);
     return (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
@@ -909,7 +945,8 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                     izs[u] = tzg[(j0 + u) * SG];
                     if (MODE == kOutNearest)
                         qs[u] = make_uint2(
-                            ((const uint32_t *)m.hq)[nearest_index<HP2>(m, xs[u], ys[u])], 0u);
+                            ((const uint32_t *)m.hq)[nearest_index<HP2, TAME>(m, xs[u], ys[u])],
+                            0u);
                     else
                         qs[u] = height_quad<HBITS, HP2, TAME>(m, xs[u], ys[u]);
                 }
@@ -919,12 +956,14 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                     float hgt = MODE == kOutNearest ? (float)(int32_t)qs[u].x
                                                     : height_interp<HBITS>(qs[u], xs[u], ys[u]);
                     float rel = ((f.cam_h - hgt) * izs[u]) + f.horizon;
-                    /* a tame frame keeps |rel| < 2^30: the cast of the
-                     * clamped value is the whole x86 semantics */
-                    int32_t r = TAME || BAND ? (int32_t)__builtin_amdgcn_fmed3f(rel, topf, Hf)
+                    /* a tame frame keeps |rel| < 2^30 (the stateless program's
+                     * heights are unbounded): the cast of the clamped value
+                     * is the whole x86 semantics */
+                    constexpr bool ROWS = TAME && MODE != kOutNearest;
+                    int32_t r = ROWS || BAND ? (int32_t)__builtin_amdgcn_fmed3f(rel, topf, Hf)
                                              : screen_row_clamped(rel, Hf);
                     if (BAND)
-                        r = TAME || rel < 2147483648.0f ? r - row0 : 0;
+                        r = ROWS || rel < 2147483648.0f ? r - row0 : 0;
                     if (j & 1)
                         ah[j / 2] |= (uint32_t)r << 16;
                     else
@@ -933,9 +972,10 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                 }
             }
         };
-        if (MODE != kOutNearest && f.tame && kr == KR)
+        const bool tame = f.tame >= (HP2 ? FSK_TAME : FSK_TAME_MOD);
+        if (tame && kr == KR)
             project(std::true_type{}, std::true_type{});
-        else if (MODE != kOutNearest && f.tame)
+        else if (tame)
             project(std::true_type{}, std::false_type{});
         else
             project(std::false_type{}, std::false_type{});
@@ -1053,7 +1093,7 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                 xs[u] = L.x + (fc * L.z);
                 ys[u] = L.y + (fc * L.w);
                 if (MODE == kOutColour)
-                    cqs[u] = color_quad<CP2>(m, xs[u], ys[u]);
+                    cqs[u] = color_quad<CP2>(m, xs[u], ys[u], f.tame);
             }
 #pragma unroll
             for (int u = 0; u < CBATCH; u++) {
@@ -1662,17 +1702,28 @@ __global__ __launch_bounds__(256) void k_shade(ShadeArgs a)
  * 6: div_rn(a, w, RN(1 / w)) == a / w for every finite f32 a and every
  *    frame width w of kSelftestWidths.
  * 7: sqrt_rn(t) == correctly rounded sqrt(t) for every f32 t >= 0
- *    (+inf included) and NaN stays NaN. */
+ *    (+inf included) and NaN stays NaN.
+ * 8: wrap_tame(v, m) == the floor-mod of v by m for every integer |v| < 2^21
+ *    and every side m of kSelftestSides. */
 constexpr int32_t kSelftestWidths[] = {1920, 1280, 800, 640, 320, 3840, 128, 96, 1024,
                                        2048, 4096, 240, 1, 3, 7, 1000, 1366};
 constexpr int kNSelftestWidths = sizeof kSelftestWidths / sizeof kSelftestWidths[0];
-__global__ void k_selftest(int which, unsigned long long *bad)
+constexpr int32_t kSelftestSides[] = {1, 2, 3, 5, 7, 90, 100, 333, 777, 1000, 1363, 1500,
+                                      4095, 65535, 1048575, 1048576};
+constexpr int kNSelftestSides = sizeof kSelftestSides / sizeof kSelftestSides[0];
+
+struct SelftestRecips {
+    float rm[kNSelftestSides];
+};
+
+__global__ void k_selftest(int which, SelftestRecips recips, unsigned long long *bad)
 {
     uint64_t n = which == 0 ? 256ull
                  : (which == 1 || which == 4) ? 0x3F800001ull
                  : which == 5 ? 0x7E000000ull
                  : which == 7 ? 0x7F800001ull
                  : which == 6 ? (uint64_t)kNSelftestWidths << 32
+                 : which == 8 ? (uint64_t)kNSelftestSides << 22
                               : 0x100000000ull;
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     unsigned long long local = 0;
@@ -1684,6 +1735,10 @@ __global__ void k_selftest(int which, unsigned long long *bad)
             ok = __float_as_uint(sqrt_rn(t)) == __float_as_uint(__builtin_sqrtf(t));
             const float nan = __uint_as_float(0x7FC00000u | (u & 0x3FFFFFu));
             ok = ok && (sqrt_rn(nan) != sqrt_rn(nan));
+        } else if (which == 8) {
+            const int32_t v = (int32_t)(u & 0x3FFFFFu) - (1 << 21), s = (int32_t)(i >> 22);
+            const int32_t m = kSelftestSides[s];
+            ok = v == -(1 << 21) || wrap_tame((float)v, m, recips.rm[s]) == fmod_i32(v, m);
         } else if (which == 5) {
             u += 0x00800000u;
             const float z = __uint_as_float(u);
@@ -2200,6 +2255,7 @@ struct DiffArgs {
     const float *cp;
     const float *sf;
     int32_t hc, wc;
+    float rhc, rwc;        /* fsk_wrap_recip of them */
     float sky_scale;
     const int32_t *src;
     const float *gimg;     /* backward: dL/dimg [3][rows][cols] */
@@ -2286,9 +2342,10 @@ __device__ __forceinline__ void norm_weights(const Bilin &b, float w[4])
  * the host).  P2: both plane sides are powers of two, so the floor-mod is
  * a mask (also for the INT_MIN of an out-of-range cast). */
 template <bool P2, bool TAME = false>
-__device__ __forceinline__ Bilin bilin_of(const fsk_frame &f, int32_t k, int32_t col, int32_t hc,
-                                          int32_t wc)
+__device__ __forceinline__ Bilin bilin_of(const DiffArgs &a, int32_t k, int32_t col)
 {
+    const fsk_frame &f = a.f;
+    const int32_t hc = a.hc, wc = a.wc;
     Slice sl = TAME || f.tame ? slice_params_tame(f, k) : slice_params(f, k);
     float fcol = (float)col;
     float x = sl.sx + (fcol * sl.dx);
@@ -2297,8 +2354,18 @@ __device__ __forceinline__ Bilin bilin_of(const fsk_frame &f, int32_t k, int32_t
     /* TAME: a tame frame keeps |x|, |y| < 2^22, where the x86 conversion
      * is the plain one */
     auto cvt = [](float v) { return TAME ? (int32_t)v : i32_f32_x86(v); };
-    int32_t ify = wrap<P2>(cvt(fy), hc), icy = wrap<P2>(cvt(cy), hc);
-    int32_t ifx = wrap<P2>(cvt(fx), wc), icx = wrap<P2>(cvt(cx), wc);
+    int32_t ify, icy, ifx, icx;
+    if (!P2 && f.tame >= FSK_TAME_MOD) {
+        ify = wrap_tame(fy, hc, a.rhc);
+        icy = wrap_tame(cy, hc, a.rhc);
+        ifx = wrap_tame(fx, wc, a.rwc);
+        icx = wrap_tame(cx, wc, a.rwc);
+    } else {
+        ify = wrap<P2>(cvt(fy), hc);
+        icy = wrap<P2>(cvt(cy), hc);
+        ifx = wrap<P2>(cvt(fx), wc);
+        icx = wrap<P2>(cvt(cx), wc);
+    }
     const uint32_t ry = P2 ? (uint32_t)ify << __builtin_ctz((uint32_t)wc)
                            : (uint32_t)ify * (uint32_t)wc;
     const uint32_t rc = P2 ? (uint32_t)icy << __builtin_ctz((uint32_t)wc)
@@ -2384,7 +2451,7 @@ __global__ __launch_bounds__(256) void k_diff_color(DiffArgs a)
         for (int ch = 0; ch < 3; ch++)
             px[ch] = sky_base(ch) * a.sky_scale;
     } else {
-        const Bilin b = bilin_of<P2, TAME>(a.f, k, col, a.hc, a.wc);
+        const Bilin b = bilin_of<P2, TAME>(a, k, col);
         float sf[4], w[4];
         const bool pairs = __ballot(!b.pair) == 0;
         quad_load(a.sf, b, pairs, sf);
@@ -2569,7 +2636,7 @@ template <bool P2>
 __device__ __forceinline__ void sample_eval(const DiffArgs &a, int32_t k, int32_t col,
                                             size_t plane, SampleEval &e)
 {
-    e.b = bilin_of<P2>(a.f, k, col, a.hc, a.wc);
+    e.b = bilin_of<P2>(a, k, col);
     float cv[3][4];
     sample_gather(a, e.b, plane, cv, e.sf);
     sample_mix(e.b, cv, e.sf, e.sv, e.px);
@@ -3083,6 +3150,11 @@ int fsk_batch_run(const fsk_batch *b, hipStream_t s)
     return b->pow2 ? launch_batch<16, true, true>(b, s) : launch_batch<16, false, false>(b, s);
 }
 
+static int32_t map_side(const fsk_map *m)
+{
+    return std::max(std::max(m->hrows, m->hcols), std::max(m->crows, m->ccols));
+}
+
 int fsk_render_slices_clear(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t,
                             int32_t *d_src, int64_t pitch, float *d_zero, size_t zero_n,
                             int32_t *cleared, hipStream_t s)
@@ -3093,8 +3165,9 @@ int fsk_render_slices_clear(const fsk_map *m, const fsk_frame *f, const fsk_tuni
         return hipSuccess;
     RenderArgs a;
     a.m = *m;
+    fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f);
+    a.f.tame = fsk_frame_tame(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = (uint32_t *)d_src;
@@ -3141,7 +3214,9 @@ static DiffArgs diff_args(const fsk_frame *f, const float *cp, const float *sf, 
 {
     DiffArgs a;
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f);
+    a.f.tame = fsk_frame_tame(f, std::max(hc, wc));
+    a.rhc = fsk_wrap_recip(hc);
+    a.rwc = fsk_wrap_recip(wc);
     a.cp = cp;
     a.sf = sf;
     a.hc = hc;
@@ -3166,8 +3241,9 @@ int fsk_render_nearest(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t
         return hipSuccess;
     RenderArgs a;
     a.m = *m;
+    fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f);
+    a.f.tame = fsk_frame_tame(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = d_out;
@@ -3329,6 +3405,7 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
         return hipSuccess;
     Render2Args a;
     a.m = *m;
+    fsk_map_recips(&a.m);
     a.color = d_color;
     a.cs = d_cs;
     a.sn = d_sn;
@@ -3349,7 +3426,23 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
     return hipGetLastError();
 }
 
-int32_t fsk_frame_tame(const fsk_frame *f)
+float fsk_wrap_recip(int32_t m)
+{
+    /* at most (1 - 2^-24) / m, so that its product with v, rounded, is not
+     * above v / m, and at least (1 - 2^-22) / m */
+    const float r = 1.0f / (float)m;
+    return nextafterf(nextafterf(r, 0.0f), 0.0f);
+}
+
+void fsk_map_recips(fsk_map *m)
+{
+    m->rhrows = fsk_wrap_recip(m->hrows);
+    m->rhcols = fsk_wrap_recip(m->hcols);
+    m->rcrows = m->crows > 0 ? fsk_wrap_recip(m->crows) : 0.0f;
+    m->rccols = m->ccols > 0 ? fsk_wrap_recip(m->ccols) : 0.0f;
+}
+
+int32_t fsk_frame_tame(const fsk_frame *f, int32_t max_side)
 {
     const float v[] = {f->cam_x, f->cam_y, f->cam_h, f->horizon, f->Lx, f->Ly,
                        f->Rx,    f->Ry,    f->d,     f->z0,      f->scale, f->fw};
@@ -3377,7 +3470,9 @@ int32_t fsk_frame_tame(const fsk_frame *f)
     /* slice depths inside [2^-100, 2^100], where the table's reciprocal
      * (rcp_rn) is exact */
     const bool zok = (double)f->z0 >= 0x1p-100 && zmax <= 0x1p100;
-    return zok && xmax < 4194304.0 && ymax < 4194304.0 && relmax < 1073741824.0;
+    if (!(zok && xmax < 4194304.0 && ymax < 4194304.0 && relmax < 1073741824.0))
+        return 0;
+    return xmax < 2097152.0 && ymax < 2097152.0 && max_side <= 1 << 20 ? FSK_TAME_MOD : FSK_TAME;
 }
 
 int32_t fsk_render_max_rows(void)
@@ -3397,9 +3492,12 @@ int32_t fsk_limit_block_rows(int32_t w, int32_t h)
 
 int fsk_selftest(int which, unsigned long long *d_bad, hipStream_t s)
 {
-    if (which < 0 || which > 7)
+    if (which < 0 || which > 8)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_selftest, dim3(4096), dim3(256), 0, s, which, d_bad);
+    SelftestRecips recips;
+    for (int i = 0; i < kNSelftestSides; i++)
+        recips.rm[i] = fsk_wrap_recip(kSelftestSides[i]);
+    hipLaunchKernelGGL(k_selftest, dim3(4096), dim3(256), 0, s, which, recips, d_bad);
     return hipGetLastError();
 }
 
@@ -3410,8 +3508,9 @@ int fsk_render(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t, uint32
         return hipSuccess;
     RenderArgs a;
     a.m = *m;
+    fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f);
+    a.f.tame = fsk_frame_tame(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = d_out;

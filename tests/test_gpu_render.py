@@ -341,3 +341,31 @@ def test_automatic_shapes(ctx, small_scene, w, h, n):
     v = View(x=70.3, y=20.6, height=280.0, angle=2.3, horizon=h * 0.3, distance=500.0, fov=1.2,
              sky_color=sky_color(0.1), h=h, w=w, d=d, z0=z0, scale=h / 2.0, n_slices=n)
     _check(ctx.render(m, v), O.render_painter_mt(v, shaded, alt, 8))
+
+
+def test_reciprocal_floor_mod_selftest(ctx):
+    """The floor-mod of sample coordinates by sides that are no powers of
+    two equals the integer one for every coordinate below 2^21."""
+    import ctypes
+    bad, first = ctypes.c_int64(-1), ctypes.c_int64(-1)
+    ctx.check(ctx.lib.fsx_selftest(ctx.ptr, 8, ctypes.byref(bad), ctypes.byref(first)),
+              "fsx_selftest")
+    assert bad.value == 0, f"{bad.value} mismatches, first input {first.value:#x}"
+
+
+@pytest.mark.parametrize("rows,cols,shade,bits", [(1, 3, 5, 8), (100, 333, 77, 16), (3, 1000, 128, 8),
+                                                  (256, 96, 100, 16), (64, 64, 333, 8)])
+def test_odd_maps_far_and_near(ctx, rows, cols, shade, bits):
+    """Maps and shaded maps whose sides are no powers of two (or only one of
+    the two is), seen from negative coordinates and from beyond the range of
+    the reciprocal floor-mod (2^21) and of the tame frames (2^22)."""
+    rng = np.random.default_rng(rows + cols)
+    hts = rng.integers(0, 200 if bits == 8 else 900, (rows, cols)).astype(np.int32)
+    col = rng.integers(0, 1 << 24, (rows, cols), dtype=np.uint32) | np.uint32(0xFF000000)
+    m = ctx.map(col, hts, height_bits=bits, shade_size=shade)
+    shaded, alt = O.update_map(col, hts, size=shade, bits=bits)
+    for x, y, distance in ((-371.3, 50.2, 300.0), (700000.4, -1500000.3, 500.0),
+                           (3000000.5, 100.25, 300.0), (20.7, 8400000.0, 300.0)):
+        v = View(x=x, y=y, height=350.0, angle=2.1, horizon=30.0, distance=distance, fov=1.2,
+                 sky_color=sky_color(0.1), h=70, w=90, d=0.004, z0=0.5, scale=60.0)
+        _check(ctx.render(m, v), O.render_off(v, shaded, alt))
