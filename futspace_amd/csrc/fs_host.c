@@ -2012,7 +2012,7 @@ int fsx_batch_new(struct futhark_context *ctx, const struct fsx_map *const *maps
         }
         const int32_t hs = m->t->rows > m->t->cols ? m->t->rows : m->t->cols;
         const int32_t cs = m->s->rows > m->s->cols ? m->s->rows : m->s->cols;
-        hv[i].f.tame = fsk_frame_tame(&hv[i].f, hs > cs ? hs : cs);
+        hv[i].f.tame = fsk_tame_level(&hv[i].f, hs > cs ? hs : cs);
         fsk_map_recips(&hv[i].m);
         hv[i].offset = offsets[i];
         hv[i].ntiles = (views[i].w + tc - 1) / tc;

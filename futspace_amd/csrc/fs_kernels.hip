@@ -3167,7 +3167,7 @@ int fsk_render_slices_clear(const fsk_map *m, const fsk_frame *f, const fsk_tuni
     a.m = *m;
     fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f, map_side(m));
+    a.f.tame = fsk_tame_level(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = (uint32_t *)d_src;
@@ -3214,7 +3214,7 @@ static DiffArgs diff_args(const fsk_frame *f, const float *cp, const float *sf, 
 {
     DiffArgs a;
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f, std::max(hc, wc));
+    a.f.tame = fsk_tame_level(f, std::max(hc, wc));
     a.rhc = fsk_wrap_recip(hc);
     a.rwc = fsk_wrap_recip(wc);
     a.cp = cp;
@@ -3243,7 +3243,7 @@ int fsk_render_nearest(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t
     a.m = *m;
     fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f, map_side(m));
+    a.f.tame = fsk_tame_level(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = d_out;
@@ -3442,16 +3442,18 @@ void fsk_map_recips(fsk_map *m)
     m->rccols = m->ccols > 0 ? fsk_wrap_recip(m->ccols) : 0.0f;
 }
 
-int32_t fsk_frame_tame(const fsk_frame *f, int32_t max_side)
+/* The frame's largest sample coordinate where its scalars and rows are
+ * tame, else infinity. */
+static double tame_extent(const fsk_frame *f)
 {
     const float v[] = {f->cam_x, f->cam_y, f->cam_h, f->horizon, f->Lx, f->Ly,
                        f->Rx,    f->Ry,    f->d,     f->z0,      f->scale, f->fw};
     for (float x : v)
         if (!std::isfinite(x))
-            return 0;
+            return INFINITY;
     if (!(f->z0 > 0.0f) || !(f->d >= 0.0f) || !(f->scale > 0.0f) || !(f->fw >= 1.0f) ||
         f->n <= 0)
-        return 0;
+        return INFINITY;
     /* z_k = (k/2)(2 z0 + (k-1) d) is non-decreasing from z_1 = z0 (every
      * f32 step of get_zs' term is monotone for z0 > 0, d >= 0), so
      * inv_z <= scale / z0; a 1e-3 margin covers the roundings */
@@ -3470,9 +3472,19 @@ int32_t fsk_frame_tame(const fsk_frame *f, int32_t max_side)
     /* slice depths inside [2^-100, 2^100], where the table's reciprocal
      * (rcp_rn) is exact */
     const bool zok = (double)f->z0 >= 0x1p-100 && zmax <= 0x1p100;
-    if (!(zok && xmax < 4194304.0 && ymax < 4194304.0 && relmax < 1073741824.0))
-        return 0;
-    return xmax < 2097152.0 && ymax < 2097152.0 && max_side <= 1 << 20 ? FSK_TAME_MOD : FSK_TAME;
+    return zok && relmax < 1073741824.0 ? std::max(xmax, ymax) : INFINITY;
+}
+
+int32_t fsk_frame_tame(const fsk_frame *f)
+{
+    return tame_extent(f) < 4194304.0 ? FSK_TAME : 0;
+}
+
+int32_t fsk_tame_level(const fsk_frame *f, int32_t max_side)
+{
+    const double extent = tame_extent(f);
+    return extent < 2097152.0 && max_side <= 1 << 20 ? FSK_TAME_MOD
+           : extent < 4194304.0 ? FSK_TAME : 0;
 }
 
 int32_t fsk_render_max_rows(void)
@@ -3510,7 +3522,7 @@ int fsk_render(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t, uint32
     a.m = *m;
     fsk_map_recips(&a.m);
     a.f = *f;
-    a.f.tame = fsk_frame_tame(f, map_side(m));
+    a.f.tame = fsk_tame_level(f, map_side(m));
     if (a.f.n < 0)
         a.f.n = 0;
     a.out = d_out;

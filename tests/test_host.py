@@ -231,3 +231,31 @@ def test_tame_bound_holds_by_brute_force():
             mx, my, mr = _extremes(f)
             assert mx < 2.0 ** 22 and my < 2.0 ** 22 and mr < 2.0 ** 30, (v, mx, my, mr)
     assert accepted >= 10
+
+
+def test_tame_level_bound_holds_by_brute_force():
+    """Random frames near the line of the reciprocal floor-mod: the level is
+    0 exactly where the frame is not tame, and 2 only where every coordinate
+    is below 2^21 and no side above 2^20."""
+    lib = ctypes.CDLL(os.path.join(ROOT, "futspace_amd", "libfutspace.so"))
+    level = lib.fsk_tame_level
+    level.restype = ctypes.c_int32
+    tame = _tame_fn()
+    rng = np.random.default_rng(33)
+    seen = set()
+    for _ in range(120):
+        v = View(x=float(rng.choice([1.0, -1.0]) * rng.uniform(1.5e6, 2.3e6)),
+                 y=float(rng.uniform(-2.2e6, 2.2e6)), height=100.0,
+                 angle=float(rng.uniform(0, 6.3)), horizon=20.0, distance=1000.0,
+                 fov=float(rng.uniform(0.5, 1.5)), h=64, w=int(rng.integers(1, 64)),
+                 d=float(rng.uniform(0.0, 0.05)), z0=float(10 ** rng.uniform(-3, 1)),
+                 scale=50.0, n_slices=int(rng.integers(1, 300)))
+        f = _frame(v)
+        got = level(ctypes.byref(f), 1 << 20)
+        seen.add(got)
+        assert (got > 0) == (tame(ctypes.byref(f)) != 0)
+        if got == 2:
+            mx, my, _ = _extremes(f)
+            assert mx < 2.0 ** 21 and my < 2.0 ** 21, (v, mx, my)
+            assert level(ctypes.byref(f), (1 << 20) + 1) == 1
+    assert {1, 2} <= seen
