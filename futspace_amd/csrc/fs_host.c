@@ -1702,9 +1702,10 @@ int fsx_render_f32_vjp(struct futhark_context *ctx, const struct fsx_view *view,
     return 0;
 }
 
-/* The fused step behind both entries; `noalloc` takes the partial sums
+/* The fused step behind its entries; `noalloc` takes the partial sums
  * from the device's fixed scratch array instead of the context's buffer
- * (which the first use allocates). */
+ * (which the first use allocates).  Without a map dev_src is not rendered
+ * but read. */
 static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
                    const struct fsx_map *map, const struct fsx_view *view,
                    const float *dev_planes, const float *dev_sf, int32_t hc, int32_t wc,
@@ -1712,7 +1713,7 @@ static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
                    int32_t *dev_src, float *dev_gimg, float *dev_gplanes, float *dev_gsky,
                    float *dev_loss)
 {
-    REQUIRE_ARGS(ctx, map && view, what);
+    REQUIRE_ARGS(ctx, view, what);
     fsk_frame f;
     if (diff_frame(ctx, what, view, hc, wc, &f))
         return 1;
@@ -1752,21 +1753,23 @@ static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
     }
     if (!noalloc && partials(ctx, &part))
         return 1;
-    fsk_map m;
-    m.hq = map->t->d_hq;
-    m.hrows = map->t->rows;
-    m.hcols = map->t->cols;
-    m.hbits = map->t->hbits;
-    m.cq = NULL;
-    m.crows = hc;
-    m.ccols = wc;
     /* unless accumulating, the gradient planes are cleared by the slice
      * render's spare workgroups (CUs its tiles leave idle) or else by a
      * launch of their own */
     int32_t cleared = 0;
-    HIPCHECK(ctx, fsk_render_slices_clear(&m, &f, &ctx->tune, dev_src, view->w,
-                                          accumulate ? NULL : dev_gplanes, nplanes, &cleared,
-                                          ctx->stream));
+    if (map) {
+        fsk_map m;
+        m.hq = map->t->d_hq;
+        m.hrows = map->t->rows;
+        m.hcols = map->t->cols;
+        m.hbits = map->t->hbits;
+        m.cq = NULL;
+        m.crows = hc;
+        m.ccols = wc;
+        HIPCHECK(ctx, fsk_render_slices_clear(&m, &f, &ctx->tune, dev_src, view->w,
+                                              accumulate ? NULL : dev_gplanes, nplanes, &cleared,
+                                              ctx->stream));
+    }
     if (!accumulate && !cleared)
         HIPCHECK(ctx, fsk_zero_f32(dev_gplanes, nplanes, ctx->stream));
     /* colour, loss terms and adjoint in one launch; the loss and sky
@@ -1786,6 +1789,7 @@ int fsx_render_f32_l2_step(struct futhark_context *ctx, const struct fsx_map *ma
                            int32_t *dev_src, float *dev_gimg, float *dev_gplanes,
                            float *dev_gsky, float *dev_loss)
 {
+    REQUIRE_ARGS(ctx, map && view, "fsx_render_f32_l2_step");
     return l2_step(ctx, "fsx_render_f32_l2_step", 0, map, view, dev_planes, dev_sf, hc, wc,
                    sky_scale, dev_target, accumulate, dev_img, dev_src, dev_gimg, dev_gplanes,
                    dev_gsky, dev_loss);
@@ -1798,8 +1802,21 @@ int fsx_render_f32_l2_step_noalloc(struct futhark_context *ctx, const struct fsx
                                    int32_t *dev_src, float *dev_gimg, float *dev_gplanes,
                                    float *dev_gsky, float *dev_loss)
 {
+    REQUIRE_ARGS(ctx, map && view, "fsx_render_f32_l2_step_noalloc");
     return l2_step(ctx, "fsx_render_f32_l2_step_noalloc", 1, map, view, dev_planes, dev_sf, hc,
                    wc, sky_scale, dev_target, accumulate, dev_img, dev_src, dev_gimg,
+                   dev_gplanes, dev_gsky, dev_loss);
+}
+
+int fsx_f32_l2_step_visible(struct futhark_context *ctx, const struct fsx_view *view,
+                            const float *dev_planes, const float *dev_sf, int32_t hc,
+                            int32_t wc, float sky_scale, const float *dev_target,
+                            int32_t accumulate, float *dev_img, const int32_t *dev_src,
+                            float *dev_gimg, float *dev_gplanes, float *dev_gsky,
+                            float *dev_loss)
+{
+    return l2_step(ctx, "fsx_f32_l2_step_visible", 0, NULL, view, dev_planes, dev_sf, hc, wc,
+                   sky_scale, dev_target, accumulate, dev_img, (int32_t *)dev_src, dev_gimg,
                    dev_gplanes, dev_gsky, dev_loss);
 }
 

@@ -16,6 +16,7 @@ and torch's current stream waits for it afterwards.
 """
 import contextlib
 import ctypes
+import dataclasses
 
 import numpy as np
 import torch
@@ -131,13 +132,16 @@ class DiffRenderer:
         return grad, loss
 
     def l2_step(self, planes, sky_scale, view: View, target, img=None, src=None, gimg=None,
-                gplanes=None, gsky=None, loss=None, accumulate=False, outputs=True):
+                gplanes=None, gsky=None, loss=None, accumulate=False, outputs=True,
+                visible=False):
         """One fitting step in one call: forward_raw, l2_loss_grad against
         target and vjp_raw with that gradient (fsx_render_f32_l2_step).
         Returns (img, src, gplanes, gsky, loss); with accumulate the loss and
         the gradients are added into the given tensors.  With outputs=False
         the image and its loss gradient are neither allocated nor written
-        (img and gimg are ignored and None is returned for img)."""
+        (img and gimg are ignored and None is returned for img).  With
+        visible=True src is not rendered but read: it holds what an earlier
+        call wrote for the same view (fsx_f32_l2_step_visible)."""
         self._check_planes(planes)
         if tuple(target.shape) != (3, view.h, view.w) or not target.is_contiguous():
             raise ValueError("target must be a contiguous [3][h][w] tensor")
@@ -145,6 +149,8 @@ class DiffRenderer:
             img = gimg = None
         elif img is None:
             img = torch.empty((3, view.h, view.w), dtype=torch.float32, device="cuda")
+        if visible and (src is None or tuple(src.shape) != (view.h, view.w)):
+            raise ValueError("visible=True needs the view's src")
         if src is None:
             src = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
         if outputs and gimg is None:
@@ -158,6 +164,14 @@ class DiffRenderer:
         if loss is None:
             loss = torch.empty(1, dtype=torch.float32, device="cuda")
         cv = view.to_c()
+        if visible:
+            with self.stream():
+                self.ctx.check(self.ctx.lib.fsx_f32_l2_step_visible(
+                    self.ctx.ptr, ctypes.byref(cv), _ptr(planes), _ptr(self.sf), self.hc,
+                    self.wc, ctypes.c_float(sky_scale), _ptr(target), 1 if accumulate else 0,
+                    _ptr_or_null(img), _ptr(src), _ptr_or_null(gimg), _ptr(gplanes), _ptr(gsky),
+                    _ptr(loss)), "fsx_f32_l2_step_visible")
+            return img, src, gplanes, gsky, loss
         with self.stream():
             self.ctx.check(self.ctx.lib.fsx_render_f32_l2_step(
                 self.ctx.ptr, self.map.ptr, ctypes.byref(cv), _ptr(planes), _ptr(self.sf),
@@ -219,6 +233,7 @@ def planes_of(color):
 
 
 COLOUR_UNIT = 255.0   # a colour-map channel step (u8) in plane units
+FIT_VISIBLE_SHARE = 0.125   # of the device's memory, for the views' visible slices in fit()
 
 
 def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None):
@@ -231,6 +246,10 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     channel / 255), so Adam moves each plane value by about lr / 255 per
     step; each step is one pass of the library's Adam kernel, which also
     clamps the planes back to [0, 1], the domain of the relaxation.
+    Visibility does not depend on the planes: each view's visible slices are
+    rendered in the first step and kept for the later ones, as far as they
+    take no more than FIT_VISIBLE_SHARE of the device's memory (an entry of
+    views that on_step changes is rendered anew).
     Returns the per-step losses (a CUDA tensor, read once at the end)."""
     planes.requires_grad_(False)
     step_lr = lr / COLOUR_UNIT
@@ -238,18 +257,34 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     m = torch.zeros_like(planes)
     v = torch.zeros_like(planes)
     gsky = torch.zeros(1, dtype=torch.float32, device="cuda")
-    src = None
+    held = {}                 # view number -> (view, map, its visible slices)
+    room = int(torch.cuda.get_device_properties(planes.device).total_memory * FIT_VISIBLE_SHARE)
+    shared = None             # the visible slices of a view that found no room
     losses = torch.zeros(steps, dtype=torch.float32, device="cuda")
     for it in range(steps):
         # one ordering of the renderer's stream against torch's per step:
         # the views' calls and the optimizer step queue back to back
         with renderer.stream():
             for i, (view, t) in enumerate(zip(views, targets)):
-                if src is None or tuple(src.shape) != (view.h, view.w):
+                have = held.get(i)
+                known = have is not None and have[0] == view and have[1] is renderer.map
+                if known:
+                    src = have[2]
+                elif have is not None and tuple(have[2].shape) == (view.h, view.w):
+                    src = have[2]
+                    held[i] = (dataclasses.replace(view), renderer.map, src)
+                elif have is None and 4 * view.h * view.w <= room:
                     src = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
+                    held[i] = (dataclasses.replace(view), renderer.map, src)
+                    room -= 4 * view.h * view.w
+                else:
+                    if shared is None or tuple(shared.shape) != (view.h, view.w):
+                        shared = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
+                    src = shared
                 # the loop needs neither the image nor its loss gradient
                 renderer.l2_step(planes, sky_scale, view, t, None, src, None, grad, gsky,
-                                 losses[it:it + 1], accumulate=i > 0, outputs=False)
+                                 losses[it:it + 1], accumulate=i > 0, outputs=False,
+                                 visible=known)
             renderer.adam_step(planes, grad, m, v, step_lr, it + 1)
         if on_step is not None:
             on_step(it)

@@ -305,6 +305,19 @@ int fsx_render_f32_l2_step_noalloc(struct futhark_context *ctx, const struct fsx
                                    int32_t *dev_src, float *dev_gimg, float *dev_gplanes,
                                    float *dev_gsky, float *dev_loss);
 
+/* fsx_render_f32_l2_step without its visibility render: dev_src is read, and
+ * holds the visible slices that an earlier step or fsx_render_f32 wrote for
+ * the same view over the same map (visibility depends on nothing else, so a
+ * fitting loop renders it once per view).  The gradient planes are cleared
+ * by a launch of their own unless accumulating; results and frame limit are
+ * the step's.  Asynchronous on the context stream. */
+int fsx_f32_l2_step_visible(struct futhark_context *ctx, const struct fsx_view *view,
+                            const float *dev_planes, const float *dev_sf, int32_t hc,
+                            int32_t wc, float sky_scale, const float *dev_target,
+                            int32_t accumulate, float *dev_img, const int32_t *dev_src,
+                            float *dev_gimg, float *dev_gplanes, float *dev_gsky,
+                            float *dev_loss);
+
 /* Render kernel shape, as chosen by the autotuner: columns per workgroup
  * tile (4 or 8), workgroups per CU (1 of 1024 threads, or 2 of 512 whose
  * depth chunks are shortened until two tiles fit in LDS) and depth slices

@@ -527,3 +527,71 @@ def test_adjoint_table_and_blocks(ctx, h, w, size, zoom):
         assert abs(float(sky[0]) - float(want_sky)) <= 1e-5 * mass
     want_loss = float(((want_img.astype(np.float64) - target.cpu().numpy()) ** 2).sum())
     assert abs(float(loss[0]) - want_loss) <= 1e-5 * want_loss
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_step_with_given_visibility(ctx, accumulate):
+    """l2_step(visible=True) over the src of a forward call: the loss bit for
+    bit and the gradients of the step that renders it, src left alone."""
+    r, col, _, _ = _setup(ctx)
+    tp = torch.from_numpy(planes_of(col)).cuda()
+    for v in VIEWS:
+        rng = np.random.default_rng(v.h)
+        target = torch.from_numpy(rng.random((3, v.h, v.w), dtype=np.float32)).cuda()
+        outs = []
+        for visible in (False, True):
+            src = r.forward_raw(tp, 0.3, v)[1]
+            before = src.clone()
+            gp, gs, loss = torch.full_like(tp, 2.0), torch.full((1,), 3.0, device="cuda"), \
+                torch.full((1,), 4.0, device="cuda")
+            torch.cuda.synchronize()
+            img, _, gp, gs, loss = r.l2_step(tp, 0.3, v, target, src=src, gplanes=gp, gsky=gs,
+                                             loss=loss, accumulate=accumulate, visible=visible)
+            torch.cuda.synchronize()
+            assert torch.equal(src, before)
+            outs.append((img, gp, gs, loss))
+        (img, gp, gs, loss), (img2, gp2, gs2, loss2) = outs
+        assert torch.equal(img, img2) and torch.equal(loss, loss2) and torch.equal(gs, gs2)
+        assert _rel_err(gp2.cpu().numpy(), gp.cpu().numpy()) <= 1e-5
+    with pytest.raises(ValueError):
+        r.l2_step(tp, 0.3, VIEWS[0], target, visible=True)
+
+
+@pytest.mark.parametrize("share", [0.125, 0.0])
+def test_fit_follows_changed_views(ctx, share, monkeypatch):
+    """fit() renders a view's visibility again when its camera or size
+    changes between steps, and where no visibility is kept."""
+    import dataclasses
+
+    from futspace_amd import diff
+    monkeypatch.setattr(diff, "FIT_VISIBLE_SHARE", share)
+    r, col, _, _ = _setup(ctx)
+    start = torch.from_numpy(planes_of(col)).cuda()
+    views = [dataclasses.replace(VIEWS[0]), dataclasses.replace(VIEWS[1])]
+    moved = dataclasses.replace(VIEWS[0], x=VIEWS[0].x + 7.3, angle=1.9)
+    other = dataclasses.replace(VIEWS[1], h=VIEWS[1].h + 3)
+    goal = (start * 0.5).contiguous()
+    targets = [r.forward_raw(goal, 0.3, v)[0] for v in views]
+    torch.cuda.synchronize()
+
+    def swap(it):
+        if it == 1:
+            views[0].x, views[0].angle = moved.x, moved.angle
+            views[1] = other
+            for i, v in enumerate(views):
+                targets[i] = r.forward_raw(goal, 0.3, v)[0]
+
+    planes = start.clone()
+    losses = fit(r, planes, views, targets, 0.3, steps=4, on_step=swap).cpu().numpy()
+    # the same steps one by one through l2_step, which always renders
+    p, g, m, s = start.clone(), torch.zeros_like(start), torch.zeros_like(start), \
+        torch.zeros_like(start)
+    for it in range(4):
+        vs = [VIEWS[0], VIEWS[1]] if it < 2 else [moved, other]
+        gs, loss = torch.zeros(1, device="cuda"), torch.zeros(1, device="cuda")
+        for i, v in enumerate(vs):
+            t = r.forward_raw(goal, 0.3, v)[0]
+            r.l2_step(p, 0.3, v, t, gplanes=g, gsky=gs, loss=loss, accumulate=i > 0)
+        r.adam_step(p, g, m, s, 0.5 / 255.0, it + 1)
+        torch.cuda.synchronize()
+        assert abs(float(loss[0]) - losses[it]) <= 1e-5 * abs(float(loss[0]))
