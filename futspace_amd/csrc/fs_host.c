@@ -38,6 +38,10 @@ struct fs_terrain;
 struct fs_shade;
 
 #define FS_POOL_SLOTS 16
+/* Bytes of freed map buffers that a context keeps: the maps of a few loads
+ * or re-shadings (a 2048^2 map and its shade take 63 MB).  Given back when
+ * the context or its caches are freed, or an allocation fails. */
+#define FS_POOL_MAP_BYTES ((size_t)256 << 20)
 
 struct futhark_context {
     int device;
@@ -48,7 +52,10 @@ struct futhark_context {
     struct {
         void *ptr;
         size_t bytes;
-    } pool[FS_POOL_SLOTS];    /* freed output buffers kept for reuse */
+        uint64_t age;         /* pool_clock when it was freed */
+        int map;              /* a map buffer, counted against FS_POOL_MAP_BYTES */
+    } pool[FS_POOL_SLOTS];    /* freed buffers kept for reuse */
+    uint64_t pool_clock;
     struct fs_terrain *empty_terrain;
     struct fs_shade *empty_shade;
     fsk_tuning tune;          /* render kernel shape (0 = automatic) */
@@ -148,23 +155,69 @@ static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
     return 0;
 }
 
-/* Return a buffer to the reuse pool (stream order keeps reuse safe: every
- * later writer runs after every earlier reader on the one stream). */
+/* Free the buffer that has been in the pool longest (of map buffers, if
+ * map_only). */
+static void pool_evict(struct futhark_context *ctx, int map_only)
+{
+    int old = -1;
+    for (int i = 0; i < FS_POOL_SLOTS; i++)
+        if (ctx->pool[i].ptr && (!map_only || ctx->pool[i].map) &&
+            (old < 0 || ctx->pool[i].age < ctx->pool[old].age))
+            old = i;
+    if (old < 0)
+        return;
+    hipStreamSynchronize(ctx->stream);
+    hipFree(ctx->pool[old].ptr);
+    ctx->pool[old].ptr = NULL;
+}
+
+/* Return a buffer to the reuse pool, in place of the one longest there if
+ * it is full (stream order keeps reuse safe: every later writer runs after
+ * every earlier reader on the one stream). */
+static void pool_put(struct futhark_context *ctx, void *p, size_t bytes, int map)
+{
+    for (int pass = 0; pass < 2; pass++) {
+        for (int i = 0; i < FS_POOL_SLOTS; i++) {
+            if (!ctx->pool[i].ptr) {
+                ctx->pool[i].ptr = p;
+                ctx->pool[i].bytes = bytes;
+                ctx->pool[i].age = ctx->pool_clock++;
+                ctx->pool[i].map = map;
+                return;
+            }
+        }
+        pool_evict(ctx, 0);
+    }
+}
+
 static void dev_release(struct futhark_context *ctx, void *p, size_t bytes)
+{
+    if (p)
+        pool_put(ctx, p, bytes ? bytes : 4, 0);
+}
+
+/* dev_release of a map buffer: at most FS_POOL_MAP_BYTES of them are kept. */
+static void map_release(struct futhark_context *ctx, void *p, size_t bytes)
 {
     if (!p)
         return;
     if (bytes == 0)
         bytes = 4;
-    for (int i = 0; i < FS_POOL_SLOTS; i++) {
-        if (!ctx->pool[i].ptr) {
-            ctx->pool[i].ptr = p;
-            ctx->pool[i].bytes = bytes;
-            return;
-        }
+    if (bytes > FS_POOL_MAP_BYTES) {
+        hipStreamSynchronize(ctx->stream);
+        hipFree(p);
+        return;
     }
-    hipStreamSynchronize(ctx->stream);
-    hipFree(p);
+    for (;;) {
+        size_t kept = 0;
+        for (int i = 0; i < FS_POOL_SLOTS; i++)
+            if (ctx->pool[i].ptr && ctx->pool[i].map)
+                kept += ctx->pool[i].bytes;
+        if (kept + bytes <= FS_POOL_MAP_BYTES)
+            break;
+        pool_evict(ctx, 1);
+    }
+    pool_put(ctx, p, bytes, 1);
 }
 
 struct futhark_context_config *futhark_context_config_new(void)
@@ -622,7 +675,7 @@ struct fs_terrain {
     uint16_t *d_hp;        /* masked heights, one per texel */
     uint32_t *d_hmax;      /* the largest of them, in parts (in d_hp's allocation) */
     uint32_t *d_color;     /* raw colour map */
-    int32_t *h_alt;        /* host copy of the masked heights */
+    uint16_t *h_alt;       /* host copy of d_hp (states' terrains, for the collision) */
 };
 
 struct fs_shade {
@@ -639,14 +692,29 @@ struct fsx_map {
     int32_t shade_size;
 };
 
+static size_t terrain_texels(const struct fs_terrain *t)
+{
+    return (size_t)t->rows * (size_t)t->cols;
+}
+
+/* d_hp, padded to 16 bytes, with d_hmax behind it. */
+static size_t terrain_hp_bytes(const struct fs_terrain *t)
+{
+    return (terrain_texels(t) * 2 + 15) & ~(size_t)15;
+}
+
+static size_t terrain_hq_bytes(const struct fs_terrain *t)
+{
+    return terrain_texels(t) * (t->hbits == 8 ? 4 : 8);
+}
+
 static void terrain_unref(struct futhark_context *ctx, struct fs_terrain *t)
 {
     if (!t || --t->refs > 0)
         return;
-    hipStreamSynchronize(ctx->stream);
-    hipFree(t->d_hq);
-    hipFree(t->d_hp);
-    hipFree(t->d_color);
+    map_release(ctx, t->d_hq, terrain_hq_bytes(t));
+    map_release(ctx, t->d_hp, terrain_hp_bytes(t) + FSK_HMAX_PARTS * 4);
+    map_release(ctx, t->d_color, terrain_texels(t) * 4);
     free(t->h_alt);
     free(t);
 }
@@ -655,17 +723,19 @@ static void shade_unref(struct futhark_context *ctx, struct fs_shade *s)
 {
     if (!s || --s->refs > 0)
         return;
-    hipStreamSynchronize(ctx->stream);
-    hipFree(s->d_shaded);
-    hipFree(s->d_cq);
+    const size_t n = (size_t)s->rows * (size_t)s->cols;
+    map_release(ctx, s->d_shaded, n * 4);
+    map_release(ctx, s->d_cq, n * 16);
     free(s);
 }
 
-/* Build a terrain from device colours and device i32 heights (both
- * [rows][cols]); heights are masked to hbits. */
-static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_t *d_color_src,
-                                      const int32_t *d_alt, int32_t rows, int32_t cols,
-                                      int32_t hbits)
+/* Build a terrain from colours (in device or host memory, as `kind` says)
+ * and device i32 heights, both [rows][cols]; heights are masked to hbits.
+ * The caller waits for the stream before the sources go.  With host_heights
+ * the masked heights are copied back as well, and waited for. */
+static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_t *color,
+                                      hipMemcpyKind kind, const int32_t *d_alt, int32_t rows,
+                                      int32_t cols, int32_t hbits, int host_heights)
 {
     if ((int64_t)rows * (int64_t)cols > ((int64_t)1 << 28)) {
         set_error(ctx, "map of %d x %d texels exceeds the supported 2^28", rows, cols);
@@ -678,37 +748,34 @@ static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_
     t->rows = rows;
     t->cols = cols;
     t->hbits = hbits;
-    size_t n = (size_t)rows * (size_t)cols;
-    size_t qbytes = n * (hbits == 8 ? 4 : 8);
-    hipError_t e = hipMalloc(&t->d_hq, qbytes ? qbytes : 4);
-    const size_t hpbytes = (n * 2 + 15) & ~(size_t)15;
-    if (e == hipSuccess) e = hipMalloc((void **)&t->d_hp, hpbytes + FSK_HMAX_PARTS * 4);
-    t->d_hmax = (uint32_t *)((char *)t->d_hp + hpbytes);
-    if (e == hipSuccess) e = hipMalloc((void **)&t->d_color, n ? n * 4 : 4);
-    t->h_alt = (int32_t *)malloc(n ? n * 4 : 4);
-    if (e != hipSuccess || !t->h_alt) {
-        set_error(ctx, "terrain allocation (%d x %d) failed: %s", rows, cols, hipGetErrorString(e));
-        hipFree(t->d_hq); hipFree(t->d_hp); hipFree(t->d_color); free(t->h_alt); free(t);
+    const size_t n = terrain_texels(t), hpbytes = terrain_hp_bytes(t);
+    int failed = dev_alloc(ctx, &t->d_hq, terrain_hq_bytes(t)) ||
+                 dev_alloc(ctx, (void **)&t->d_hp, hpbytes + FSK_HMAX_PARTS * 4) ||
+                 dev_alloc(ctx, (void **)&t->d_color, n * 4);
+    if (!failed && host_heights) {
+        t->h_alt = (uint16_t *)malloc(n ? n * 2 : 2);
+        failed = !t->h_alt;
+    }
+    if (failed) {
+        set_error(ctx, "terrain allocation (%d x %d) failed", rows, cols);
+        terrain_unref(ctx, t);
         return NULL;
     }
+    t->d_hmax = (uint32_t *)((char *)t->d_hp + hpbytes);
     if (n) {
-        e = hipMemcpyAsync(t->d_color, d_color_src, n * 4, hipMemcpyDeviceToDevice, ctx->stream);
+        hipError_t e = hipMemcpyAsync(t->d_color, color, n * 4, kind, ctx->stream);
         if (e == hipSuccess)
             e = (hipError_t)fsk_height_quads(d_alt, rows, cols, hbits, t->d_hq, t->d_hp,
                                              t->d_hmax, ctx->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(t->h_alt, d_alt, n * 4, hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess)
+        if (e == hipSuccess && host_heights)
+            e = hipMemcpyAsync(t->h_alt, t->d_hp, n * 2, hipMemcpyDeviceToHost, ctx->stream);
+        if (e == hipSuccess && host_heights)
             e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) {
             set_error(ctx, "terrain upload failed: %s", hipGetErrorString(e));
-            t->refs = 1;
             terrain_unref(ctx, t);
             return NULL;
         }
-        uint32_t mk = hbits == 8 ? 0xFFu : 0xFFFFu;
-        for (size_t i = 0; i < n; i++)
-            t->h_alt[i] = (int32_t)((uint32_t)t->h_alt[i] & mk);
     }
     return t;
 }
@@ -741,16 +808,13 @@ static struct fs_shade *shade_new(struct futhark_context *ctx, const struct fs_t
     s->rows = size;
     s->cols = size;
     size_t n = (size_t)size * (size_t)size;
-    hipError_t e = hipMalloc((void **)&s->d_shaded, n * 4);
-    if (e == hipSuccess)
-        e = hipMalloc(&s->d_cq, n * 16);
-    if (e != hipSuccess) {
-        set_error(ctx, "shade allocation (%d^2) failed: %s", size, hipGetErrorString(e));
-        hipFree(s->d_shaded); hipFree(s->d_cq); free(s);
+    if (dev_alloc(ctx, (void **)&s->d_shaded, n * 4) || dev_alloc(ctx, &s->d_cq, n * 16)) {
+        set_error(ctx, "shade allocation (%d^2) failed", size);
+        shade_unref(ctx, s);
         return NULL;
     }
     sun_vector(sun_height, sun_ang, s->sun);
-    e = (hipError_t)fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, t->d_color, s->sun, size,
+    hipError_t e = (hipError_t)fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, t->d_color, s->sun, size,
                               s->d_shaded, ctx->stream);
     if (e == hipSuccess)
         e = (hipError_t)fsk_color_quads(s->d_shaded, size, size, s->d_cq, ctx->stream);
@@ -774,7 +838,7 @@ static struct fs_terrain *terrain_zero(struct futhark_context *ctx)
         hipFree(d_alt); hipFree(d_col);
         return NULL;
     }
-    struct fs_terrain *t = terrain_new(ctx, d_col, d_alt, 2, 1, 8);
+    struct fs_terrain *t = terrain_new(ctx, d_col, hipMemcpyDeviceToDevice, d_alt, 2, 1, 8, 1);
     hipStreamSynchronize(ctx->stream);
     hipFree(d_alt);
     hipFree(d_col);
@@ -789,11 +853,11 @@ static struct fs_shade *shade_zero(struct futhark_context *ctx)
     s->refs = 1;
     s->rows = 2;
     s->cols = 1;
-    if (hipMalloc((void **)&s->d_shaded, 8) != hipSuccess || hipMalloc(&s->d_cq, 32) != hipSuccess ||
+    if (dev_alloc(ctx, (void **)&s->d_shaded, 8) || dev_alloc(ctx, &s->d_cq, 32) ||
         hipMemsetAsync(s->d_shaded, 0, 8, ctx->stream) != hipSuccess ||
         hipMemsetAsync(s->d_cq, 0, 32, ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
-        hipFree(s->d_shaded); hipFree(s->d_cq); free(s);
+        shade_unref(ctx, s);
         return NULL;
     }
     return s;
@@ -1245,8 +1309,8 @@ int futhark_entry_update_map(struct futhark_context *ctx, struct futhark_opaque_
     }
     if (hipSetDevice(ctx->device) != hipSuccess)
         return 1;
-    struct fs_terrain *t = terrain_new(ctx, in0->d, in1->d, (int32_t)in0->shape[0],
-                                       (int32_t)in0->shape[1], 8);
+    struct fs_terrain *t = terrain_new(ctx, in0->d, hipMemcpyDeviceToDevice, in1->d,
+                                       (int32_t)in0->shape[0], (int32_t)in0->shape[1], 8, 1);
     if (!t)
         return 1;
     struct fs_shade *s = shade_new(ctx, t, 1024, in2->sun_height, in2->sun_ang);
@@ -1372,18 +1436,23 @@ int fsx_map_new(struct futhark_context *ctx, struct fsx_map **out,
         set_error(ctx, "fsx_map_new: invalid shade size %d", shade_size);
         return 1;
     }
-    struct futhark_u32_2d *c = futhark_new_u32_2d(ctx, color, rows, cols);
-    struct futhark_i32_2d *h = futhark_new_i32_2d(ctx, height, rows, cols);
-    if (!c || !h) {
-        futhark_free_u32_2d(ctx, c);
-        futhark_free_i32_2d(ctx, h);
+    if (!dims_ok(ctx, rows, cols))
         return 1;
-    }
-    struct fsx_map *m = (struct fsx_map *)calloc(1, sizeof *m);
+    /* the colours go straight into the terrain; the heights pass through a
+     * buffer of their own, which the quads are made from */
+    const size_t bytes = (size_t)(rows * cols) * 4;
+    int32_t *d_alt = NULL;
+    if (hipSetDevice(ctx->device) != hipSuccess || dev_alloc(ctx, (void **)&d_alt, bytes))
+        return 1;
+    hipError_t e = hipMemcpyAsync(d_alt, height, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e != hipSuccess)
+        set_error(ctx, "fsx_map_new: %s", hipGetErrorString(e));
+    struct fsx_map *m = e == hipSuccess ? (struct fsx_map *)calloc(1, sizeof *m) : NULL;
     int rc = 1;
     if (m) {
         m->shade_size = shade_size == 0 ? 1024 : shade_size;
-        m->t = terrain_new(ctx, c->d, h->d, (int32_t)rows, (int32_t)cols, height_bits);
+        m->t = terrain_new(ctx, color, hipMemcpyHostToDevice, d_alt, (int32_t)rows,
+                           (int32_t)cols, height_bits, 0);
         if (m->t)
             m->s = shade_new(ctx, m->t, m->shade_size, sun_height, sun_ang);
         if (m->t && m->s) {
@@ -1394,9 +1463,15 @@ int fsx_map_new(struct futhark_context *ctx, struct fsx_map **out,
             m = NULL;
         }
     }
-    hipStreamSynchronize(ctx->stream);
-    futhark_free_u32_2d(ctx, c);
-    futhark_free_i32_2d(ctx, h);
+    /* the caller's arrays are read until here */
+    e = hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess && rc == 0) {
+        set_error(ctx, "fsx_map_new: %s", hipGetErrorString(e));
+        fsx_map_free(ctx, m);
+        m = NULL;
+        rc = 1;
+    }
+    map_release(ctx, d_alt, bytes);
     *out = m;
     return rc;
 }

@@ -134,3 +134,51 @@ def test_depth_slice_limit(ctx, small):
     ok = _view(8, 16)
     ok.n_slices = 1 << 12
     assert ctx.render(m, ok).shape == (8, 16)
+
+
+def test_map_buffers_are_reused_safely(ctx):
+    """Maps loaded and freed in turn, of equal and of many different sizes
+    (more than the context keeps), with renders and a batch in flight: every
+    frame is of the map it names, and a batch keeps a freed map's buffers."""
+    from futspace_amd import sky_color
+    from oracle import fs_oracle as O
+    v = View(x=20.3, y=30.7, height=300.0, angle=0.9, horizon=20.0, distance=300.0, fov=1.2,
+             sky_color=sky_color(0.1), h=40, w=56, d=0.004, z0=0.5, scale=50.0)
+    kept = ctx.map(*scene.scene_maps(60, 64), shade_size=64)
+    shaded0, alt0 = O.update_map(*scene.scene_maps(60, 64), size=64)
+    want0 = O.render_off(v, shaded0, alt0)
+    out = torch.zeros(v.h * v.w, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    batch = ctx.batch([kept], [v], out, [0])
+    kept.close()
+    frames = []
+    for i in range(24):
+        side = 64 if i % 3 else 32 << (i % 4)
+        col, hts = scene.scene_maps(61 + i, side)
+        m = ctx.map(col, hts, height_bits=16 if i % 5 == 0 else 8, shade_size=64 if i % 2 else 48)
+        frame = torch.zeros((v.h, v.w), dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.render(m, v, frame)
+        shaded, alt = O.update_map(col, hts, size=m.shade_size, bits=m.height_bits)
+        frames.append((frame, O.render_off(v, shaded, alt)))
+        batch.run()
+        m.close()                        # the render may still be running
+    ctx.sync()
+    for frame, want in frames:
+        assert np.array_equal(frame.cpu().numpy().view(np.uint32), want)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32).reshape(v.h, v.w), want0)
+    batch.close()
+
+
+def test_terrain_collision_of_negative_heights(ctx):
+    """update_map masks heights to a byte for the collision as for the
+    frames (the host copy comes from the masked map)."""
+    col, hts = scene.scene_maps(62, 64)
+    for value, ground in ((-1, 255.0), (256 + 77, 77.0), (200, 200.0)):
+        s = Session(ctx)
+        s.update_map(col, np.full((64, 64), value, np.int32))
+        s.key(True, "f")                     # down, until the ground holds
+        for _ in range(30):
+            s.step()
+        assert s.text_content()[3] == ground
+        s.close()
