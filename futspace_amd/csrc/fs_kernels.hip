@@ -2346,7 +2346,7 @@ __device__ __forceinline__ Bilin bilin_of(const DiffArgs &a, int32_t k, int32_t 
 {
     const fsk_frame &f = a.f;
     const int32_t hc = a.hc, wc = a.wc;
-    Slice sl = TAME || f.tame ? slice_params_tame(f, k) : slice_params(f, k);
+    Slice sl = TAME ? slice_params_tame(f, k) : slice_params(f, k);
     float fcol = (float)col;
     float x = sl.sx + (fcol * sl.dx);
     float y = sl.sy + (fcol * sl.dy);
@@ -2355,7 +2355,7 @@ __device__ __forceinline__ Bilin bilin_of(const DiffArgs &a, int32_t k, int32_t 
      * is the plain one */
     auto cvt = [](float v) { return TAME ? (int32_t)v : i32_f32_x86(v); };
     int32_t ify, icy, ifx, icx;
-    if (!P2 && f.tame >= FSK_TAME_MOD) {
+    if (TAME && !P2 && f.tame >= FSK_TAME_MOD) {
         ify = wrap_tame(fy, hc, a.rhc);
         icy = wrap_tame(cy, hc, a.rhc);
         ifx = wrap_tame(fx, wc, a.rwc);
@@ -2412,9 +2412,9 @@ __device__ __forceinline__ void sample_gather(const DiffArgs &a, const Bilin &b,
 /* The colour of a visible sample from its gathered quad, per channel (the
  * relaxed png_color_filtered); sv[ch][t] = cv[ch][t] * sf[t]. */
 __device__ __forceinline__ void sample_mix(const Bilin &b, const float cv[3][4],
-                                           const float sf[4], float sv[3][4], float px[3])
+                                           const float sf[4], float w[4], float sv[3][4],
+                                           float px[3])
 {
-    float w[4];
     norm_weights(b, w);
 #pragma unroll
     for (int ch = 0; ch < 3; ch++) {
@@ -2554,21 +2554,36 @@ __device__ __forceinline__ bool segment_sum_quad(const uint32_t key[4], float (&
     return !same_next;
 }
 
-/* Workgroups of the adjoint: 64 columns by 4 waves, with a table of 1024
- * texels each (28 KiB), so that five of them share a CU.  512 threads with
- * 2048 texels: two per CU, 1900 x 1000 98 against 89 us per fused step; 128
- * with 512: 94 us. */
+/* Workgroups of the adjoint: 64 columns by 4 waves.  512 threads with a
+ * table of 2048 texels: 1900 x 1000 98 against 89 us per fused step; 128 with
+ * 512: 94 us. */
 constexpr int kGradThreads = 256;
 /* Rows per thread in the adjoint: 2, or 4 in frames of kGradTallPixels
- * pixels or more.  A run of equal src down a thread's rows is merged in
- * registers, so more rows mean fewer texel inserts per pixel, which pays
- * where there are many workgroups per CU (3840 x 2160: 213 against 222 us
- * per fused step), while smaller frames need the waves (1280 x 720: 72
- * against 86 us). */
-constexpr int64_t kGradTallPixels = (int64_t)1 << 22;
-constexpr int kGradCapLog = 10;
-constexpr int kGradCap = 1 << kGradCapLog;   /* texel slots of a workgroup's LDS table */
-constexpr int kGradFill = kGradCap / 8 * 7;  /* slots taken before new texels go past it */
+ * pixels or more.  A run of equal src down a thread's rows is one evaluation
+ * and one insertion, so more rows mean fewer of both per pixel, which pays
+ * where a frame's runs are long and its workgroups many (2560 x 1440 over
+ * 2048 slices: 72 against 83 us, 3840 x 2160 over 4096 slices: 119 against
+ * 144 us), while smaller frames need the waves (1920 x 1080: 59 against 85
+ * us).  8 rows: 88 against 92 us where heights of 10 bits make long runs,
+ * 144 against 119 us where they do not. */
+constexpr int64_t kGradTallPixels = (int64_t)3 << 20;
+constexpr int kGradRowsLow = 2, kGradRowsTall = 4;
+/* Texel slots of a workgroup's table (28 bytes each), and the workgroups of
+ * a CU that they leave room for.  A texel that the table has no slot for
+ * costs scattered global atomics.  With 2 rows, 512 pixels, distant ground
+ * gives a workgroup up to some 1200 distinct texels: 1408 slots hold them
+ * (1280 x 720: 45 us with 1408 slots and four workgroups, 52 with 1024 and
+ * five, 59 with 816 and six).  With 4 rows, in frames whose runs are longer,
+ * 944 slots and six workgroups: 92 us, 1024 and five 100 us, 512 and six 91
+ * us there and 143 against 119 us over an 8-bit map. */
+constexpr int grad_cap(int rows)
+{
+    return rows == kGradRowsLow ? 1408 : 944;
+}
+constexpr int grad_waves(int rows)
+{
+    return rows == kGradRowsLow ? 4 : 6;
+}
 constexpr int kGradProbes = 4;
 constexpr int kGradRunLog = 4;               /* texels of a row that hash to adjacent slots */
 
@@ -2585,12 +2600,15 @@ constexpr int kGradRunLog = 4;               /* texels of a row that hash to adj
  * slots, which adjacent lanes flush, are then adjacent in memory, and a
  * wave's global atomics come as a few lines instead of one per lane
  * (1280 x 720: 94 -> 81 us per fused step; the flush no longer shows). */
+template <int kGradCap>
 __device__ __forceinline__ bool table_add(uint32_t *keys, double *vals, const uint32_t *fill,
                                           float *gcp, size_t plane, uint32_t key, const float v[3])
 {
     constexpr uint32_t kRun = 1u << kGradRunLog;
-    uint32_t h = (((key >> kGradRunLog) * 2654435761u) >> (32 - kGradCapLog + kGradRunLog)) * kRun +
-                 (key & (kRun - 1u));
+    static_assert(kGradCap % kRun == 0 && kGradCap / kRun <= 256, "whole runs, 32-bit product");
+    constexpr int kGradFill = kGradCap / 8 * 7;  /* slots taken before new texels go past it */
+    uint32_t h = (__umul24(((key >> kGradRunLog) * 2654435761u) >> 8, kGradCap / kRun) >> 24) *
+                     kRun + (key & (kRun - 1u));
     /* a relaxed atomic load, which becomes an LDS read: a volatile read
      * through this generic pointer was a flat load that waited for every
      * global atomic of the wave still in flight */
@@ -2607,12 +2625,12 @@ __device__ __forceinline__ bool table_add(uint32_t *keys, double *vals, const ui
         if (mine || k == key) {
 #pragma unroll
             for (int ch = 0; ch < 3; ch++)
-                if (v[ch] != 0.0f)
-                    __hip_atomic_fetch_add(&vals[ch * kGradCap + h], (double)v[ch],
-                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(&vals[ch * kGradCap + h], (double)v[ch],
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             return mine;
         }
-        h = (h + kRun) & (kGradCap - 1);
+        h += kRun;
+        h = h < (uint32_t)kGradCap ? h : h - kGradCap;
     }
 #pragma unroll
     for (int ch = 0; ch < 3; ch++)
@@ -2627,29 +2645,37 @@ __device__ __forceinline__ bool table_add(uint32_t *keys, double *vals, const ui
  * X1 = mix(wx0, s0, wx1, s1): d px / d s0 = wy0' * wx0' * s0 / px (X1
  * cancels), likewise for the other texels, 0 where px == 0. */
 struct SampleEval {
-    Bilin b;
+    uint32_t t[4];           /* the quad's texels */
+    float w[4];              /* norm_weights of the sample */
     float sf[4];             /* shade factors of the quad */
     float sv[3][4], px[3];   /* shaded texel values, pixel colour */
 };
 
-template <bool P2>
+template <bool P2, bool TAME>
 __device__ __forceinline__ void sample_eval(const DiffArgs &a, int32_t k, int32_t col,
                                             size_t plane, SampleEval &e)
 {
-    e.b = bilin_of<P2>(a, k, col);
+    /* the caller's src may name slices past the frame's last, which the tame
+     * bounds do not cover */
+    Bilin b;
+    if (TAME && !__ballot(k >= a.f.n))
+        b = bilin_of<P2, TAME>(a, k, col);
+    else
+        b = bilin_of<P2, false>(a, k, col);
     float cv[3][4];
-    sample_gather(a, e.b, plane, cv, e.sf);
-    sample_mix(e.b, cv, e.sf, e.sv, e.px);
+    sample_gather(a, b, plane, cv, e.sf);
+    sample_mix(b, cv, e.sf, e.w, e.sv, e.px);
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+        e.t[t] = b.t[t];
 }
 
 __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval &e,
                                             const float run[3], uint32_t key[4], float val[4][3])
 {
-    const Bilin &b = e.b;
     const float(&sv)[3][4] = e.sv;
     const float(&px)[3] = e.px;
-    float w[4];
-    norm_weights(b, w);
+    const float(&w)[4] = e.w;
     const float wt[4] = {w[2] * w[0], w[2] * w[1], w[3] * w[0], w[3] * w[1]};
     /* gradients are not bit-exact quantities: the hardware reciprocal
      * (within an ulp) stands in for the division, and the texel's weight
@@ -2661,21 +2687,11 @@ __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval 
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const float ws = wt[t] * e.sf[t];
-        key[t] = b.t[t];
+        key[t] = e.t[t];
 #pragma unroll
         for (int ch = 0; ch < 3; ch++)
             val[t][ch] = (q[ch] * ws) * sv[ch][t];
     }
-}
-
-template <bool P2>
-__device__ __forceinline__ void sample_terms(const DiffArgs &a, int32_t k, int32_t col,
-                                             size_t plane, const float run[3], uint32_t key[4],
-                                             float val[4][3])
-{
-    SampleEval e;
-    sample_eval<P2>(a, k, col, plane, e);
-    sample_grad(a, e, run, key, val);
 }
 
 /* Adjoint.  A workgroup covers 64 adjacent columns x 4 kGradRows rows; each
@@ -2703,9 +2719,11 @@ __device__ __forceinline__ void sample_terms(const DiffArgs &a, int32_t k, int32
  * workgroup leaves one partial of the loss, sum (px - target)^2, and one of
  * the sky term.  Otherwise each workgroup leaves one partial of the sky
  * term. */
-template <bool P2, bool FWD, int kGradRows>
-__global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
+template <bool P2, bool TAME, bool FWD, int kGradRows>
+__global__ __launch_bounds__(kGradThreads, grad_waves(kGradRows))
+void k_diff_grad(DiffArgs a)
 {
+    constexpr int kGradCap = grad_cap(kGradRows);
     constexpr int kGradBlockRows = (kGradThreads / 64) * kGradRows;
     __shared__ uint32_t keys[kGradCap];
     __shared__ double vals[3 * kGradCap];
@@ -2719,115 +2737,131 @@ __global__ __launch_bounds__(kGradThreads) void k_diff_grad(DiffArgs a)
     if (threadIdx.x == 0)
         fill = 0u;
     const int32_t col = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int32_t r0 = blockIdx.y * kGradBlockRows + (threadIdx.x >> 6) * kGradRows;
+    /* the row is the wave's: scalar, so that a pixel's address is a scalar
+     * row pointer and the column */
+    const int32_t wave = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x >> 6);
+    const int32_t r0 = blockIdx.y * kGradBlockRows + wave * kGradRows;
     const int32_t H = a.f.rows, W = a.f.cols;
-    const bool ok = col < W && r0 < H;
+    const uint32_t lcol = (uint32_t)min(col, W - 1);
     const size_t plane = (size_t)a.hc * a.wc, fplane = (size_t)H * W;
     /* global-space views of the per-pixel inputs (loads through the
      * generic pointers came out as flat loads) */
     const FS_GLOBAL float *gin = (const FS_GLOBAL float *)(FWD ? a.tgt : a.gimg);
     const FS_GLOBAL int32_t *srcp = (const FS_GLOBAL int32_t *)a.src;
     int32_t src[kGradRows];
-    float g[3][kGradRows];     /* FWD: the target until the pixel's g replaces it */
+    float g[3][kGradRows];     /* FWD: the target */
 #pragma unroll
     for (int j = 0; j < kGradRows; j++) {
-        const int32_t r = r0 + j;
-        const bool in = ok && r < H;
-        const size_t p = (size_t)r * W + col;
-        src[j] = in ? srcp[p] : INT32_MIN;
+        /* threads outside the frame load the pixel at its edge */
+        const size_t row = (size_t)min(r0 + j, H - 1) * W;
+        src[j] = (srcp + row)[lcol];
 #pragma unroll
         for (int ch = 0; ch < 3; ch++)
-            g[ch][j] = in ? gin[ch * fplane + p] : 0.0f;
+            g[ch][j] = (gin + ch * fplane + row)[lcol];
     }
+#pragma unroll
+    for (int j = 0; j < kGradRows; j++)
+        if (!(col < W && r0 + j < H))
+            src[j] = INT32_MIN;
     __syncthreads();
     /* the sky term cancels where gradients of both signs meet: f64 keeps its
      * sum as exact as the gradients */
     double sky_acc = 0.0;
     float loss_acc = 0.0f;
-    float run[3] = {0.0f, 0.0f, 0.0f};
-    SampleEval e;              /* FWD: the current run's sample */
+    /* one pixel of the fused step: its loss term and g = 2 (px - target) */
+    auto pixel = [&](int j, uint32_t c, const float px[3], float (&gd)[3]) {
+        const size_t row = (size_t)(r0 + j) * W;
+#pragma unroll
+        for (int ch = 0; ch < 3; ch++) {
+            const float d = px[ch] - g[ch][j];
+            gd[ch] = 2.0f * d;
+            if (a.img)
+                ((FS_GLOBAL float *)a.img + ch * fplane + row)[c] = px[ch];
+            if (a.gout)
+                ((FS_GLOBAL float *)a.gout + ch * fplane + row)[c] = gd[ch];
+            loss_acc += d * d;
+        }
+    };
+    uint32_t starts = 0u;      /* rows where a run of a visible sample starts */
 #pragma unroll
     for (int j = 0; j < kGradRows; j++) {
         const int32_t k = src[j];
-        if constexpr (FWD) {
-            const bool starts = k != INT32_MIN && (j == 0 || src[j - 1] != k);
-            if (starts && k < 0) {
-#pragma unroll
-                for (int ch = 0; ch < 3; ch++)
-                    e.px[ch] = sky_base(ch) * a.sky_scale;
-            }
-            const bool eval = starts && k >= 0;
-            if (__ballot(eval)) {
-                if (eval)
-                    sample_eval<P2>(a, k, col, plane, e);
-            }
-            if (k != INT32_MIN) {
-                const size_t p = (size_t)(r0 + j) * W + col;
-#pragma unroll
-                for (int ch = 0; ch < 3; ch++) {
-                    const float d = e.px[ch] - g[ch][j];
-                    const float gd = 2.0f * d;
-                    if (a.img)
-                        a.img[ch * fplane + p] = e.px[ch];
-                    if (a.gout)
-                        a.gout[ch * fplane + p] = gd;
-                    loss_acc += d * d;
-                    g[ch][j] = gd;
-                }
-            }
-        }
-#pragma unroll
-        for (int ch = 0; ch < 3; ch++)
-            run[ch] += g[ch][j];
-        const bool ends = (j == kGradRows - 1 || src[j + 1] != k) && k != INT32_MIN;
+        if (k >= 0 && (j == 0 || src[j - 1] != k))
+            starts |= 1u << j;
         if (k < 0 && k != INT32_MIN) {
+            float gd[3] = {g[0][j], g[1][j], g[2][j]};
+            if constexpr (FWD) {
+                const float px[3] = {sky_base(0) * a.sky_scale, sky_base(1) * a.sky_scale,
+                                     sky_base(2) * a.sky_scale};
+                pixel(j, lcol, px, gd);
+            }
 #pragma unroll
             for (int ch = 0; ch < 3; ch++)
-                sky_acc += (double)g[ch][j] * (double)sky_base(ch);
+                sky_acc += (double)gd[ch] * (double)sky_base(ch);
         }
-        const bool flush = ends && k >= 0;
-        if (__ballot(flush)) {
-            float val[4][3];
-            uint32_t key[4] = {kNoKey, kNoKey, kNoKey, kNoKey};
+    }
+    while (__ballot(starts != 0u)) {
+        /* the loop's own column: the stores' addresses (two images of three
+         * planes, each row) would otherwise be formed before it and spilled */
+        uint32_t c = lcol;
+        asm volatile("" : "+v"(c));
+        float val[4][3];
+        uint32_t key[4] = {kNoKey, kNoKey, kNoKey, kNoKey};
 #pragma unroll
-            for (int t = 0; t < 4; t++)
-                val[t][0] = val[t][1] = val[t][2] = 0.0f;
-            if (flush) {
-                if constexpr (FWD)
-                    sample_grad(a, e, run, key, val);
-                else
-                    sample_terms<P2>(a, k, col, plane, run, key, val);
-            }
-            const bool last = segment_sum_quad(key, val);
+        for (int t = 0; t < 4; t++)
+            val[t][0] = val[t][1] = val[t][2] = 0.0f;
+        if (starts) {
+            const int first = __builtin_ctz(starts);
+            starts &= starts - 1u;
+            int32_t k = src[0];
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                bool inserted = false;
-                if (last && key[t] != kNoKey)
-                    inserted = table_add(keys, vals, &fill, a.gcp, plane, key[t], val[t]);
-                /* the slot count is kept per wave, not per insertion: one
-                 * LDS atomic instead of one per inserting lane */
-                const uint64_t ins = __ballot(inserted);
-                if (ins && (threadIdx.x & 63) == 0)
-                    atomicAdd(&fill, (uint32_t)__popcll(ins));
+            for (int j = 1; j < kGradRows; j++)
+                k = j == first ? src[j] : k;
+            SampleEval e;
+            sample_eval<P2, TAME>(a, k, col, plane, e);
+            float run[3] = {0.0f, 0.0f, 0.0f};
+            bool in = false;
+#pragma unroll
+            for (int j = 0; j < kGradRows; j++) {
+                in = j == first || (in && src[j] == k);
+                if (in) {
+                    float gd[3] = {g[0][j], g[1][j], g[2][j]};
+                    if constexpr (FWD)
+                        pixel(j, c, e.px, gd);
+#pragma unroll
+                    for (int ch = 0; ch < 3; ch++)
+                        run[ch] += gd[ch];
+                }
             }
+            sample_grad(a, e, run, key, val);
         }
-        if (ends) {
-            run[0] = run[1] = run[2] = 0.0f;
+        const bool last = segment_sum_quad(key, val);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            bool inserted = false;
+            if (last && key[t] != kNoKey)
+                inserted = table_add<kGradCap>(keys, vals, &fill, a.gcp, plane, key[t], val[t]);
+            /* the slot count is kept per wave, not per insertion: one
+             * LDS atomic instead of one per inserting lane */
+            const uint64_t ins = __ballot(inserted);
+            if (ins && (threadIdx.x & 63) == 0)
+                atomicAdd(&fill, (uint32_t)__popcll(ins));
         }
     }
     /* per-workgroup partials, summed in a fixed order by the next launch */
     __shared__ double wsky[kGradThreads / 64];
-    __shared__ float wloss[kGradThreads / 64];
+    __shared__ double wloss[kGradThreads / 64];
+    double loss_sum = (double)loss_acc;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         sky_acc += __shfl_xor(sky_acc, off);
         if (FWD)
-            loss_acc += __shfl_xor(loss_acc, off);
+            loss_sum += __shfl_xor(loss_sum, off);
     }
     if ((threadIdx.x & 63) == 0) {
         wsky[threadIdx.x >> 6] = sky_acc;
         if (FWD)
-            wloss[threadIdx.x >> 6] = loss_acc;
+            wloss[threadIdx.x >> 6] = loss_sum;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -3054,6 +3088,20 @@ double *g_scratch_ptr[64];   /* device address of `scratch` on each device */
 
 }  // namespace
 
+/* The adjoint's kernel for a's planes and frame, with `rows` rows per
+ * thread. */
+template <bool FWD>
+static void launch_diff_grad(const DiffArgs &a, int32_t rows, dim3 grid, hipStream_t s)
+{
+    void (*const kern[2][2][2])(DiffArgs) = {
+        {{k_diff_grad<false, false, FWD, kGradRowsLow>, k_diff_grad<false, false, FWD, kGradRowsTall>},
+         {k_diff_grad<false, true, FWD, kGradRowsLow>, k_diff_grad<false, true, FWD, kGradRowsTall>}},
+        {{k_diff_grad<true, false, FWD, kGradRowsLow>, k_diff_grad<true, false, FWD, kGradRowsTall>},
+         {k_diff_grad<true, true, FWD, kGradRowsLow>, k_diff_grad<true, true, FWD, kGradRowsTall>}}};
+    hipLaunchKernelGGL(kern[pow2(a.hc) && pow2(a.wc)][a.f.tame != 0][rows != kGradRowsLow], grid,
+                       dim3(kGradThreads), 0, s, a);
+}
+
 extern "C" {
 
 int fsk_device_init(void)
@@ -3206,7 +3254,7 @@ int fsk_render_slices(const fsk_map *m, const fsk_frame *f, const fsk_tuning *t,
 /* Rows per thread of the adjoint on a w x h frame. */
 static int32_t grad_rows(int32_t w, int32_t h)
 {
-    return (int64_t)w * (int64_t)h >= kGradTallPixels ? 4 : 2;
+    return (int64_t)w * (int64_t)h >= kGradTallPixels ? kGradRowsTall : kGradRowsLow;
 }
 
 static DiffArgs diff_args(const fsk_frame *f, const float *cp, const float *sf, int32_t hc,
@@ -3358,10 +3406,7 @@ int fsk_diff_grad(const fsk_frame *f, const float *d_cp, const float *d_sf, int3
     dim3 grid((f->cols + 63) / 64, (f->rows + br - 1) / br);
     if ((int64_t)grid.x * grid.y > n_partials)
         return hipErrorInvalidValue;
-    const bool p2 = pow2(hc) && pow2(wc), tall = rows == 4;
-    void (*kern)(DiffArgs) = p2 ? (tall ? k_diff_grad<true, false, 4> : k_diff_grad<true, false, 2>)
-                                : (tall ? k_diff_grad<false, false, 4> : k_diff_grad<false, false, 2>);
-    hipLaunchKernelGGL(kern, grid, dim3(kGradThreads), 0, s, a);
+    launch_diff_grad<false>(a, rows, grid, s);
     hipLaunchKernelGGL(k_sum_partials<double>, dim3(1), dim3(1024), 0, s, d_partials,
                        (int32_t)(grid.x * grid.y), d_gsky, sky_accumulate);
     return hipGetLastError();
@@ -3389,10 +3434,7 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
     const int64_t nb = (int64_t)grid.x * grid.y;
     if (nb > n_partials)
         return hipErrorInvalidValue;
-    const bool p2 = pow2(hc) && pow2(wc), tall = rows == 4;
-    void (*kern)(DiffArgs) = p2 ? (tall ? k_diff_grad<true, true, 4> : k_diff_grad<true, true, 2>)
-                                : (tall ? k_diff_grad<false, true, 4> : k_diff_grad<false, true, 2>);
-    hipLaunchKernelGGL(kern, grid, dim3(kGradThreads), 0, s, a);
+    launch_diff_grad<true>(a, rows, grid, s);
     hipLaunchKernelGGL(k_sum_step, dim3(1), dim3(1024), 0, s, d_loss_part, d_sky_part,
                        (int32_t)nb, d_loss, loss_accumulate, d_gsky, sky_accumulate);
     return hipGetLastError();
@@ -3499,7 +3541,7 @@ int32_t fsk_batch_max_rows(void)
 
 int32_t fsk_limit_block_rows(int32_t w, int32_t h)
 {
-    return (int64_t)w * (int64_t)h >= kGradTallPixels ? 32 : 16;
+    return (int64_t)w * (int64_t)h >= (int64_t)1 << 22 ? 32 : 16;
 }
 
 int fsk_selftest(int which, unsigned long long *d_bad, hipStream_t s)

@@ -595,3 +595,54 @@ def test_fit_follows_changed_views(ctx, share, monkeypatch):
         r.adam_step(p, g, m, s, 0.5 / 255.0, it + 1)
         torch.cuda.synchronize()
         assert abs(float(loss[0]) - losses[it]) <= 1e-5 * abs(float(loss[0]))
+
+
+@pytest.mark.parametrize("h,w,size", [(1537, 2049, 256), (1535, 2049, 256), (1537, 2049, 200)])
+def test_adjoint_rows_per_thread(ctx, h, w, size):
+    """Both adjoints against the oracle on either side of 3 * 2^20 pixels,
+    where a thread takes four rows instead of two, with ragged last blocks
+    (an odd row, one column)."""
+    col, hts = scene.scene_maps(31, 256)
+    r = DiffRenderer(ctx, ctx.map(col, hts, shade_size=size))
+    sf = O.shade_factor(O.shadow_counts(np.asarray(hts, np.int32) & 255, O.sun(0.1, 0.1), size))
+    rng = np.random.default_rng(h + size)
+    planes = rng.random((3, size, size), dtype=np.float32)
+    d, z0 = scene.depth_for(700, 500.0)
+    v = View(x=50.3, y=20.7, height=290.0, angle=0.9, horizon=0.1 * h, distance=500.0, fov=1.2,
+             h=h, w=w, d=d, z0=z0, n_slices=700)
+    tp = torch.from_numpy(planes).cuda()
+    target = torch.from_numpy(rng.random((3, h, w), dtype=np.float32)).cuda()
+    img, src, gp, gs, loss = r.l2_step(tp, 0.4, v, target)
+    gimg = torch.from_numpy(rng.standard_normal((3, h, w)).astype(np.float32)).cuda()
+    gp2, gs2 = r.vjp_raw(tp, src, gimg, v)
+    torch.cuda.synchronize()
+    want_img, want_src = O.render_f32(v, planes, sf, np.asarray(hts, np.int32) & 255, 0.4)
+    assert np.array_equal(img.cpu().numpy().view(np.uint32), want_img.view(np.uint32))
+    g = 2.0 * (want_img - target.cpu().numpy())
+    for got, sky, gi in ((gp, gs, g.astype(np.float32)), (gp2, gs2, gimg.cpu().numpy())):
+        want, want_sky = O.render_f32_vjp(v, planes, sf, want_src, gi)
+        assert _rel_err(got.cpu().numpy(), want) <= 1e-5
+        mass = np.abs(gi[:, want_src < 0]).sum() + 1e-3
+        assert abs(float(sky[0]) - float(want_sky)) <= 1e-5 * mass
+    want_loss = float(((want_img.astype(np.float64) - target.cpu().numpy()) ** 2).sum())
+    assert abs(float(loss[0]) - want_loss) <= 1e-5 * want_loss
+
+
+@pytest.mark.parametrize("size", [128, 100])
+def test_adjoint_of_slices_past_the_views_last(ctx, size):
+    """vjp over a src that names slices past the view's own count (the same
+    depths, more of them): the gradient is that of the longer view."""
+    import dataclasses
+    r, col, _, _ = _setup(ctx, size=128)
+    r = DiffRenderer(ctx, ctx.map(*scene.scene_maps(11, 128), shade_size=size))
+    long = dataclasses.replace(VIEWS[0], n_slices=200)
+    short = dataclasses.replace(long, n_slices=20)
+    planes = torch.from_numpy(np.ascontiguousarray(planes_of(col)[:, :size, :size])).cuda()
+    src = r.forward_raw(planes, 0.3, long)[1]
+    rng = np.random.default_rng(5)
+    gimg = torch.from_numpy(rng.standard_normal((3, long.h, long.w)).astype(np.float32)).cuda()
+    want = r.vjp_raw(planes, src, gimg, long)[0]
+    got = r.vjp_raw(planes, src, gimg, short)[0]
+    torch.cuda.synchronize()
+    assert int(src.max()) >= 20
+    assert _rel_err(got.cpu().numpy(), want.cpu().numpy()) <= 1e-5
