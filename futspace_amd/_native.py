@@ -118,6 +118,7 @@ FUTSPACE_SIGNATURES = {
                                           P, P]),
     "fsx_l2_loss": (ctypes.c_int, [P, P, P, I64, I32, P, P]),
     "fsx_adam_step": (ctypes.c_int, [P, P, P, P, P, I64, F64, F64, F64, F64, I32, F32, F32]),
+    "fsx_adam_first_step": (ctypes.c_int, [P, P, P, P, P, I64, F64, F64, F64, F64, F32, F32]),
     "fsx_render_f32_l2_step": (ctypes.c_int, [P, P, ctypes.POINTER(FsxView), P, P, I32, I32, F32,
                                               P, I32, P, P, P, P, P, P]),
     "fsx_f32_l2_step_visible": (ctypes.c_int, [P, ctypes.POINTER(FsxView), P, P, I32, I32, F32, P,

@@ -1895,9 +1895,10 @@ int fsx_f32_l2_step_visible(struct futhark_context *ctx, const struct fsx_view *
                    dev_gplanes, dev_gsky, dev_loss);
 }
 
-int fsx_adam_step(struct futhark_context *ctx, float *dev_param, const float *dev_grad,
-                  float *dev_m, float *dev_v, int64_t n, double lr, double beta1,
-                  double beta2, double eps, int32_t step, float lo, float hi)
+static int adam_step(struct futhark_context *ctx, const char *who, float *dev_param,
+                     const float *dev_grad, float *dev_m, float *dev_v, int64_t n, double lr,
+                     double beta1, double beta2, double eps, int32_t step, int first, float lo,
+                     float hi)
 {
     if (!ctx)
         return 1;
@@ -1905,14 +1906,30 @@ int fsx_adam_step(struct futhark_context *ctx, float *dev_param, const float *de
         ((!dev_param || !dev_grad || !dev_m || !dev_v) && n > 0) ||
         (((uintptr_t)dev_param | (uintptr_t)dev_grad | (uintptr_t)dev_m | (uintptr_t)dev_v) &
          15u)) {
-        set_error(ctx, "fsx_adam_step: invalid arguments (null or misaligned buffer, step < 1 "
-                       "or a beta outside [0, 1))");
+        set_error(ctx, "%s: invalid arguments (null or misaligned buffer, step < 1 "
+                       "or a beta outside [0, 1))", who);
         return 1;
     }
     HIPCHECK(ctx, hipSetDevice(ctx->device));
     HIPCHECK(ctx, fsk_adam(dev_param, dev_grad, dev_m, dev_v, (size_t)n, lr, beta1, beta2, eps,
-                           step, lo, hi, ctx->stream));
+                           step, first, lo, hi, ctx->stream));
     return 0;
+}
+
+int fsx_adam_step(struct futhark_context *ctx, float *dev_param, const float *dev_grad,
+                  float *dev_m, float *dev_v, int64_t n, double lr, double beta1,
+                  double beta2, double eps, int32_t step, float lo, float hi)
+{
+    return adam_step(ctx, "fsx_adam_step", dev_param, dev_grad, dev_m, dev_v, n, lr, beta1, beta2,
+                     eps, step, 0, lo, hi);
+}
+
+int fsx_adam_first_step(struct futhark_context *ctx, float *dev_param, const float *dev_grad,
+                        float *dev_m, float *dev_v, int64_t n, double lr, double beta1,
+                        double beta2, double eps, float lo, float hi)
+{
+    return adam_step(ctx, "fsx_adam_first_step", dev_param, dev_grad, dev_m, dev_v, n, lr, beta1,
+                     beta2, eps, 1, 1, lo, hi);
 }
 
 int fsx_l2_loss(struct futhark_context *ctx, const float *dev_img, const float *dev_target,

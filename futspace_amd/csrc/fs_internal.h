@@ -190,10 +190,11 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
                      double *d_loss_part, double *d_sky_part, int32_t n_partials, hipStream_t s);
 int fsk_zero_f32(float *d_p, size_t n, hipStream_t s);
 /* One bias-corrected Adam step (step t >= 1) on d_p[n] with gradient d_g
- * and moments d_m, d_v, then d_p clamped to [lo, hi]. */
+ * and moments d_m, d_v, then d_p clamped to [lo, hi].  first: the moments
+ * are zero and only written. */
 int fsk_adam(float *d_p, const float *d_g, float *d_m, float *d_v, size_t n, double lr,
-             double beta1, double beta2, double eps, int32_t step, float lo, float hi,
-             hipStream_t s);
+             double beta1, double beta2, double eps, int32_t step, int32_t first, float lo,
+             float hi, hipStream_t s);
 int fsk_fill_u32(uint32_t *d_p, size_t n, uint32_t v, hipStream_t s);
 /* Reductions write one partial sum per workgroup into d_partials (at most
  * n_partials) and a one-workgroup pass adds their sum, in a fixed order,

@@ -181,16 +181,26 @@ class DiffRenderer:
         return img, src, gplanes, gsky, loss
 
     def adam_step(self, param, grad, m, v, lr, step, betas=(0.9, 0.999), eps=1e-8, lo=0.0,
-                  hi=1.0):
+                  hi=1.0, first=False):
         """One Adam step (fsx_adam_step: bias-corrected, no weight decay,
         step >= 1) on param in place, its moments m and v updated in place,
-        then param clamped to [lo, hi]; on the context stream."""
+        then param clamped to [lo, hi]; on the context stream.  With
+        first=True (and step 1) the moments are taken as zero and only
+        written (fsx_adam_first_step)."""
+        if first and step != 1:
+            raise ValueError("first=True is step 1")
         for t in (param, grad, m, v):
             if (t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous()
                     or t.shape != param.shape):
                 raise ValueError("param, grad, m and v must be contiguous CUDA float32 "
                                  "tensors of one shape")
         with self.stream():
+            if first:
+                self.ctx.check(self.ctx.lib.fsx_adam_first_step(
+                    self.ctx.ptr, _ptr(param), _ptr(grad), _ptr(m), _ptr(v), param.numel(),
+                    float(lr), float(betas[0]), float(betas[1]), float(eps), ctypes.c_float(lo),
+                    ctypes.c_float(hi)), "fsx_adam_first_step")
+                return
             self.ctx.check(self.ctx.lib.fsx_adam_step(
                 self.ctx.ptr, _ptr(param), _ptr(grad), _ptr(m), _ptr(v), param.numel(),
                 float(lr), float(betas[0]), float(betas[1]), float(eps), int(step),
@@ -254,8 +264,8 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     planes.requires_grad_(False)
     step_lr = lr / COLOUR_UNIT
     grad = torch.zeros_like(planes)
-    m = torch.zeros_like(planes)
-    v = torch.zeros_like(planes)
+    m = torch.empty_like(planes)
+    v = torch.empty_like(planes)      # the first step writes both moments
     gsky = torch.zeros(1, dtype=torch.float32, device="cuda")
     held = {}                 # view number -> (view, map, its visible slices)
     room = int(torch.cuda.get_device_properties(planes.device).total_memory * FIT_VISIBLE_SHARE)
@@ -285,7 +295,7 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
                 renderer.l2_step(planes, sky_scale, view, t, None, src, None, grad, gsky,
                                  losses[it:it + 1], accumulate=i > 0, outputs=False,
                                  visible=known)
-            renderer.adam_step(planes, grad, m, v, step_lr, it + 1)
+            renderer.adam_step(planes, grad, m, v, step_lr, it + 1, first=it == 0)
         if on_step is not None:
             on_step(it)
     return losses

@@ -262,6 +262,12 @@ int fsx_adam_step(struct futhark_context *ctx, float *dev_param, const float *de
                   float *dev_m, float *dev_v, int64_t n, double lr, double beta1,
                   double beta2, double eps, int32_t step, float lo, float hi);
 
+/* fsx_adam_step with step 1 from zero moments: dev_m and dev_v are written
+ * but not read, and need not hold anything. */
+int fsx_adam_first_step(struct futhark_context *ctx, float *dev_param, const float *dev_grad,
+                        float *dev_m, float *dev_v, int64_t n, double lr, double beta1,
+                        double beta2, double eps, float lo, float hi);
+
 /* One fitting step of the differentiable renderer in one call: the same
  * results as fsx_render_f32, then fsx_l2_loss against dev_target[3][h][w]
  * (dev_gimg = 2 (img - target), *dev_loss), then fsx_render_f32_vjp with

@@ -646,3 +646,23 @@ def test_adjoint_of_slices_past_the_views_last(ctx, size):
     torch.cuda.synchronize()
     assert int(src.max()) >= 20
     assert _rel_err(got.cpu().numpy(), want.cpu().numpy()) <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 1027, 4096 * 1024 + 5])
+def test_adam_first_step_takes_the_moments_as_zero(ctx, n):
+    """adam_step(first=True) over moments of any content: bit for bit the
+    first step from zero moments (vector part and scalar tail)."""
+    r, _, _, _ = _setup(ctx)
+    rng = np.random.default_rng(n)
+    p = torch.from_numpy(rng.random(n, dtype=np.float32)).cuda()
+    g = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
+    g[0] = -0.0
+    q, zeros = p.clone(), [torch.zeros_like(p) for _ in range(2)]
+    junk = [torch.full_like(p, float("nan")) for _ in range(2)]
+    r.adam_step(p, g, *zeros, 0.01, 1)
+    r.adam_step(q, g, *junk, 0.01, 1, first=True)
+    torch.cuda.synchronize()
+    for a, b in zip([p] + zeros, [q] + junk):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    with pytest.raises(ValueError):
+        r.adam_step(p, g, *zeros, 0.01, 2, first=True)
