@@ -2699,17 +2699,24 @@ __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval 
  * is one visible sample: its incoming gradient is summed in registers and
  * pushed through the three mixes once.  For px = mix(wy0, X1, wy1, X2),
  * X1 = mix(wx0, s0, wx1, s1): d px / d s0 = wy0' * wx0' * s0 / px (X1
- * cancels), likewise for the other texels, 0 where px == 0.  The texel
- * terms are summed in two stages before any global atomic: lanes of a
- * wave that end a run on the same row and hit the same texel (adjacent
+ * cancels), likewise for the other texels, 0 where px == 0.  A wave loops over
+ * its lanes' runs, every lane at its next one wherever that starts: row by
+ * row, a wave evaluated and inserted on each row where any lane began a run
+ * (0.94 of a 4K view's rows; now 0.66 evaluations per row, 54 M instead of
+ * 70 M vector instructions).  The texel terms are summed in two stages before
+ * any global atomic: lanes of a wave whose runs hit the same texels (adjacent
  * columns magnifying one near texel) are merged by a segmented reduction
  * across the wave, so that the LDS table below sees distinct texels per
  * instruction; then an LDS hash table sums the terms per texel over the
  * whole block (neighbouring samples share texels: a block touches
- * several times fewer texels than it has sample-texel terms).  Short
- * per-thread row runs keep many waves in flight for the gathers.  Each
- * table entry is then added into the global f32 gradient with one atomic
- * per channel.
+ * several times fewer texels than it has sample-texel terms).  Few rows per
+ * thread keep many waves in flight for the gathers.  Each table entry is then
+ * added into the global f32 gradient with one atomic per channel.
+ *
+ * What bounds it: in large frames the vector instructions (3840 x 2160 fitting
+ * view 127 -> 92 us); in small ones the inserts and the flush's atomics, with
+ * the latency of a block's chain behind them (1280 x 720: 51 -> 46 us, 24
+ * without inserts; 800 x 600 vjp 32 -> 26 us).
  *
  * FWD (the fused L2 step): the incoming gradient is not read but formed
  * here from the target, g = 2 (px - target), with the colour px of each
