@@ -2246,7 +2246,7 @@ __device__ __forceinline__ void block_sum_partials(const T *__restrict__ part, i
         double t = 0.0;
         for (int w = 0; w < NT / 64; w++)
             t += wsum[w];
-        *dst = accumulate ? *dst + (float)t : (float)t;
+        *dst = (float)(accumulate ? (double)*dst + t : t);
     }
 }
 
@@ -2773,8 +2773,7 @@ void k_diff_grad(DiffArgs a)
     __syncthreads();
     /* the sky term cancels where gradients of both signs meet: f64 keeps its
      * sum as exact as the gradients */
-    double sky_acc = 0.0;
-    float loss_acc = 0.0f;
+    double sky_acc = 0.0, loss_sum = 0.0;
     /* one pixel of the fused step: its loss term and g = 2 (px - target) */
     auto pixel = [&](int j, uint32_t c, const float px[3], float (&gd)[3]) {
         const size_t row = (size_t)(r0 + j) * W;
@@ -2786,7 +2785,7 @@ void k_diff_grad(DiffArgs a)
                 ((FS_GLOBAL float *)a.img + ch * fplane + row)[c] = px[ch];
             if (a.gout)
                 ((FS_GLOBAL float *)a.gout + ch * fplane + row)[c] = gd[ch];
-            loss_acc += d * d;
+            loss_sum += (double)d * (double)d;
         }
     };
     uint32_t starts = 0u;      /* rows where a run of a visible sample starts */
@@ -2858,7 +2857,6 @@ void k_diff_grad(DiffArgs a)
     /* per-workgroup partials, summed in a fixed order by the next launch */
     __shared__ double wsky[kGradThreads / 64];
     __shared__ double wloss[kGradThreads / 64];
-    double loss_sum = (double)loss_acc;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         sky_acc += __shfl_xor(sky_acc, off);
@@ -2941,7 +2939,7 @@ __global__ __launch_bounds__(1024) void k_sum_step(const double *__restrict__ lo
         for (int w = 0; w < NT / 64; w++)
             t += wsum[k][w];
         float *dst = k ? gsky : loss;
-        *dst = (k ? sky_acc : loss_acc) ? *dst + (float)t : (float)t;
+        *dst = (float)((k ? sky_acc : loss_acc) ? (double)*dst + t : t);
     }
 }
 
