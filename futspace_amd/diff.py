@@ -16,7 +16,6 @@ and torch's current stream waits for it afterwards.
 """
 import contextlib
 import ctypes
-import dataclasses
 
 import numpy as np
 import torch
@@ -267,7 +266,7 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     m = torch.empty_like(planes)
     v = torch.empty_like(planes)      # the first step writes both moments
     gsky = torch.zeros(1, dtype=torch.float32, device="cuda")
-    held = {}                 # view number -> (view, map, its visible slices)
+    held = {}                 # view number -> (view's C form, map, its visible slices)
     room = int(torch.cuda.get_device_properties(planes.device).total_memory * FIT_VISIBLE_SHARE)
     shared = None             # the visible slices of a view that found no room
     losses = torch.zeros(steps, dtype=torch.float32, device="cuda")
@@ -276,16 +275,19 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
         # the views' calls and the optimizer step queue back to back
         with renderer.stream():
             for i, (view, t) in enumerate(zip(views, targets)):
-                have = held.get(i)
-                known = have is not None and have[0] == view and have[1] is renderer.map
+                # the values that the renderer gets decide, not the objects
+                # that hold them; a closed map is refused by the step itself
+                have, key = held.get(i), bytes(view.to_c())
+                known = (have is not None and have[0] == key and have[1] is renderer.map
+                         and bool(renderer.map.ptr))
                 if known:
                     src = have[2]
                 elif have is not None and tuple(have[2].shape) == (view.h, view.w):
                     src = have[2]
-                    held[i] = (dataclasses.replace(view), renderer.map, src)
+                    held[i] = (key, renderer.map, src)
                 elif have is None and 4 * view.h * view.w <= room:
                     src = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
-                    held[i] = (dataclasses.replace(view), renderer.map, src)
+                    held[i] = (key, renderer.map, src)
                     room -= 4 * view.h * view.w
                 else:
                     if shared is None or tuple(shared.shape) != (view.h, view.w):

@@ -666,3 +666,63 @@ def test_adam_first_step_takes_the_moments_as_zero(ctx, n):
         assert torch.equal(a.view(torch.int32), b.view(torch.int32))
     with pytest.raises(ValueError):
         r.adam_step(p, g, *zeros, 0.01, 2, first=True)
+
+
+class _Recorder(DiffRenderer):
+    """A renderer that notes, per l2_step, whether src was given as known and
+    where it lies."""
+
+    def __init__(self, *args):
+        super().__init__(*args)
+        self.known, self.at = [], []
+
+    def l2_step(self, planes, sky, view, target, img=None, src=None, *args, visible=False, **kw):
+        self.known.append(visible)
+        self.at.append(src.data_ptr())
+        return super().l2_step(planes, sky, view, target, img, src, *args, visible=visible, **kw)
+
+
+def _fit_setup(ctx, views):
+    _, col, _, _ = _setup(ctx)
+    r = _Recorder(ctx, ctx.map(*scene.scene_maps(11, 128), shade_size=128))
+    planes = torch.from_numpy(planes_of(col)).cuda()
+    goal = (planes * 0.5).contiguous()
+    targets = [r.forward_raw(goal, 0.3, v)[0] for v in views]
+    torch.cuda.synchronize()
+    return r, planes, goal, targets
+
+
+def test_fit_follows_a_camera_moved_in_place(ctx):
+    """A view whose fields are arrays that on_step changes in place is
+    rendered anew: what counts are the values handed to the renderer, not the
+    objects that hold them."""
+    import dataclasses
+    view = dataclasses.replace(VIEWS[0], x=np.array(VIEWS[0].x))
+    r, planes, goal, targets = _fit_setup(ctx, [view])
+    moved = dataclasses.replace(VIEWS[0], x=float(view.x) + 7.25)
+
+    def move(it):
+        if it == 0:
+            view.x += 7.25
+            targets[0] = r.forward_raw(goal, 0.3, moved)[0]
+
+    fit(r, planes, [view], targets, 0.3, steps=3, on_step=move)
+    assert r.known == [False, False, True]
+
+
+def test_fit_takes_any_view_that_gives_its_c_form(ctx):
+    """A camera needs h, w and to_c, and no more."""
+    from types import SimpleNamespace
+    view = SimpleNamespace(h=VIEWS[0].h, w=VIEWS[0].w, to_c=VIEWS[0].to_c)
+    r, planes, _, targets = _fit_setup(ctx, [VIEWS[0]])
+    other = planes.clone()
+    losses = fit(r, planes, [view], targets, 0.3, steps=2).cpu().numpy()
+    want = fit(r, other, [VIEWS[0]], targets, 0.3, steps=2).cpu().numpy()
+    assert np.allclose(losses, want, rtol=1e-5, atol=0.0)
+    assert r.known == [False, True, False, True]
+
+
+def test_fit_refuses_a_map_closed_meanwhile(ctx):
+    r, planes, _, targets = _fit_setup(ctx, [VIEWS[0]])
+    with pytest.raises(Exception, match="fsx_render_f32_l2_step"):
+        fit(r, planes, [VIEWS[0]], targets, 0.3, steps=2, on_step=lambda it: r.map.close())
