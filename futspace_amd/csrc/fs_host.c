@@ -19,6 +19,7 @@
 
 #include <math.h>
 #include <stdarg.h>
+#include <stdatomic.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -45,6 +46,7 @@ struct fs_shade;
 
 struct futhark_context {
     int device;
+    uint64_t id;              /* of no other context, before or after */
     int debugging, logging;
     hipStream_t own_stream;
     hipStream_t stream;
@@ -196,14 +198,16 @@ static void dev_release(struct futhark_context *ctx, void *p, size_t bytes)
         pool_put(ctx, p, bytes ? bytes : 4, 0);
 }
 
-/* dev_release of a map buffer: at most FS_POOL_MAP_BYTES of them are kept. */
-static void map_release(struct futhark_context *ctx, void *p, size_t bytes)
+/* dev_release of a map buffer: at most FS_POOL_MAP_BYTES of them are kept.
+ * A buffer that other streams than the context's may be reading (not pooled)
+ * is freed, which waits for the whole device. */
+static void map_release(struct futhark_context *ctx, void *p, size_t bytes, int pooled)
 {
     if (!p)
         return;
     if (bytes == 0)
         bytes = 4;
-    if (bytes > FS_POOL_MAP_BYTES) {
+    if (!pooled || bytes > FS_POOL_MAP_BYTES) {
         hipStreamSynchronize(ctx->stream);
         hipFree(p);
         return;
@@ -325,6 +329,8 @@ struct futhark_context *futhark_context_new(struct futhark_context_config *cfg)
         return NULL;
     }
     ctx->stream = ctx->own_stream;
+    static atomic_uint_fast64_t contexts;
+    ctx->id = atomic_fetch_add(&contexts, 1) + 1;
     fsk_default_tuning(&ctx->tune);
     if (fsk_device_init() != hipSuccess) {
         fprintf(stderr, "futspace: device table upload failed\n");
@@ -668,8 +674,18 @@ const int64_t *futhark_shape_i32_2d(struct futhark_context *ctx, struct futhark_
 /* colours), both immutable and reference-counted so states share them */
 /* ------------------------------------------------------------------ */
 
+/* Who may be reading a resident object's buffers.  Work of its owner on the
+ * owner's one stream is in order with a later use of the buffers, so that they
+ * can be pooled on release without a wait; work of another context, or a
+ * captured graph, which replays on any stream, is not. */
+struct fs_readers {
+    uint64_t owner;        /* id of the context that made it */
+    int elsewhere;         /* read outside the owner's stream order */
+};
+
 struct fs_terrain {
     int refs;
+    struct fs_readers readers;
     int32_t rows, cols, hbits;
     void *d_hq;            /* bilinear height quads */
     uint16_t *d_hp;        /* masked heights, one per texel */
@@ -680,6 +696,7 @@ struct fs_terrain {
 
 struct fs_shade {
     int refs;
+    struct fs_readers readers;
     int32_t rows, cols;
     float sun[3];          /* the sun vector it was shaded with */
     uint32_t *d_shaded;
@@ -691,6 +708,28 @@ struct fsx_map {
     struct fs_shade *s;
     int32_t shade_size;
 };
+
+/* ctx is about to queue work that reads t and s (either may be NULL).
+ * Copies and batches need no note: the one is waited for, and the other keeps
+ * its references until its own memory has been freed. */
+static void note_readers(struct futhark_context *ctx, struct fs_terrain *t, struct fs_shade *s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+    }
+    const int graph = cap != hipStreamCaptureStatusNone;
+    if (t && (graph || t->readers.owner != ctx->id))
+        t->readers.elsewhere = 1;
+    if (s && (graph || s->readers.owner != ctx->id))
+        s->readers.elsewhere = 1;
+}
+
+static int only_read_by(const struct futhark_context *ctx, const struct fs_readers *r)
+{
+    return r->owner == ctx->id && !r->elsewhere;
+}
 
 static size_t terrain_texels(const struct fs_terrain *t)
 {
@@ -712,9 +751,10 @@ static void terrain_unref(struct futhark_context *ctx, struct fs_terrain *t)
 {
     if (!t || --t->refs > 0)
         return;
-    map_release(ctx, t->d_hq, terrain_hq_bytes(t));
-    map_release(ctx, t->d_hp, terrain_hp_bytes(t) + FSK_HMAX_PARTS * 4);
-    map_release(ctx, t->d_color, terrain_texels(t) * 4);
+    const int pooled = only_read_by(ctx, &t->readers);
+    map_release(ctx, t->d_hq, terrain_hq_bytes(t), pooled);
+    map_release(ctx, t->d_hp, terrain_hp_bytes(t) + FSK_HMAX_PARTS * 4, pooled);
+    map_release(ctx, t->d_color, terrain_texels(t) * 4, pooled);
     free(t->h_alt);
     free(t);
 }
@@ -724,8 +764,9 @@ static void shade_unref(struct futhark_context *ctx, struct fs_shade *s)
     if (!s || --s->refs > 0)
         return;
     const size_t n = (size_t)s->rows * (size_t)s->cols;
-    map_release(ctx, s->d_shaded, n * 4);
-    map_release(ctx, s->d_cq, n * 16);
+    const int pooled = only_read_by(ctx, &s->readers);
+    map_release(ctx, s->d_shaded, n * 4, pooled);
+    map_release(ctx, s->d_cq, n * 16, pooled);
     free(s);
 }
 
@@ -745,6 +786,7 @@ static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_
     if (!t)
         return NULL;
     t->refs = 1;
+    t->readers.owner = ctx->id;
     t->rows = rows;
     t->cols = cols;
     t->hbits = hbits;
@@ -798,13 +840,14 @@ static void sun_vector(float sun_height, float sun_ang, float out[3])
     out[2] = (-sa) * v0;
 }
 
-static struct fs_shade *shade_new(struct futhark_context *ctx, const struct fs_terrain *t,
+static struct fs_shade *shade_new(struct futhark_context *ctx, struct fs_terrain *t,
                                   int32_t size, float sun_height, float sun_ang)
 {
     struct fs_shade *s = (struct fs_shade *)calloc(1, sizeof *s);
     if (!s)
         return NULL;
     s->refs = 1;
+    s->readers.owner = ctx->id;
     s->rows = size;
     s->cols = size;
     size_t n = (size_t)size * (size_t)size;
@@ -814,6 +857,7 @@ static struct fs_shade *shade_new(struct futhark_context *ctx, const struct fs_t
         return NULL;
     }
     sun_vector(sun_height, sun_ang, s->sun);
+    note_readers(ctx, t, NULL);
     hipError_t e = (hipError_t)fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, t->d_color, s->sun, size,
                               s->d_shaded, ctx->stream);
     if (e == hipSuccess)
@@ -851,6 +895,7 @@ static struct fs_shade *shade_zero(struct futhark_context *ctx)
     if (!s)
         return NULL;
     s->refs = 1;
+    s->readers.owner = ctx->id;
     s->rows = 2;
     s->cols = 1;
     if (dev_alloc(ctx, (void **)&s->d_shaded, 8) || dev_alloc(ctx, &s->d_cq, 32) ||
@@ -917,9 +962,8 @@ static void frame_of_view(const struct fsx_view *v, fsk_frame *f)
     f->tame = 0;
 }
 
-static int render_into(struct futhark_context *ctx, const struct fs_terrain *t,
-                       const struct fs_shade *s, const struct fsx_view *v,
-                       uint32_t *d_out, int64_t pitch)
+static int render_into(struct futhark_context *ctx, struct fs_terrain *t, struct fs_shade *s,
+                       const struct fsx_view *v, uint32_t *d_out, int64_t pitch)
 {
     if (v->h < 0 || v->w < 0) {
         set_error(ctx, "render: negative frame size %d x %d", v->h, v->w);
@@ -944,6 +988,7 @@ static int render_into(struct futhark_context *ctx, const struct fs_terrain *t,
     m.crows = s->rows;
     m.ccols = s->cols;
     HIPCHECK(ctx, hipSetDevice(ctx->device));
+    note_readers(ctx, t, s);
     int pe = prof_begin(ctx);
     HIPCHECK(ctx, fsk_render(&m, &f, &ctx->tune, d_out, pitch > 0 ? pitch : v->w, ctx->stream));
     prof_end(ctx, pe);
@@ -1471,7 +1516,7 @@ int fsx_map_new(struct futhark_context *ctx, struct fsx_map **out,
         m = NULL;
         rc = 1;
     }
-    map_release(ctx, d_alt, bytes);
+    map_release(ctx, d_alt, bytes, 1);
     *out = m;
     return rc;
 }
@@ -1576,6 +1621,7 @@ int fsx_render2(struct futhark_context *ctx, const struct fsx_map *map,
     m.cq = NULL;
     m.crows = 0;
     m.ccols = 0;
+    note_readers(ctx, map->t, NULL);
     int pe = prof_begin(ctx);
     HIPCHECK(ctx, fsk_render2(&m, &f, ctx->d_trig, ctx->d_trig + view->w, map->t->d_color, n,
                               dev_out, pitch > 0 ? pitch : view->w, ctx->stream));
@@ -1672,6 +1718,7 @@ int fsx_map_shade_factor(struct futhark_context *ctx, const struct fsx_map *map,
     const struct fs_terrain *t = map->t;
     const struct fs_shade *s = map->s;
     HIPCHECK(ctx, hipSetDevice(ctx->device));
+    note_readers(ctx, map->t, NULL);
     HIPCHECK(ctx, fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, NULL, s->sun, s->rows, dev_sf,
                             ctx->stream));
     return 0;
@@ -1731,6 +1778,7 @@ int fsx_render_f32(struct futhark_context *ctx, const struct fsx_map *map,
     m.crows = hc;
     m.ccols = wc;
     HIPCHECK(ctx, hipSetDevice(ctx->device));
+    note_readers(ctx, map->t, NULL);
     int pe = prof_begin(ctx);
     HIPCHECK(ctx, fsk_render_slices(&m, &f, &ctx->tune, dev_src, view->w, ctx->stream));
     HIPCHECK(ctx, fsk_diff_color(&f, dev_planes, dev_sf, hc, wc, sky_scale, dev_src, dev_img,
@@ -1833,6 +1881,7 @@ static int l2_step(struct futhark_context *ctx, const char *what, int noalloc,
      * launch of their own */
     int32_t cleared = 0;
     if (map) {
+        note_readers(ctx, map->t, NULL);
         fsk_map m;
         m.hq = map->t->d_hq;
         m.hrows = map->t->rows;
@@ -2259,7 +2308,7 @@ int fsx_batch_free(struct futhark_context *ctx, struct fsx_batch *batch)
         hipGraphExecDestroy(batch->exec);
     if (batch->graph)
         hipGraphDestroy(batch->graph);
-    hipFree(batch->d_mem);
+    hipFree(batch->d_mem);        /* waits for every stream: no reader is left */
     for (int32_t i = 0; i < batch->n_maps; i++) {
         terrain_unref(ctx, batch->terrains[i]);
         shade_unref(ctx, batch->shades[i]);

@@ -149,6 +149,11 @@ struct fsx_map;
 int fsx_map_new(struct futhark_context *ctx, struct fsx_map **out,
                 const uint32_t *color, const int32_t *height, int64_t rows, int64_t cols,
                 int32_t height_bits, int32_t shade_size, float sun_height, float sun_ang);
+/* The map may be read by any context on its device.  On return every reader
+ * of its buffers has ended, or is ordered before their next use: readers on the
+ * stream of the context that made it by stream order, readers of other
+ * contexts and captured graphs by a wait for the device.  A graph that reads
+ * the map must not be launched afterwards. */
 int fsx_map_free(struct futhark_context *ctx, struct fsx_map *map);
 /* Copy the shaded colour map (shade_size^2 u32) to host memory. */
 int fsx_map_shaded(struct futhark_context *ctx, const struct fsx_map *map, uint32_t *host_out);

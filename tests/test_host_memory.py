@@ -1,0 +1,131 @@
+"""Device memory as the host code handles it, without a GPU: fs_host.c over a
+HIP runtime of host memory (hip_stub.c) that counts allocations and frees."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from futspace_amd import View
+from futspace_amd._native import FUTSPACE_SIGNATURES
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SIDE = 32
+VIEW = View(x=3.0, y=4.0, height=300.0, angle=0.4, horizon=8.0, h=12, w=16, d=0.01, z0=0.5)
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libstub.so")
+    subprocess.run(["gcc", "-std=gnu11", "-O1", "-fPIC", "-shared", "-ffp-contract=off", "-w",
+                    "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", out,
+                    os.path.join(ROOT, "futspace_amd", "csrc", "fs_host.c"),
+                    os.path.join(ROOT, "tests", "hip_stub.c"), "-lm"], check=True)
+    so = ctypes.CDLL(out)
+    for name, (res, args) in FUTSPACE_SIGNATURES.items():
+        if hasattr(so, name):
+            getattr(so, name).restype, getattr(so, name).argtypes = res, args
+    return so
+
+
+class Ctx:
+    """A context of the stub, freed at the end of the test."""
+
+    def __init__(self, lib):
+        self.lib, self.ptr = lib, lib.futhark_context_new(None)
+        assert self.ptr
+
+    def map(self, side=SIDE, want=0):
+        p = ctypes.c_void_p()
+        a = np.zeros((side, side), np.uint32)
+        rc = self.lib.fsx_map_new(self.ptr, ctypes.byref(p), a.ctypes.data,
+                                  a.ctypes.data, side, side, 8, side, 0.1, 0.1)
+        assert rc == want
+        return p.value
+
+    def free(self, m):
+        assert self.lib.fsx_map_free(self.ptr, m) == 0
+
+    def output(self, nbytes=12 * 16 * 4):
+        return ctypes.create_string_buffer(nbytes)
+
+
+def _get(lib, name, kind=ctypes.c_int64):
+    return kind.in_dll(lib, name).value
+
+
+def _set(lib, name, value, kind=ctypes.c_int64):
+    kind.in_dll(lib, name).value = value
+
+
+@pytest.fixture
+def contexts(lib):
+    made = [Ctx(lib), Ctx(lib)]
+    yield made
+    _set(lib, "stub_capturing", 0, ctypes.c_int)
+    _set(lib, "stub_limit", 2 ** 63 - 1)
+    for c in made:
+        lib.futhark_context_free(c.ptr)
+
+
+def _readers(lib, c, m):
+    """The calls that queue work over a map's buffers."""
+    view, f32 = VIEW.to_c(), ctypes.create_string_buffer(64 * SIDE * SIDE)
+    ref = ctypes.byref(view)
+    return {
+        "render": lambda: lib.fsx_render(c.ptr, m, ref, f32, 0),
+        "render2": lambda: lib.fsx_render2(c.ptr, m, ref, f32, 0),
+        "shade_factor": lambda: lib.fsx_map_shade_factor(c.ptr, m, f32),
+        "forward": lambda: lib.fsx_render_f32(c.ptr, m, ref, f32, f32, SIDE, SIDE, 0.1, f32, f32),
+        "step": lambda: lib.fsx_render_f32_l2_step_noalloc(
+            c.ptr, m, ref, f32, f32, SIDE, SIDE, 0.1, f32, 0, f32, f32, f32, f32, f32, f32),
+    }
+
+
+MAP_BUFFERS = 5      # heights twice, colours, shaded colours and their quads
+
+
+@pytest.mark.parametrize("call", ["render", "render2", "shade_factor", "forward", "step"])
+@pytest.mark.parametrize("where", ["own", "other", "graph"])
+def test_buffers_read_elsewhere_are_freed_and_not_reused(lib, contexts, call, where):
+    """A map that another context or a captured graph reads goes back to the
+    driver, whose free waits for the device; only a map that the owner's own
+    stream alone reads is kept for the next load."""
+    a, b = contexts
+    m = a.map()
+    _set(lib, "stub_capturing", int(where == "graph"), ctypes.c_int)
+    assert _readers(lib, b if where == "other" else a, m)[call]() == 0
+    _set(lib, "stub_capturing", 0, ctypes.c_int)
+    frees = _get(lib, "stub_frees")
+    a.free(m)
+    freed = _get(lib, "stub_frees") - frees
+    # only render reads the shade's two buffers as well
+    assert freed == (0 if where == "own" else MAP_BUFFERS if call == "render" else 3)
+
+
+def test_a_map_freed_through_another_context_leaves_no_pool(lib, contexts):
+    a, b = contexts
+    m = a.map()
+    frees = _get(lib, "stub_frees")
+    b.free(m)
+    assert _get(lib, "stub_frees") - frees == MAP_BUFFERS
+
+
+def test_a_state_rendered_elsewhere_keeps_its_buffers_out_of_the_pool(lib, contexts):
+    a, b = contexts
+    maps = np.zeros((SIDE, SIDE), np.uint32)
+    col = lib.futhark_new_u32_2d(a.ptr, maps.ctypes.data, SIDE, SIDE)
+    hts = lib.futhark_new_i32_2d(a.ptr, maps.ctypes.data, SIDE, SIDE)
+    s0, s1, out = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.futhark_entry_init(a.ptr, ctypes.byref(s0), 0) == 0
+    assert lib.futhark_entry_update_map(a.ptr, ctypes.byref(s1), ctypes.c_void_p(col),
+                                        ctypes.c_void_p(hts), s0) == 0
+    assert lib.futhark_entry_render(b.ptr, ctypes.byref(out), s1) == 0
+    frees = _get(lib, "stub_frees")
+    lib.futhark_free_opaque_state(a.ptr, s1)
+    assert _get(lib, "stub_frees") - frees == MAP_BUFFERS
+    lib.futhark_free_opaque_state(a.ptr, s0)
+    lib.futhark_free_u32_2d(a.ptr, col)
+    lib.futhark_free_i32_2d(a.ptr, hts)
+    lib.futhark_free_u32_2d(b.ptr, out)
