@@ -127,6 +127,33 @@ static void set_error(struct futhark_context *ctx, const char *fmt, ...)
         }                                                                           \
     } while (0)
 
+static void pool_clear(struct futhark_context *ctx)
+{
+    for (int i = 0; i < FS_POOL_SLOTS; i++)
+        if (ctx->pool[i].ptr) {
+            hipFree(ctx->pool[i].ptr);
+            ctx->pool[i].ptr = NULL;
+        }
+}
+
+/* hipMalloc that gives the pooled buffers back and tries once more when
+ * memory runs out.  A failed call stays HIP's last error until it is asked
+ * for, and the next launch would report it as its own. */
+static hipError_t dev_malloc(struct futhark_context *ctx, void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        pool_clear(ctx);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = NULL;
+    }
+    return e;
+}
+
 static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
 {
     *p = NULL;
@@ -139,18 +166,8 @@ static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
             return 0;
         }
     }
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = dev_malloc(ctx, p, bytes);
     if (e != hipSuccess) {
-        /* release cached buffers and retry once */
-        for (int i = 0; i < FS_POOL_SLOTS; i++)
-            if (ctx->pool[i].ptr) {
-                hipFree(ctx->pool[i].ptr);
-                ctx->pool[i].ptr = NULL;
-            }
-        e = hipMalloc(p, bytes);
-    }
-    if (e != hipSuccess) {
-        *p = NULL;
         set_error(ctx, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
         return 1;
     }
@@ -357,9 +374,7 @@ void futhark_context_free(struct futhark_context *ctx)
         terrain_unref(ctx, ctx->empty_terrain);
     if (ctx->empty_shade)
         shade_unref(ctx, ctx->empty_shade);
-    for (int i = 0; i < FS_POOL_SLOTS; i++)
-        if (ctx->pool[i].ptr)
-            hipFree(ctx->pool[i].ptr);
+    pool_clear(ctx);
     if (ctx->prof_ev) {
         for (int i = 0; i < 2 * FS_PROF_MAX; i++)
             if (ctx->prof_ev[i])
@@ -399,11 +414,7 @@ int futhark_context_clear_caches(struct futhark_context *ctx)
     if (!ctx)
         return 1;
     HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < FS_POOL_SLOTS; i++)
-        if (ctx->pool[i].ptr) {
-            hipFree(ctx->pool[i].ptr);
-            ctx->pool[i].ptr = NULL;
-        }
+    pool_clear(ctx);
     return 0;
 }
 
@@ -1595,7 +1606,7 @@ int fsx_render2(struct futhark_context *ctx, const struct fsx_map *map,
             HIPCHECK(ctx, hipFree(ctx->d_trig));
         ctx->d_trig = NULL;
         ctx->trig_cap = 0;
-        HIPCHECK(ctx, hipMalloc((void **)&ctx->d_trig, sizeof(float) * need));
+        HIPCHECK(ctx, dev_malloc(ctx, (void **)&ctx->d_trig, sizeof(float) * need));
         ctx->trig_cap = need;
     }
     float *h = (float *)malloc(sizeof(float) * need);
@@ -1729,9 +1740,9 @@ int fsx_map_shade_factor(struct futhark_context *ctx, const struct fsx_map *map,
 static int partials(struct futhark_context *ctx, double **p)
 {
     if (!ctx->d_partials) {
-        hipError_t e = hipMalloc((void **)&ctx->d_partials, sizeof(double) * FSK_PARTIALS);
+        hipError_t e =
+            dev_malloc(ctx, (void **)&ctx->d_partials, sizeof(double) * FSK_PARTIALS);
         if (e != hipSuccess) {
-            ctx->d_partials = NULL;
             set_error(ctx, "scratch allocation failed: %s", hipGetErrorString(e));
             return 1;
         }
@@ -2188,7 +2199,7 @@ int fsx_batch_new(struct futhark_context *ctx, const struct fsx_map *const *maps
         grid = (int32_t)n_items;
     int rc = 1;
     if (hitems && hipSetDevice(ctx->device) == hipSuccess &&
-        hipMalloc(&bt->d_mem, vb + ib + mb + cpad + cb) == hipSuccess) {
+        dev_malloc(ctx, &bt->d_mem, vb + ib + mb + cpad + cb) == hipSuccess) {
         deal_items(hv, n_views, hitems, hitems + n_items);
         fsk_batch_counters_init((uint32_t *)((char *)hitems + ib + mb + cpad), grid, FS_QUEUES);
         char *base = (char *)bt->d_mem;

@@ -67,6 +67,7 @@ def contexts(lib):
     _set(lib, "stub_limit", 2 ** 63 - 1)
     for c in made:
         lib.futhark_context_free(c.ptr)
+    lib.hipGetLastError()
 
 
 def _readers(lib, c, m):
@@ -129,3 +130,62 @@ def test_a_state_rendered_elsewhere_keeps_its_buffers_out_of_the_pool(lib, conte
     lib.futhark_free_u32_2d(a.ptr, col)
     lib.futhark_free_i32_2d(a.ptr, hts)
     lib.futhark_free_u32_2d(b.ptr, out)
+
+
+def _calls_that_allocate(lib, c, m):
+    """Calls whose first use, or every use, takes device memory of its own."""
+    view, buf = VIEW.to_c(), ctypes.create_string_buffer(4096)
+    wide = View(**{**VIEW.__dict__, "w": 4096, "h": 1}).to_c()
+    maps, off, out = (ctypes.c_void_p * 1)(m), ctypes.c_int64(0), ctypes.c_void_p()
+    aligned = ctypes.c_void_p((ctypes.addressof(buf) + 63) & ~63)
+
+    def batch():
+        rc = lib.fsx_batch_new(c.ptr, maps, 1, ctypes.byref(view), 1, aligned,
+                               ctypes.addressof(off), ctypes.byref(out))
+        if rc == 0:
+            lib.fsx_batch_free(c.ptr, out)
+        return rc
+
+    def load():
+        p, a = ctypes.c_void_p(), np.zeros((40, 40), np.uint32)
+        rc = lib.fsx_map_new(c.ptr, ctypes.byref(p), a.ctypes.data, a.ctypes.data, 40, 40, 8, 40,
+                             0.1, 0.1)
+        if rc == 0:
+            c.free(p.value)
+        return rc
+
+    def array():
+        a = lib.futhark_new_u32_2d(c.ptr, buf, 8, 8)
+        if a:
+            lib.futhark_free_u32_2d(c.ptr, a)
+        return int(not a)
+
+    return {"batch": batch, "load": load, "array": array,
+            "loss": lambda: lib.fsx_l2_loss(c.ptr, aligned, aligned, 16, 0, aligned, aligned),
+            "render2": lambda: lib.fsx_render2(c.ptr, m, ctypes.byref(wide), aligned, 0)}
+
+
+@pytest.mark.parametrize("call", ["batch", "load", "array", "loss", "render2"])
+def test_pooled_buffers_are_given_back_where_memory_runs_out(lib, contexts, call):
+    """A call that fits once the pool is given back succeeds, whichever way it
+    allocates, and so does the next launch; one that does not fit fails alone."""
+    c = contexts[0]
+    m = c.map()
+    call = _calls_that_allocate(lib, c, m)[call]
+    c.free(c.map(side=256))                      # 1.9 MB into the pool
+    _set(lib, "stub_limit", _get(lib, "stub_live") + 16)
+    assert call() == 0
+    assert _readers(lib, c, m)["render"]() == 0
+    assert lib.futhark_context_clear_caches(c.ptr) == 0
+
+
+@pytest.mark.parametrize("call", ["batch", "load", "array", "loss", "render2"])
+def test_a_refused_allocation_leaves_no_error_behind(lib, contexts, call):
+    c = contexts[0]
+    m = c.map()
+    call = _calls_that_allocate(lib, c, m)[call]
+    lib.futhark_context_clear_caches(c.ptr)
+    _set(lib, "stub_limit", _get(lib, "stub_live") + 16)
+    assert call() == 1
+    assert _readers(lib, c, m)["render"]() == 0
+    assert lib.futhark_context_sync(c.ptr) == 0
