@@ -242,7 +242,19 @@ def planes_of(color):
 
 
 COLOUR_UNIT = 255.0   # a colour-map channel step (u8) in plane units
-FIT_VISIBLE_SHARE = 0.125   # of the device's memory, for the views' visible slices in fit()
+FIT_VISIBLE_SHARE = 0.125   # of the free memory, for the views' visible slices in fit()
+
+
+def _visible_slices(view, held):
+    """A buffer for a view's visible slices; where memory runs out, those
+    that fit() holds are given up first."""
+    try:
+        return torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
+    except torch.cuda.OutOfMemoryError:
+        if not held:
+            raise
+        held.clear()
+    return torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
 
 
 def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None):
@@ -257,8 +269,9 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     clamps the planes back to [0, 1], the domain of the relaxation.
     Visibility does not depend on the planes: each view's visible slices are
     rendered in the first step and kept for the later ones, as far as they
-    take no more than FIT_VISIBLE_SHARE of the device's memory (an entry of
-    views that on_step changes is rendered anew).
+    take no more than FIT_VISIBLE_SHARE of the memory that is free when fit()
+    starts, on the device and in torch's cache (an entry of views that on_step
+    changes is rendered anew).
     Returns the per-step losses (a CUDA tensor, read once at the end)."""
     planes.requires_grad_(False)
     step_lr = lr / COLOUR_UNIT
@@ -267,7 +280,10 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
     v = torch.empty_like(planes)      # the first step writes both moments
     gsky = torch.zeros(1, dtype=torch.float32, device="cuda")
     held = {}                 # view number -> (view's C form, map, its visible slices)
-    room = int(torch.cuda.get_device_properties(planes.device).total_memory * FIT_VISIBLE_SHARE)
+    room = cached = 0
+    if steps > 1:             # a single step has no use for what it rendered
+        room = int(torch.cuda.mem_get_info(planes.device)[0] * FIT_VISIBLE_SHARE)
+        cached = None         # torch's part, asked for once and only if needed
     shared = None             # the visible slices of a view that found no room
     losses = torch.zeros(steps, dtype=torch.float32, device="cuda")
     for it in range(steps):
@@ -285,14 +301,20 @@ def fit(renderer, planes, views, targets, sky_scale, steps, lr=0.5, on_step=None
                 elif have is not None and tuple(have[2].shape) == (view.h, view.w):
                     src = have[2]
                     held[i] = (key, renderer.map, src)
-                elif have is None and 4 * view.h * view.w <= room:
-                    src = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
-                    held[i] = (key, renderer.map, src)
-                    room -= 4 * view.h * view.w
                 else:
-                    if shared is None or tuple(shared.shape) != (view.h, view.w):
-                        shared = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
-                    src = shared
+                    need = 4 * view.h * view.w
+                    if need > room and cached is None:
+                        cached = (torch.cuda.memory_reserved(planes.device)
+                                  - torch.cuda.memory_allocated(planes.device))
+                        room += int(cached * FIT_VISIBLE_SHARE)
+                    if have is None and need <= room:
+                        src = _visible_slices(view, held)
+                        held[i] = (key, renderer.map, src)
+                        room -= need
+                    else:
+                        if shared is None or tuple(shared.shape) != (view.h, view.w):
+                            shared = _visible_slices(view, held)
+                        src = shared
                 # the loop needs neither the image nor its loss gradient
                 renderer.l2_step(planes, sky_scale, view, t, None, src, None, grad, gsky,
                                  losses[it:it + 1], accumulate=i > 0, outputs=False,

@@ -726,3 +726,53 @@ def test_fit_refuses_a_map_closed_meanwhile(ctx):
     r, planes, _, targets = _fit_setup(ctx, [VIEWS[0]])
     with pytest.raises(Exception, match="fsx_render_f32_l2_step"):
         fit(r, planes, [VIEWS[0]], targets, 0.3, steps=2, on_step=lambda it: r.map.close())
+
+
+def _no_memory_free(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (0, 1 << 38))
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda *a: 1 << 20)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda *a: 1 << 20)
+
+
+@pytest.mark.parametrize("steps,full", [(1, False), (3, True)])
+def test_fit_shares_one_buffer_where_it_keeps_none(ctx, steps, full, monkeypatch):
+    """With no memory free, or one step only, views of one size share a
+    buffer of visible slices."""
+    import dataclasses
+    views = [dataclasses.replace(VIEWS[0], angle=a) for a in (0.4, 1.4, 2.4)]
+    r, planes, _, targets = _fit_setup(ctx, views)
+    if full:
+        _no_memory_free(monkeypatch)
+    fit(r, planes, views, targets, 0.3, steps=steps)
+    assert len(set(r.at)) == 1 and not any(r.known)
+
+
+def test_fit_counts_the_memory_torch_holds_unused(ctx, monkeypatch):
+    r, planes, _, targets = _fit_setup(ctx, [VIEWS[0]])
+    _no_memory_free(monkeypatch)
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda *a: 1 << 30)
+    fit(r, planes, [VIEWS[0]], targets, 0.3, steps=2)
+    assert r.known == [False, True]
+
+
+def test_fit_gives_up_what_it_holds_where_memory_runs_out(ctx, monkeypatch):
+    """An allocation that fails while views' visible slices are held is
+    repeated without them, and the fit goes on to the same result."""
+    import dataclasses
+
+    from futspace_amd import diff
+    views = [dataclasses.replace(VIEWS[0], angle=a) for a in (0.4, 1.4, 2.4)]
+    r, planes, _, targets = _fit_setup(ctx, views)
+    want = fit(r, planes.clone(), views, targets, 0.3, steps=3).cpu().numpy()
+    empty, made = torch.empty, []
+
+    def short(*args, **kw):
+        if kw.get("dtype") == torch.int32:
+            made.append(args[0])
+            if len(made) == 3:
+                raise torch.cuda.OutOfMemoryError("no room for a third buffer")
+        return empty(*args, **kw)
+
+    monkeypatch.setattr(diff.torch, "empty", short)
+    got = fit(r, planes.clone(), views, targets, 0.3, steps=3).cpu().numpy()
+    assert len(made) > 3 and np.allclose(got, want, rtol=1e-5, atol=0.0)
