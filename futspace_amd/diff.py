@@ -148,8 +148,11 @@ class DiffRenderer:
             img = gimg = None
         elif img is None:
             img = torch.empty((3, view.h, view.w), dtype=torch.float32, device="cuda")
-        if visible and (src is None or tuple(src.shape) != (view.h, view.w)):
-            raise ValueError("visible=True needs the view's src")
+        if visible and (src is None or tuple(src.shape) != (view.h, view.w)
+                        or src.dtype not in (torch.int32, torch.uint32) or not src.is_cuda
+                        or not src.is_contiguous()):
+            raise ValueError("visible=True needs the view's src: a contiguous CUDA int32 tensor "
+                             f"of shape ({view.h}, {view.w})")
         if src is None:
             src = torch.empty((view.h, view.w), dtype=torch.int32, device="cuda")
         if outputs and gimg is None:

@@ -776,3 +776,22 @@ def test_fit_gives_up_what_it_holds_where_memory_runs_out(ctx, monkeypatch):
     monkeypatch.setattr(diff.torch, "empty", short)
     got = fit(r, planes.clone(), views, targets, 0.3, steps=3).cpu().numpy()
     assert len(made) > 3 and np.allclose(got, want, rtol=1e-5, atol=0.0)
+
+
+def test_given_visibility_is_a_dense_int32_image_on_the_device(ctx):
+    """With visible=True src is read: what is not laid out as the kernel reads
+    it is refused before anything is queued."""
+    r, col, _, _ = _setup(ctx)
+    tp, v = torch.from_numpy(planes_of(col)).cuda(), VIEWS[0]
+    _, src = r.forward_raw(tp, 0.3, v)
+    target = torch.zeros((3, v.h, v.w), device="cuda")
+    torch.cuda.synchronize()
+    wide = torch.zeros((v.h, 2 * v.w), dtype=torch.int32, device="cuda")
+    row = torch.zeros((1, v.w), dtype=torch.int32, device="cuda")
+    for bad in (src.long(), src.short(), src.float(), src.cpu(), wide[:, ::2], wide[:, :v.w],
+                row.expand(v.h, v.w), src.t().contiguous().t()):
+        assert tuple(bad.shape) == (v.h, v.w)
+        with pytest.raises(ValueError):
+            r.l2_step(tp, 0.3, v, target, src=bad, visible=True)
+    r.l2_step(tp, 0.3, v, target, src=src, visible=True)
+    torch.cuda.synchronize()
