@@ -40,9 +40,22 @@ struct fs_shade;
 
 #define FS_POOL_SLOTS 16
 /* Bytes of freed map buffers that a context keeps: the maps of a few loads
- * or re-shadings (a 2048^2 map and its shade take 63 MB).  Given back when
- * the context or its caches are freed, or an allocation fails. */
+ * or re-shadings (a 2048^2 map with a 1024^2 shade takes 79 MB; the colour
+ * quads of one 4096^2 shade fill it, so that loads of that size reuse little).
+ * Given back when the context or its caches are freed, or an allocation
+ * fails. */
 #define FS_POOL_MAP_BYTES ((size_t)256 << 20)
+
+/* Freed buffers kept for reuse, by size (stream order keeps reuse safe:
+ * every later writer runs after every earlier reader on the one stream). */
+struct fs_pool {
+    struct {
+        void *ptr;
+        size_t bytes;
+        uint64_t age;         /* clock when it was freed */
+    } slot[FS_POOL_SLOTS];
+    uint64_t clock;
+};
 
 struct futhark_context {
     int device;
@@ -51,13 +64,9 @@ struct futhark_context {
     hipStream_t own_stream;
     hipStream_t stream;
     char *error;
-    struct {
-        void *ptr;
-        size_t bytes;
-        uint64_t age;         /* pool_clock when it was freed */
-        int map;              /* a map buffer, counted against FS_POOL_MAP_BYTES */
-    } pool[FS_POOL_SLOTS];    /* freed buffers kept for reuse */
-    uint64_t pool_clock;
+    /* output arrays and map buffers do not compete for slots: a load between
+     * two frames of a render loop must not cost the loop its buffer */
+    struct fs_pool outputs, maps;
     struct fs_terrain *empty_terrain;
     struct fs_shade *empty_shade;
     fsk_tuning tune;          /* render kernel shape (0 = automatic) */
@@ -127,13 +136,46 @@ static void set_error(struct futhark_context *ctx, const char *fmt, ...)
         }                                                                           \
     } while (0)
 
-static void pool_clear(struct futhark_context *ctx)
+static void pool_clear(struct fs_pool *pool)
 {
     for (int i = 0; i < FS_POOL_SLOTS; i++)
-        if (ctx->pool[i].ptr) {
-            hipFree(ctx->pool[i].ptr);
-            ctx->pool[i].ptr = NULL;
+        if (pool->slot[i].ptr) {
+            hipFree(pool->slot[i].ptr);
+            pool->slot[i].ptr = NULL;
         }
+}
+
+static void *pool_take(struct fs_pool *pool, size_t bytes)
+{
+    for (int i = 0; i < FS_POOL_SLOTS; i++)
+        if (pool->slot[i].ptr && pool->slot[i].bytes == bytes) {
+            void *p = pool->slot[i].ptr;
+            pool->slot[i].ptr = NULL;
+            return p;
+        }
+    return NULL;
+}
+
+/* Keeps p; 0 if there is no slot for it. */
+static int pool_put(struct fs_pool *pool, void *p, size_t bytes)
+{
+    for (int i = 0; i < FS_POOL_SLOTS; i++)
+        if (!pool->slot[i].ptr) {
+            pool->slot[i].ptr = p;
+            pool->slot[i].bytes = bytes;
+            pool->slot[i].age = pool->clock++;
+            return 1;
+        }
+    return 0;
+}
+
+static size_t pool_bytes(const struct fs_pool *pool)
+{
+    size_t kept = 0;
+    for (int i = 0; i < FS_POOL_SLOTS; i++)
+        if (pool->slot[i].ptr)
+            kept += pool->slot[i].bytes;
+    return kept;
 }
 
 /* hipMalloc that gives the pooled buffers back and tries once more when
@@ -144,7 +186,8 @@ static hipError_t dev_malloc(struct futhark_context *ctx, void **p, size_t bytes
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        pool_clear(ctx);
+        pool_clear(&ctx->outputs);
+        pool_clear(&ctx->maps);
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
@@ -154,18 +197,13 @@ static hipError_t dev_malloc(struct futhark_context *ctx, void **p, size_t bytes
     return e;
 }
 
-static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
+static int pool_alloc(struct futhark_context *ctx, struct fs_pool *pool, void **p, size_t bytes)
 {
-    *p = NULL;
     if (bytes == 0)
         bytes = 4;
-    for (int i = 0; i < FS_POOL_SLOTS; i++) {
-        if (ctx->pool[i].ptr && ctx->pool[i].bytes == bytes) {
-            *p = ctx->pool[i].ptr;
-            ctx->pool[i].ptr = NULL;
-            return 0;
-        }
-    }
+    *p = pool_take(pool, bytes);
+    if (*p)
+        return 0;
     hipError_t e = dev_malloc(ctx, p, bytes);
     if (e != hipSuccess) {
         set_error(ctx, "device allocation of %zu bytes failed: %s", bytes, hipGetErrorString(e));
@@ -174,50 +212,31 @@ static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
     return 0;
 }
 
-/* Free the buffer that has been in the pool longest (of map buffers, if
- * map_only). */
-static void pool_evict(struct futhark_context *ctx, int map_only)
+static void wait_and_free(struct futhark_context *ctx, void *p)
 {
-    int old = -1;
-    for (int i = 0; i < FS_POOL_SLOTS; i++)
-        if (ctx->pool[i].ptr && (!map_only || ctx->pool[i].map) &&
-            (old < 0 || ctx->pool[i].age < ctx->pool[old].age))
-            old = i;
-    if (old < 0)
-        return;
     hipStreamSynchronize(ctx->stream);
-    hipFree(ctx->pool[old].ptr);
-    ctx->pool[old].ptr = NULL;
+    hipFree(p);
 }
 
-/* Return a buffer to the reuse pool, in place of the one longest there if
- * it is full (stream order keeps reuse safe: every later writer runs after
- * every earlier reader on the one stream). */
-static void pool_put(struct futhark_context *ctx, void *p, size_t bytes, int map)
+static int dev_alloc(struct futhark_context *ctx, void **p, size_t bytes)
 {
-    for (int pass = 0; pass < 2; pass++) {
-        for (int i = 0; i < FS_POOL_SLOTS; i++) {
-            if (!ctx->pool[i].ptr) {
-                ctx->pool[i].ptr = p;
-                ctx->pool[i].bytes = bytes;
-                ctx->pool[i].age = ctx->pool_clock++;
-                ctx->pool[i].map = map;
-                return;
-            }
-        }
-        pool_evict(ctx, 0);
-    }
+    return pool_alloc(ctx, &ctx->outputs, p, bytes);
 }
 
 static void dev_release(struct futhark_context *ctx, void *p, size_t bytes)
 {
-    if (p)
-        pool_put(ctx, p, bytes ? bytes : 4, 0);
+    if (p && !pool_put(&ctx->outputs, p, bytes ? bytes : 4))
+        wait_and_free(ctx, p);
 }
 
-/* dev_release of a map buffer: at most FS_POOL_MAP_BYTES of them are kept.
- * A buffer that other streams than the context's may be reading (not pooled)
- * is freed, which waits for the whole device. */
+static int map_alloc(struct futhark_context *ctx, void **p, size_t bytes)
+{
+    return pool_alloc(ctx, &ctx->maps, p, bytes);
+}
+
+/* At most FS_POOL_MAP_BYTES of map buffers are kept, in place of those
+ * longest there.  A buffer that other streams than the context's may be
+ * reading (not pooled) is freed, which waits for the whole device. */
 static void map_release(struct futhark_context *ctx, void *p, size_t bytes, int pooled)
 {
     if (!p)
@@ -225,20 +244,18 @@ static void map_release(struct futhark_context *ctx, void *p, size_t bytes, int 
     if (bytes == 0)
         bytes = 4;
     if (!pooled || bytes > FS_POOL_MAP_BYTES) {
-        hipStreamSynchronize(ctx->stream);
-        hipFree(p);
+        wait_and_free(ctx, p);
         return;
     }
-    for (;;) {
-        size_t kept = 0;
+    struct fs_pool *pool = &ctx->maps;
+    while (pool_bytes(pool) + bytes > FS_POOL_MAP_BYTES || !pool_put(pool, p, bytes)) {
+        int old = -1;
         for (int i = 0; i < FS_POOL_SLOTS; i++)
-            if (ctx->pool[i].ptr && ctx->pool[i].map)
-                kept += ctx->pool[i].bytes;
-        if (kept + bytes <= FS_POOL_MAP_BYTES)
-            break;
-        pool_evict(ctx, 1);
+            if (pool->slot[i].ptr && (old < 0 || pool->slot[i].age < pool->slot[old].age))
+                old = i;
+        wait_and_free(ctx, pool->slot[old].ptr);
+        pool->slot[old].ptr = NULL;
     }
-    pool_put(ctx, p, bytes, 1);
 }
 
 struct futhark_context_config *futhark_context_config_new(void)
@@ -374,7 +391,8 @@ void futhark_context_free(struct futhark_context *ctx)
         terrain_unref(ctx, ctx->empty_terrain);
     if (ctx->empty_shade)
         shade_unref(ctx, ctx->empty_shade);
-    pool_clear(ctx);
+    pool_clear(&ctx->outputs);
+    pool_clear(&ctx->maps);
     if (ctx->prof_ev) {
         for (int i = 0; i < 2 * FS_PROF_MAX; i++)
             if (ctx->prof_ev[i])
@@ -414,7 +432,8 @@ int futhark_context_clear_caches(struct futhark_context *ctx)
     if (!ctx)
         return 1;
     HIPCHECK(ctx, hipStreamSynchronize(ctx->stream));
-    pool_clear(ctx);
+    pool_clear(&ctx->outputs);
+    pool_clear(&ctx->maps);
     return 0;
 }
 
@@ -802,9 +821,9 @@ static struct fs_terrain *terrain_new(struct futhark_context *ctx, const uint32_
     t->cols = cols;
     t->hbits = hbits;
     const size_t n = terrain_texels(t), hpbytes = terrain_hp_bytes(t);
-    int failed = dev_alloc(ctx, &t->d_hq, terrain_hq_bytes(t)) ||
-                 dev_alloc(ctx, (void **)&t->d_hp, hpbytes + FSK_HMAX_PARTS * 4) ||
-                 dev_alloc(ctx, (void **)&t->d_color, n * 4);
+    int failed = map_alloc(ctx, &t->d_hq, terrain_hq_bytes(t)) ||
+                 map_alloc(ctx, (void **)&t->d_hp, hpbytes + FSK_HMAX_PARTS * 4) ||
+                 map_alloc(ctx, (void **)&t->d_color, n * 4);
     if (!failed && host_heights) {
         t->h_alt = (uint16_t *)malloc(n ? n * 2 : 2);
         failed = !t->h_alt;
@@ -862,7 +881,7 @@ static struct fs_shade *shade_new(struct futhark_context *ctx, struct fs_terrain
     s->rows = size;
     s->cols = size;
     size_t n = (size_t)size * (size_t)size;
-    if (dev_alloc(ctx, (void **)&s->d_shaded, n * 4) || dev_alloc(ctx, &s->d_cq, n * 16)) {
+    if (map_alloc(ctx, (void **)&s->d_shaded, n * 4) || map_alloc(ctx, &s->d_cq, n * 16)) {
         set_error(ctx, "shade allocation (%d^2) failed", size);
         shade_unref(ctx, s);
         return NULL;
@@ -909,7 +928,7 @@ static struct fs_shade *shade_zero(struct futhark_context *ctx)
     s->readers.owner = ctx->id;
     s->rows = 2;
     s->cols = 1;
-    if (dev_alloc(ctx, (void **)&s->d_shaded, 8) || dev_alloc(ctx, &s->d_cq, 32) ||
+    if (map_alloc(ctx, (void **)&s->d_shaded, 8) || map_alloc(ctx, &s->d_cq, 32) ||
         hipMemsetAsync(s->d_shaded, 0, 8, ctx->stream) != hipSuccess ||
         hipMemsetAsync(s->d_cq, 0, 32, ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess) {
@@ -1498,7 +1517,7 @@ int fsx_map_new(struct futhark_context *ctx, struct fsx_map **out,
      * buffer of their own, which the quads are made from */
     const size_t bytes = (size_t)(rows * cols) * 4;
     int32_t *d_alt = NULL;
-    if (hipSetDevice(ctx->device) != hipSuccess || dev_alloc(ctx, (void **)&d_alt, bytes))
+    if (hipSetDevice(ctx->device) != hipSuccess || map_alloc(ctx, (void **)&d_alt, bytes))
         return 1;
     hipError_t e = hipMemcpyAsync(d_alt, height, bytes, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess)

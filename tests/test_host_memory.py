@@ -189,3 +189,56 @@ def test_a_refused_allocation_leaves_no_error_behind(lib, contexts, call):
     assert call() == 1
     assert _readers(lib, c, m)["render"]() == 0
     assert lib.futhark_context_sync(c.ptr) == 0
+
+
+def _array(lib, c, rows):
+    a = lib.futhark_new_u32_2d(c.ptr, None, rows, 4)
+    assert a
+    lib.futhark_free_u32_2d(c.ptr, a)
+
+
+def test_map_loads_leave_a_render_loop_its_buffer(lib, contexts):
+    """More freed map buffers than the pool has slots, and one of the frame's
+    own size, take nothing from the output arrays."""
+    c = contexts[0]
+    lib.futhark_context_clear_caches(c.ptr)
+    _array(lib, c, 16 * 16)
+    for side in (64, 65, 66, 67, 16):
+        c.free(c.map(side=side))
+    kept = c.map(side=16)
+    mallocs = _get(lib, "stub_mallocs")
+    _array(lib, c, 16 * 16)
+    assert _get(lib, "stub_mallocs") == mallocs
+    c.free(kept)
+
+
+def test_output_arrays_of_many_sizes_keep_their_slots(lib, contexts):
+    """Frames of one size more than the pool has slots, one after the other:
+    all but one find their buffer again."""
+    c = contexts[0]
+    lib.futhark_context_clear_caches(c.ptr)
+    for _ in range(2):
+        mallocs = _get(lib, "stub_mallocs")
+        for rows in range(1, 18):
+            _array(lib, c, rows)
+    assert _get(lib, "stub_mallocs") - mallocs == 1
+
+
+def test_map_buffers_are_reused_up_to_the_bound(lib, contexts):
+    """A load after a load of its size allocates nothing; what is kept stays
+    within 256 MiB, the newest first, and goes with the caches."""
+    c = contexts[0]
+    lib.futhark_context_clear_caches(c.ptr)
+    before = _get(lib, "stub_live")
+    for side in (2048, 1024, 1024):
+        mallocs = _get(lib, "stub_mallocs")
+        c.free(c.map(side=side))
+    assert _get(lib, "stub_mallocs") == mallocs
+    for side in range(1400, 1410):
+        c.free(c.map(side=side))
+        assert _get(lib, "stub_live") - before <= 256 << 20
+    mallocs = _get(lib, "stub_mallocs")
+    c.free(c.map(side=1409))
+    assert _get(lib, "stub_mallocs") == mallocs
+    lib.futhark_context_clear_caches(c.ptr)
+    assert _get(lib, "stub_live") == before
