@@ -201,13 +201,14 @@ __device__ __forceinline__ uint32_t argb_mix(float m1, uint32_t c1, float m2, ui
 typedef uint32_t fs_u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t fs_u32x4 __attribute__((ext_vector_type(4)));
 
-template <int HBITS, bool HP2, bool TAME = false>
+template <int HBITS, bool HP2, int TAME = 0>
 __device__ __forceinline__ uint2 height_quad(const fsk_map &m, float x, float y)
 {
-    /* TAME: |x|, |y| < 2^22 (2^21 where the sides are no powers of two), so
-     * floor converts exactly without a clamp */
+    /* TAME: the frame's level (fsk_tame_level).  From FSK_TAME on |x| and |y|
+     * are below 2^22, so that floor converts exactly without a clamp; at
+     * FSK_TAME_MOD they are below 2^21 and wrap by reciprocals. */
     int32_t ix, iy;
-    if (TAME && !HP2) {
+    if (TAME == FSK_TAME_MOD && !HP2) {
         ix = wrap_tame(floorf(x), m.hcols, m.rhcols);
         iy = wrap_tame(floorf(y), m.hrows, m.rhrows);
     } else {
@@ -217,8 +218,8 @@ __device__ __forceinline__ uint2 height_quad(const fsk_map &m, float x, float y)
     /* maps are at most 2^28 texels (host-checked), so 32-bit offsets; the
      * wrapped index is always inside the map, whatever x and y are */
     uint32_t t = HP2 ? ((uint32_t)iy << __builtin_ctz((uint32_t)m.hcols)) + (uint32_t)ix
-                 : TAME ? __umul24((uint32_t)iy, (uint32_t)m.hcols) + (uint32_t)ix
-                        : (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
+                 : TAME == FSK_TAME_MOD ? __umul24((uint32_t)iy, (uint32_t)m.hcols) + (uint32_t)ix
+                                        : (uint32_t)iy * (uint32_t)m.hcols + (uint32_t)ix;
     const FS_GLOBAL char *hq = (const FS_GLOBAL char *)m.hq;
     if (HBITS == 8)
         return make_uint2(*(const FS_GLOBAL uint32_t *)(hq + t * 4u), 0u);
@@ -748,13 +749,13 @@ __device__ __forceinline__ uint32_t painted_value(uint32_t v, bool sky_cell, uin
 /* Texel index of the stateless program's sample at (x, y): i32.f32 of
  * each coordinate (x86 truncation), floor-mod by the map size.  TAME as in
  * height_quad. */
-template <bool P2, bool TAME = false>
+template <bool P2, int TAME = 0>
 __device__ __forceinline__ uint32_t nearest_index(const fsk_map &m, float x, float y)
 {
     if (TAME && P2)
         return (uint32_t)wrap<P2>((int32_t)y, m.hrows) * (uint32_t)m.hcols +
                (uint32_t)wrap<P2>((int32_t)x, m.hcols);
-    if (TAME)
+    if (TAME == FSK_TAME_MOD)
         return __umul24((uint32_t)wrap_tame(truncf(y), m.hrows, m.rhrows), (uint32_t)m.hcols) +
                (uint32_t)wrap_tame(truncf(x), m.hcols, m.rhcols);
     int32_t ix = wrap<P2>(i32_f32_x86(x), m.hcols);
@@ -921,7 +922,7 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
         const float4 *tlg = tl + g;
         const float *tzg = tz + g;
         auto project = [&](auto tame_tag, auto full_tag) {
-            constexpr bool TAME = decltype(tame_tag)::value;
+            constexpr int TAME = decltype(tame_tag)::value;
             constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
             for (int j0 = 0; j0 < KR; j0 += GATHER) {
@@ -972,13 +973,23 @@ __device__ __forceinline__ void render_tile(const fsk_map &m, const fsk_frame &f
                 }
             }
         };
-        const bool tame = f.tame >= (HP2 ? FSK_TAME : FSK_TAME_MOD);
-        if (tame && kr == KR)
-            project(std::true_type{}, std::true_type{});
-        else if (tame)
-            project(std::true_type{}, std::false_type{});
+        /* middle: sides that are no powers of two at coordinates between 2^21
+         * and 2^22 (or longer than 2^20) wrap by the integer modulo, still
+         * without the x86 casts' clamps (1363 x 767, 1531 slices at x = 3e6:
+         * 18.8 us, 19.5 through the casts; with reciprocals, nearer the
+         * origin, 17.3) */
+        constexpr std::integral_constant<int, HP2 ? FSK_TAME : FSK_TAME_MOD> best{};
+        constexpr std::integral_constant<int, FSK_TAME> middle{};
+        if (f.tame >= best && kr == KR)
+            project(best, std::true_type{});
+        else if (f.tame >= best)
+            project(best, std::false_type{});
+        else if (!HP2 && MODE != kOutNearest && f.tame >= FSK_TAME && kr == KR)
+            project(middle, std::true_type{});
+        else if (!HP2 && MODE != kOutNearest && f.tame >= FSK_TAME)
+            project(middle, std::false_type{});
         else
-            project(std::false_type{}, std::false_type{});
+            project(std::integral_constant<int, 0>{}, std::false_type{});
         /* lanes holding samples past the chunk, past kr (a last gather
          * group kr does not fill) or right of the frame: those samples
          * become row H */

@@ -369,3 +369,34 @@ def test_odd_maps_far_and_near(ctx, rows, cols, shade, bits):
         v = View(x=x, y=y, height=350.0, angle=2.1, horizon=30.0, distance=distance, fov=1.2,
                  sky_color=sky_color(0.1), h=70, w=90, d=0.004, z0=0.5, scale=60.0)
         _check(ctx.render(m, v), O.render_off(v, shaded, alt))
+
+
+@pytest.mark.parametrize("w,h,n", [(90, 70, 1024), (2100, 40, 2048), (20, 7700, 1024), (33, 30, 701)])
+@pytest.mark.parametrize("rows,cols,bits", [(100, 333, 16), (3, 1000, 8)])
+def test_odd_maps_between_the_coordinate_lines(ctx, w, h, n, rows, cols, bits):
+    """Maps whose sides are no powers of two, at coordinates between 2^21 and
+    2^22, where a tame frame wraps by the integer modulo: full and partial
+    depth chunks, bands of rows, frames and the differentiable forward."""
+    import torch
+
+    from futspace_amd.diff import DiffRenderer
+    rng = np.random.default_rng(rows + w)
+    hts = rng.integers(0, 200 if bits == 8 else 900, (rows, cols)).astype(np.int32)
+    col = rng.integers(0, 1 << 24, (rows, cols), dtype=np.uint32) | np.uint32(0xFF000000)
+    m = ctx.map(col, hts, height_bits=bits, shade_size=90)
+    shaded, alt = O.update_map(col, hts, size=90, bits=bits)
+    d, z0 = scene.depth_for(n, 400.0)
+    r = DiffRenderer(ctx, m)
+    planes = rng.random((3, 90, 90), dtype=np.float32)
+    sf = O.shade_factor(O.shadow_counts(alt, O.sun(0.1, 0.1), 90))
+    for x, y in ((3000000.5, -2500000.25), (-4000000.25, 17.6)):
+        v = View(x=x, y=y, height=350.0, angle=2.1, horizon=0.3 * h, distance=400.0, fov=1.2,
+                 sky_color=sky_color(0.1), h=h, w=w, d=d, z0=z0, scale=h / 2.0, n_slices=n)
+        _check(ctx.render(m, v), O.render_painter_mt(v, shaded, alt, 8))
+        img, src = r.forward_raw(torch.from_numpy(planes).cuda(), 0.3, v)
+        torch.cuda.synchronize()
+        want_img, want_src = O.render_f32(v, planes, sf, alt, 0.3)
+        src = src.cpu().numpy()
+        at = np.where(src < 0, -1, src * w + np.arange(w, dtype=np.int32)[None, :])
+        assert np.array_equal(at, want_src)
+        assert np.array_equal(img.cpu().numpy().view(np.uint32), want_img.view(np.uint32))
