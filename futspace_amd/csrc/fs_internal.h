@@ -43,14 +43,16 @@ typedef struct {
 /* FSK_TAME when every sample of the frame stays where the render kernel may
  * skip the out-of-range branches of the x86 casts: finite scalars, slice
  * depths increasing from z0 > 0, every sample coordinate below 2^22 and every
- * projected row below 2^30 in magnitude for any 16-bit height; else 0. */
-#define FSK_TAME 1
-int32_t fsk_frame_tame(const fsk_frame *f);
-/* The same, but FSK_TAME_MOD when besides the coordinates are below 2^21 and max_side, the
+ * projected row below 2^30 in magnitude for any 16-bit height; else 0.
+ * FSK_TAME_MOD when besides the coordinates are below 2^21 and max_side, the
  * longest side of the sampled maps, is at most 2^20, so that sides that are
  * no powers of two may be wrapped by reciprocals. */
+#define FSK_TAME 1
 #define FSK_TAME_MOD 2
 int32_t fsk_tame_level(const fsk_frame *f, int32_t max_side);
+/* The level of a frame over maps of any size: FSK_TAME or 0.  The line that
+ * the tests evaluate by brute force is thereby the one that the launchers use. */
+int32_t fsk_frame_tame(const fsk_frame *f);
 /* A reciprocal of m a little below 1 / m, for such wraps; a map's four. */
 float fsk_wrap_recip(int32_t m);
 void fsk_map_recips(fsk_map *m);

@@ -3540,16 +3540,16 @@ static double tame_extent(const fsk_frame *f)
     return zok && relmax < 1073741824.0 ? std::max(xmax, ymax) : INFINITY;
 }
 
-int32_t fsk_frame_tame(const fsk_frame *f)
-{
-    return tame_extent(f) < 4194304.0 ? FSK_TAME : 0;
-}
-
 int32_t fsk_tame_level(const fsk_frame *f, int32_t max_side)
 {
     const double extent = tame_extent(f);
     return extent < 2097152.0 && max_side <= 1 << 20 ? FSK_TAME_MOD
            : extent < 4194304.0 ? FSK_TAME : 0;
+}
+
+int32_t fsk_frame_tame(const fsk_frame *f)
+{
+    return fsk_tame_level(f, INT32_MAX);
 }
 
 int32_t fsk_render_max_rows(void)
