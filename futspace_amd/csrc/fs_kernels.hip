@@ -3470,7 +3470,6 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
         return hipSuccess;
     Render2Args a;
     a.m = *m;
-    fsk_map_recips(&a.m);
     a.color = d_color;
     a.cs = d_cs;
     a.sn = d_sn;
