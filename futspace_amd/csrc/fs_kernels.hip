@@ -2100,7 +2100,15 @@ struct BatchArgs {
  * The counters are as fsk_batch_counters_init left them before the first
  * launch; the last workgroup to end leaves them so for the next one, so that
  * no launch has to reset them first.  Every claim of a workgroup has
- * returned before it counts itself as ended. */
+ * returned before it counts itself as ended.
+ *
+ * Launches of one batch that overlap (two contexts, or an eager launch beside
+ * a replay) share the counters: between them they hand out every item, some
+ * of them twice, with the same pixels.  The ended workgroups are counted over
+ * all of them and the count is lowered by a launch's worth, not cleared, so
+ * that none is lost; the last of all to end finds a whole number of launches
+ * and leaves the counters reset.  Atomic stores, since a plain one would
+ * reach memory when its launch ends, maybe over another's claims. */
 __host__ __device__ constexpr uint32_t batch_first_claim(uint32_t grid, uint32_t q, uint32_t nq)
 {
     return (grid + nq - 1u - q) / nq;      /* workgroups that start on queue q */
@@ -2166,10 +2174,12 @@ __global__ __launch_bounds__(NT, WPE) void k_render_batch(BatchArgs b)
     }
     if (threadIdx.x == 0) {
         uint32_t *ended = b.counters + nq * FSK_COUNTER_STRIDE;
-        if (atomicAdd(ended, 1u) == gridDim.x - 1u) {
+        if (atomicAdd(ended, 1u) % gridDim.x == gridDim.x - 1u) {
             for (uint32_t i = 0; i < nq; i++)
-                b.counters[i * FSK_COUNTER_STRIDE] = batch_first_claim(gridDim.x, i, nq);
-            *ended = 0u;
+                __hip_atomic_store(b.counters + i * FSK_COUNTER_STRIDE,
+                                   batch_first_claim(gridDim.x, i, nq), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            atomicSub(ended, gridDim.x);
         }
     }
 }

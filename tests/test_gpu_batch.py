@@ -204,3 +204,45 @@ def test_small_batches_replayed(ctx, widths):
         for v, o, w in zip(views, offs, want):
             assert np.array_equal(got[o:o + v.h * v.w].reshape(v.h, v.w), w)
     b.close()
+
+
+@pytest.mark.parametrize("widths", [(3,), (40, 333, 8), (2048, 900, 17, 512)])
+def test_overlapping_launches_of_one_batch(ctx, widths):
+    """A batch launched on two contexts' streams at once, eager and replayed:
+    the launches share the claim counters, render every view between them, and
+    leave a batch whose next launch alone renders every view again."""
+    from futspace_amd import Context
+    col, hts = scene.scene_maps(31, 128)
+    m = ctx.map(col, hts, shade_size=128)
+    views = [View(x=10.0 * i + 5.3, y=40.6, height=270.0, angle=0.7 * i, horizon=20.0,
+                  distance=400.0, fov=1.2, sky_color=sky_color(0.1), h=24 + i, w=w, d=0.004,
+                  z0=0.5, scale=60.0) for i, w in enumerate(widths)]
+    offs = np.cumsum([0] + [v.h * v.w for v in views]).astype(np.int64)
+    out = torch.empty(int(offs[-1]), dtype=torch.int32, device="cuda")
+    b = ctx.batch([m], views, out, offs[:-1])
+    b.capture()
+    other = Context(device=0)
+
+    def beside():
+        other.check(other.lib.fsx_batch_run(other.ptr, b.ptr), "fsx_batch_run")
+
+    def rendered():
+        ctx.sync()
+        other.sync()
+        flat = out.cpu().numpy().view(np.uint32)
+        _check_views(ctx, {0: m}, views, flat, offs)
+        out.fill_(-1)
+        torch.cuda.synchronize()
+
+    out.fill_(-1)
+    torch.cuda.synchronize()
+    for launches in range(1, 9):
+        for _ in range(launches):
+            b.run()
+            beside()
+            b.replay()
+        rendered()
+        b.run()
+        rendered()
+    other.close()
+    b.close()
