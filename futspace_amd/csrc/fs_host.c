@@ -739,9 +739,10 @@ struct fsx_map {
     int32_t shade_size;
 };
 
-/* ctx is about to queue work that reads t and s (either may be NULL).
- * Copies and batches need no note: the one is waited for, and the other keeps
- * its references until its own memory has been freed. */
+/* ctx is about to queue work that reads t and s (either may be NULL), or that
+ * writes a new s, as every replay of a captured shading pass does.  Copies and
+ * batches need no note: the one is waited for, and the other keeps its
+ * references until its own memory has been freed. */
 static void note_readers(struct futhark_context *ctx, struct fs_terrain *t, struct fs_shade *s)
 {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -887,7 +888,7 @@ static struct fs_shade *shade_new(struct futhark_context *ctx, struct fs_terrain
         return NULL;
     }
     sun_vector(sun_height, sun_ang, s->sun);
-    note_readers(ctx, t, NULL);
+    note_readers(ctx, t, s);
     hipError_t e = (hipError_t)fsk_shade(t->d_hp, t->d_hmax, t->rows, t->cols, t->d_color, s->sun, size,
                               s->d_shaded, ctx->stream);
     if (e == hipSuccess)

@@ -132,6 +132,32 @@ def test_a_state_rendered_elsewhere_keeps_its_buffers_out_of_the_pool(lib, conte
     lib.futhark_free_u32_2d(b.ptr, out)
 
 
+def test_a_shade_that_a_captured_graph_writes_is_freed_and_not_reused(lib, contexts):
+    """A step under capture shades into a buffer that every replay of the graph
+    writes again."""
+    a = contexts[0]
+    maps = np.zeros((SIDE, SIDE), np.uint32)
+    col = lib.futhark_new_u32_2d(a.ptr, maps.ctypes.data, SIDE, SIDE)
+    hts = lib.futhark_new_i32_2d(a.ptr, maps.ctypes.data, SIDE, SIDE)
+    states = [ctypes.c_void_p() for _ in range(4)]
+    init, loaded, keyed, stepped = states
+    assert lib.futhark_entry_init(a.ptr, ctypes.byref(init), 0) == 0
+    assert lib.futhark_entry_update_map(a.ptr, ctypes.byref(loaded), ctypes.c_void_p(col),
+                                        ctypes.c_void_p(hts), init) == 0
+    assert lib.futhark_entry_key(a.ptr, ctypes.byref(keyed), 0, ord("u"), loaded) == 0
+    _set(lib, "stub_capturing", 1, ctypes.c_int)
+    assert lib.futhark_entry_step(a.ptr, ctypes.byref(stepped), 0.016, keyed) == 0
+    _set(lib, "stub_capturing", 0, ctypes.c_int)
+    frees = _get(lib, "stub_frees")
+    for s in states:
+        lib.futhark_free_opaque_state(a.ptr, s)
+    # the heights and colours that the graph reads, and the shade it writes;
+    # the shade of the loaded state is read by nothing and kept
+    assert _get(lib, "stub_frees") - frees == MAP_BUFFERS
+    lib.futhark_free_u32_2d(a.ptr, col)
+    lib.futhark_free_i32_2d(a.ptr, hts)
+
+
 def _calls_that_allocate(lib, c, m):
     """Calls whose first use, or every use, takes device memory of its own."""
     view, buf = VIEW.to_c(), ctypes.create_string_buffer(4096)
