@@ -2596,14 +2596,18 @@ constexpr int kGradRowsLow = 2, kGradRowsTall = 4;
  * (1280 x 720: 45 us with 1408 slots and four workgroups, 52 with 1024 and
  * five, 59 with 816 and six).  With 4 rows, in frames whose runs are longer,
  * 944 slots and six workgroups: 92 us, 1024 and five 100 us, 512 and six 91
- * us there and 143 against 119 us over an 8-bit map. */
-constexpr int grad_cap(int rows)
+ * us there and 143 against 119 us over an 8-bit map.  With images to write
+ * (out) a thread also holds its pixels until the run loop has ended, and six
+ * or five workgroups would spill them (110 against 78 us for a 3840 x 2160
+ * step that is nine tenths sky), so 4 rows take four workgroups too, and the
+ * slots that these leave room for. */
+constexpr int grad_cap(int rows, bool out)
 {
-    return rows == kGradRowsLow ? 1408 : 944;
+    return rows == kGradRowsLow || out ? 1408 : 944;
 }
-constexpr int grad_waves(int rows)
+constexpr int grad_waves(int rows, bool out)
 {
-    return rows == kGradRowsLow ? 4 : 6;
+    return rows == kGradRowsLow || out ? 4 : 6;
 }
 constexpr int kGradProbes = 4;
 constexpr int kGradRunLog = 4;               /* texels of a row that hash to adjacent slots */
@@ -2743,15 +2747,20 @@ __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval 
  * here from the target, g = 2 (px - target), with the colour px of each
  * run's sample evaluated where the run starts (the same evaluation as
  * k_diff_color's, so img and g are bit-identical to the separate calls);
- * img and g are written only where the caller asks for them, and each
- * workgroup leaves one partial of the loss, sum (px - target)^2, and one of
- * the sky term.  Otherwise each workgroup leaves one partial of the sky
- * term. */
-template <bool P2, bool TAME, bool FWD, int kGradRows>
-__global__ __launch_bounds__(kGradThreads, grad_waves(kGradRows))
+ * each workgroup leaves one partial of the loss, sum (px - target)^2, and one
+ * of the sky term.  Otherwise each workgroup leaves one partial of the sky
+ * term.
+ *
+ * OUT: img and g are written, where the caller asks for them, after the run
+ * loop, a row of the wave at a time.  Written from within it, by the lanes
+ * whose run was at hand and with six workgroups per CU, a 3840 x 2160 frame
+ * that is all sky took 97 us and one that is two thirds sky 114; now 58 and
+ * 94, of which the two images' 199 MB are 26 and 29. */
+template <bool P2, bool TAME, bool FWD, bool OUT, int kGradRows>
+__global__ __launch_bounds__(kGradThreads, grad_waves(kGradRows, OUT))
 void k_diff_grad(DiffArgs a)
 {
-    constexpr int kGradCap = grad_cap(kGradRows);
+    constexpr int kGradCap = grad_cap(kGradRows, OUT);
     constexpr int kGradBlockRows = (kGradThreads / 64) * kGradRows;
     __shared__ uint32_t keys[kGradCap];
     __shared__ double vals[3 * kGradCap];
@@ -2777,7 +2786,8 @@ void k_diff_grad(DiffArgs a)
     const FS_GLOBAL float *gin = (const FS_GLOBAL float *)(FWD ? a.tgt : a.gimg);
     const FS_GLOBAL int32_t *srcp = (const FS_GLOBAL int32_t *)a.src;
     int32_t src[kGradRows];
-    float g[3][kGradRows];     /* FWD: the target */
+    float g[3][kGradRows];     /* FWD: the target; OUT: g, once that is known */
+    float img[3][kGradRows];   /* OUT: the pixel */
 #pragma unroll
     for (int j = 0; j < kGradRows; j++) {
         /* threads outside the frame load the pixel at its edge */
@@ -2793,20 +2803,21 @@ void k_diff_grad(DiffArgs a)
             src[j] = INT32_MIN;
     __syncthreads();
     /* the sky term cancels where gradients of both signs meet: f64 keeps its
-     * sum as exact as the gradients */
-    double sky_acc = 0.0, loss_sum = 0.0;
+     * sum as exact as the gradients.  Its channels are weighted once per
+     * thread: an all-sky 3840 x 2160 step without outputs 50 -> 32 us */
+    double sky_acc = 0.0, loss_sum = 0.0, sky[3] = {0.0, 0.0, 0.0};
     /* one pixel of the fused step: its loss term and g = 2 (px - target) */
-    auto pixel = [&](int j, uint32_t c, const float px[3], float (&gd)[3]) {
-        const size_t row = (size_t)(r0 + j) * W;
+    auto pixel = [&](int j, const float px[3], float (&gd)[3]) {
 #pragma unroll
         for (int ch = 0; ch < 3; ch++) {
             const float d = px[ch] - g[ch][j];
             gd[ch] = 2.0f * d;
-            if (a.img)
-                ((FS_GLOBAL float *)a.img + ch * fplane + row)[c] = px[ch];
-            if (a.gout)
-                ((FS_GLOBAL float *)a.gout + ch * fplane + row)[c] = gd[ch];
-            loss_sum += (double)d * (double)d;
+            if constexpr (OUT) {
+                img[ch][j] = px[ch];
+                g[ch][j] = gd[ch];
+            }
+            /* the product is exact in f64 */
+            loss_sum = __builtin_fma((double)d, (double)d, loss_sum);
         }
     };
     uint32_t starts = 0u;      /* rows where a run of a visible sample starts */
@@ -2820,18 +2831,17 @@ void k_diff_grad(DiffArgs a)
             if constexpr (FWD) {
                 const float px[3] = {sky_base(0) * a.sky_scale, sky_base(1) * a.sky_scale,
                                      sky_base(2) * a.sky_scale};
-                pixel(j, lcol, px, gd);
+                pixel(j, px, gd);
             }
 #pragma unroll
             for (int ch = 0; ch < 3; ch++)
-                sky_acc += (double)gd[ch] * (double)sky_base(ch);
+                sky[ch] += (double)gd[ch];
         }
     }
+#pragma unroll
+    for (int ch = 0; ch < 3; ch++)
+        sky_acc += sky[ch] * (double)sky_base(ch);
     while (__ballot(starts != 0u)) {
-        /* the loop's own column: the stores' addresses (two images of three
-         * planes, each row) would otherwise be formed before it and spilled */
-        uint32_t c = lcol;
-        asm volatile("" : "+v"(c));
         float val[4][3];
         uint32_t key[4] = {kNoKey, kNoKey, kNoKey, kNoKey};
 #pragma unroll
@@ -2854,7 +2864,7 @@ void k_diff_grad(DiffArgs a)
                 if (in) {
                     float gd[3] = {g[0][j], g[1][j], g[2][j]};
                     if constexpr (FWD)
-                        pixel(j, c, e.px, gd);
+                        pixel(j, e.px, gd);
 #pragma unroll
                     for (int ch = 0; ch < 3; ch++)
                         run[ch] += gd[ch];
@@ -2873,6 +2883,21 @@ void k_diff_grad(DiffArgs a)
             const uint64_t ins = __ballot(inserted);
             if (ins && (threadIdx.x & 63) == 0)
                 atomicAdd(&fill, (uint32_t)__popcll(ins));
+        }
+    }
+    if constexpr (OUT) {
+#pragma unroll
+        for (int j = 0; j < kGradRows; j++) {
+            const size_t row = (size_t)(r0 + j) * W;
+            if (src[j] != INT32_MIN) {
+#pragma unroll
+                for (int ch = 0; ch < 3; ch++) {
+                    if (a.img)
+                        ((FS_GLOBAL float *)a.img + ch * fplane + row)[lcol] = img[ch][j];
+                    if (a.gout)
+                        ((FS_GLOBAL float *)a.gout + ch * fplane + row)[lcol] = g[ch][j];
+                }
+            }
         }
     }
     /* per-workgroup partials, summed in a fixed order by the next launch */
@@ -3121,15 +3146,16 @@ double *g_scratch_ptr[64];   /* device address of `scratch` on each device */
 }  // namespace
 
 /* The adjoint's kernel for a's planes and frame, with `rows` rows per
- * thread. */
-template <bool FWD>
+ * thread; OUT where an image is to be written. */
+template <bool FWD, bool OUT>
 static void launch_diff_grad(const DiffArgs &a, int32_t rows, dim3 grid, hipStream_t s)
 {
+    constexpr int L = kGradRowsLow, T = kGradRowsTall;
     void (*const kern[2][2][2])(DiffArgs) = {
-        {{k_diff_grad<false, false, FWD, kGradRowsLow>, k_diff_grad<false, false, FWD, kGradRowsTall>},
-         {k_diff_grad<false, true, FWD, kGradRowsLow>, k_diff_grad<false, true, FWD, kGradRowsTall>}},
-        {{k_diff_grad<true, false, FWD, kGradRowsLow>, k_diff_grad<true, false, FWD, kGradRowsTall>},
-         {k_diff_grad<true, true, FWD, kGradRowsLow>, k_diff_grad<true, true, FWD, kGradRowsTall>}}};
+        {{k_diff_grad<false, false, FWD, OUT, L>, k_diff_grad<false, false, FWD, OUT, T>},
+         {k_diff_grad<false, true, FWD, OUT, L>, k_diff_grad<false, true, FWD, OUT, T>}},
+        {{k_diff_grad<true, false, FWD, OUT, L>, k_diff_grad<true, false, FWD, OUT, T>},
+         {k_diff_grad<true, true, FWD, OUT, L>, k_diff_grad<true, true, FWD, OUT, T>}}};
     hipLaunchKernelGGL(kern[pow2(a.hc) && pow2(a.wc)][a.f.tame != 0][rows != kGradRowsLow], grid,
                        dim3(kGradThreads), 0, s, a);
 }
@@ -3439,7 +3465,7 @@ int fsk_diff_grad(const fsk_frame *f, const float *d_cp, const float *d_sf, int3
     dim3 grid((f->cols + 63) / 64, (f->rows + br - 1) / br);
     if ((int64_t)grid.x * grid.y > n_partials)
         return hipErrorInvalidValue;
-    launch_diff_grad<false>(a, rows, grid, s);
+    launch_diff_grad<false, false>(a, rows, grid, s);
     hipLaunchKernelGGL(k_sum_partials<double>, dim3(1), dim3(1024), 0, s, d_partials,
                        (int32_t)(grid.x * grid.y), d_gsky, sky_accumulate);
     return hipGetLastError();
@@ -3467,7 +3493,10 @@ int fsk_diff_step_l2(const fsk_frame *f, const float *d_cp, const float *d_sf, i
     const int64_t nb = (int64_t)grid.x * grid.y;
     if (nb > n_partials)
         return hipErrorInvalidValue;
-    launch_diff_grad<true>(a, rows, grid, s);
+    if (d_img || d_g)
+        launch_diff_grad<true, true>(a, rows, grid, s);
+    else
+        launch_diff_grad<true, false>(a, rows, grid, s);
     hipLaunchKernelGGL(k_sum_step, dim3(1), dim3(1024), 0, s, d_loss_part, d_sky_part,
                        (int32_t)nb, d_loss, loss_accumulate, d_gsky, sky_accumulate);
     return hipGetLastError();

@@ -795,3 +795,46 @@ def test_given_visibility_is_a_dense_int32_image_on_the_device(ctx):
             r.l2_step(tp, 0.3, v, target, src=bad, visible=True)
     r.l2_step(tp, 0.3, v, target, src=src, visible=True)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("h,w", [(33, 70), (9, 1), (1537, 2049), (1543, 2050)])
+@pytest.mark.parametrize("which", ["img", "gimg", "both", "none"])
+def test_step_writes_the_images_it_is_given(ctx, h, w, which):
+    """img and dL/dimg, each, both or neither, at both rows per thread and
+    with partial blocks at either edge: bit-equal to the separate calls, in
+    every pixel and in none beyond the frame, and the same loss and gradients
+    whatever is written."""
+    import ctypes
+
+    from futspace_amd.diff import _ptr
+    r, col, _, _ = _setup(ctx)
+    tp = torch.from_numpy(planes_of(col)).cuda()
+    v = View(x=64.3, y=100.7, height=260.0, angle=0.4, horizon=h * 0.6, distance=300.0, fov=1.2,
+             h=h, w=w, d=0.01, z0=0.5, scale=h / 2.0)
+    target = torch.rand((3, h, w), device="cuda",
+                        generator=torch.Generator(device="cuda").manual_seed(h))
+    img, src = r.forward_raw(tp, 0.37, v)
+    gimg, loss = r.l2_loss_grad(img, target)
+    gp, gs = r.vjp_raw(tp, src, gimg, v)
+    n = 3 * h * w
+    out = {k: torch.full((n + 64,), 7.0, device="cuda") for k in ("img", "gimg")}
+    given = {k: _ptr(b) if which in (k, "both") else None for k, b in out.items()}
+    f_gp, f_src = torch.full_like(tp, 9.0), torch.full_like(src, 5)
+    f_gs, f_loss = torch.ones(1, device="cuda"), torch.ones(1, device="cuda")
+    torch.cuda.synchronize()
+    cv = v.to_c()
+    ctx.check(ctx.lib.fsx_render_f32_l2_step(
+        ctx.ptr, r.map.ptr, ctypes.byref(cv), _ptr(tp), _ptr(r.sf), r.hc, r.wc,
+        ctypes.c_float(0.37), _ptr(target), 0, given["img"], _ptr(f_src), given["gimg"],
+        _ptr(f_gp), _ptr(f_gs), _ptr(f_loss)), "fsx_render_f32_l2_step")
+    ctx.sync()
+    for k, want in (("img", img), ("gimg", gimg)):
+        if given[k]:
+            assert torch.equal(out[k][:n], want.reshape(-1)) and bool((out[k][n:] == 7.0).all())
+        else:
+            assert bool((out[k] == 7.0).all())
+    assert torch.equal(f_src, src)
+    assert abs(float(f_loss[0]) - float(loss[0])) <= 1e-5 * float(loss[0])
+    assert _rel_err(f_gp.cpu().numpy(), gp.cpu().numpy()) <= 1e-5
+    sky = float(gimg[:, src < 0].abs().sum())
+    assert abs(float(f_gs[0]) - float(gs[0])) <= 1e-5 * max(sky, 1e-3)
