@@ -1358,15 +1358,23 @@ __global__ __launch_bounds__(NT, WPE) void k_render(RenderArgs a)
  * computed on the host with the C library as `futhark c` does.
  *
  * The terrain height under a ray point does not depend on the pixel's row:
- * a workgroup evaluates the heights of its 64 columns once for its
- * kR2Rows rows, kR2Chunk dists at a time, into LDS.  A pixel then searches
- * them: along dist the line of sight cam_h - dist * vert_ang is monotone,
- * also in f32, so if its lower end over a group of 16 dists is not below the
- * group's highest terrain, none of them hits.  Wave w of the 16 evaluates
- * group w of a chunk, and so has the group's maximum in registers.  800 x 600
- * pixels, 200 steps: 15 us, against 98 us with one thread per pixel marching
- * through the map; bound by the latency of its two phases on 247
- * workgroups. */
+ * a workgroup evaluates the heights of its 64 columns once for its ROWS rows,
+ * a chunk of dists at a time, into LDS.  A pixel then searches them: along
+ * dist the line of sight cam_h - dist * vert_ang is monotone, also in f32, so
+ * if its lower end over a group of dists is not below the group's highest
+ * terrain, none of them hits.  Wave w of the 16 evaluates group w of a chunk,
+ * and so has the group's maximum in registers.  800 x 600 pixels, 200 steps:
+ * 12 us, against 98 us with one thread per pixel marching through the map;
+ * bound by the latency of its two phases on 247 workgroups.
+ *
+ * A camera on the ground, or one that looks steeply down from little above it,
+ * has its hits within a few steps, and the full first chunk of 256 dists took
+ * longer than the marching threads had (3840 x 2160: a call of 159 us, 79 by
+ * the marching threads).  NEAR: where the line of sight of a workgroup's first
+ * row comes below the ground under the camera within a chunk of 16 groups of
+ * kR2Near dists, such a chunk goes first (93 us, with launch_render2's shapes;
+ * 121 without).  Frames of one workgroup per CU go without it: 32 instead of
+ * 34 us for such a camera at 800 x 600, but 40.2 instead of 39.6 for any other. */
 struct Render2Args {
     fsk_map m;
     const uint32_t *color;     /* unshaded colours [hrows][hcols] */
@@ -1389,88 +1397,106 @@ __device__ __forceinline__ uint4 raw_color_quad(const uint32_t *col, int32_t row
     return make_uint4(col[fy * w + fx], col[fy * w + cx], col[cy * w + fx], col[cy * w + cx]);
 }
 
-constexpr int kR2Group = 16;                      /* dists per group */
-constexpr int kR2Chunk = 16 * kR2Group;           /* a group per wave */
-constexpr int kR2Rows = 32;                       /* frame rows per workgroup */
+constexpr int kR2Group = 16;                      /* dists per group, a group per wave */
+constexpr int kR2Near = 4;                        /* in the first chunk of a low camera */
 
-template <int HBITS, bool HP2>
-__global__ __launch_bounds__(1024) void k_render2(Render2Args a)
+template <int HBITS, bool HP2, int ROWS, int WPE, bool NEAR>
+__global__ __launch_bounds__(1024, WPE) void k_render2(Render2Args a)
 {
     __shared__ float sq[256];
-    __shared__ float hs[kR2Chunk][64], top[kR2Chunk / kR2Group][64];
+    __shared__ float hs[16 * kR2Group][64], top[16][64];
     const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int32_t x = blockIdx.x * 64 + lane;
     const float ca = a.cs[min(x, a.cols - 1)], sa = a.sn[min(x, a.cols - 1)];
     fill_square_lut(sq, threadIdx.x);
-    constexpr int PX = kR2Rows / 16;
+    constexpr int PX = ROWS / 16;
     float vert_ang[PX];
     int32_t hit[PX];
 #pragma unroll
     for (int u = 0; u < PX; u++) {
-        const int32_t y = blockIdx.y * kR2Rows + u * 16 + wave;
+        const int32_t y = blockIdx.y * ROWS + u * 16 + wave;
         vert_ang[u] = (a.horizon / 50.0f) + (((float)y / ((float)a.rows - 0.0f)) * (1.5f - 1.0f));
         hit[u] = -1;
     }
-    for (int32_t base = 0; base <= a.n; base += kR2Chunk) {
-        const int32_t d0 = base + wave * kR2Group;
+    /* a chunk of 16 groups of G dists; whether any pixel is left without a hit */
+    auto march = [&](int32_t base, auto group) -> bool {
+        constexpr int G = decltype(group)::value, B = G < 8 ? G : 8;
+        const int32_t d0 = base + wave * G;
         float high = -INFINITY;
 #pragma unroll
-        for (int j0 = 0; j0 < kR2Group; j0 += 8) {
+        for (int j0 = 0; j0 < G; j0 += B) {
             if (d0 + j0 > a.n) {
                 /* past the march: nothing is below the lowest height */
 #pragma unroll
-                for (int j = j0; j < j0 + 8; j++)
-                    hs[wave * kR2Group + j][lane] = -INFINITY;
+                for (int j = j0; j < j0 + B; j++)
+                    hs[wave * G + j][lane] = -INFINITY;
                 continue;
             }
-            float px[8], py[8];
-            uint2 q[8];
+            float px[B], py[B];
+            uint2 q[B];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (int j = 0; j < B; j++) {
                 const float fd = (float)(d0 + j0 + j);
                 px[j] = a.cam_x + (fd * ca);
                 py[j] = a.cam_y + (fd * sa);
                 q[j] = height_quad<HBITS, HP2>(a.m, px[j], py[j]);
             }
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
+            for (int j = 0; j < B; j++) {
                 float h = height_interp<HBITS>(q[j], px[j], py[j]);
                 h = d0 + j0 + j <= a.n ? h : -INFINITY;
-                hs[wave * kR2Group + j0 + j][lane] = h;
+                hs[wave * G + j0 + j][lane] = h;
                 high = fmaxf(high, h);
             }
         }
         top[wave][lane] = high;
         __syncthreads();
-        const int32_t groups = min(kR2Chunk, a.n + 1 - base + kR2Group - 1) / kR2Group;
+        const int32_t groups = min(16 * G, a.n + 1 - base + G - 1) / G;
         bool pending = false;
 #pragma unroll
         for (int u = 0; u < PX; u++) {
             for (int32_t g = 0; g < groups && hit[u] < 0; g++) {
-                const float f0 = (float)(base + g * kR2Group);
+                const float f0 = (float)(base + g * G);
                 const float t0 = a.cam_h - (f0 * vert_ang[u]);
-                const float t1 = a.cam_h - ((f0 + (float)(kR2Group - 1)) * vert_ang[u]);
+                const float t1 = a.cam_h - ((f0 + (float)(G - 1)) * vert_ang[u]);
                 if (!(fminf(t0, t1) < top[g][lane]))
                     continue;
                 uint32_t below = 0u;
 #pragma unroll
-                for (int j = 0; j < kR2Group; j++)
-                    below |= (a.cam_h - ((f0 + (float)j) * vert_ang[u])) <
-                                     hs[g * kR2Group + j][lane] ? 1u << j : 0u;
+                for (int j = 0; j < G; j++)
+                    below |= (a.cam_h - ((f0 + (float)j) * vert_ang[u])) < hs[g * G + j][lane]
+                                 ? 1u << j : 0u;
                 if (below)
-                    hit[u] = base + g * kR2Group + __builtin_ctz(below);
+                    hit[u] = base + g * G + __builtin_ctz(below);
             }
             pending = pending || hit[u] < 0;
         }
         /* also keeps the next chunk's heights from those still being read */
-        if (!__syncthreads_or(pending))
-            break;
+        return __syncthreads_or(pending);
+    };
+    int32_t base = 0;
+    bool more = a.n >= 0;
+    if constexpr (NEAR) {
+        /* does the first row's line of sight come below the camera's ground
+         * within the short chunk?  Only a guess of where the hits are, so that
+         * one texel will do for the ground */
+        const float vert_lo = (a.horizon / 50.0f) + (((float)(blockIdx.y * ROWS) /
+                                                      ((float)a.rows - 0.0f)) * (1.5f - 1.0f));
+        const uint32_t ground = height_quad<HBITS, HP2>(a.m, a.cam_x, a.cam_y).x &
+                                (HBITS == 8 ? 0xFFu : 0xFFFFu);
+        const bool low = (a.cam_h - ((float)(16 * kR2Near) * vert_lo)) < (float)ground;
+        if (__builtin_amdgcn_readfirstlane(more && low)) {
+            more = march(0, std::integral_constant<int, kR2Near>{});
+            base = 16 * kR2Near;
+        }
     }
+    for (; more && base <= a.n; base += 16 * kR2Group)
+        more = march(base, std::integral_constant<int, kR2Group>{});
     if (a.n < 0)
         __syncthreads();                          /* the squares */
 #pragma unroll
     for (int u = 0; u < PX; u++) {
-        const int32_t y = blockIdx.y * kR2Rows + u * 16 + wave;
+        const int32_t y = blockIdx.y * ROWS + u * 16 + wave;
         if (x >= a.cols || y >= a.rows)
             continue;
         uint32_t c = 0u;
@@ -3160,6 +3186,27 @@ static void launch_diff_grad(const DiffArgs &a, int32_t rows, dim3 grid, hipStre
                        dim3(kGradThreads), 0, s, a);
 }
 
+/* render2 by the workgroups that a frame has: up to one per CU, 32 rows and
+ * all the registers the kernel asks for; more than that, two on a CU (64
+ * registers, which spill a little: 1920 x 1080 67 us instead of 75 per call,
+ * but 160 x 120 41 instead of 39); and 128 rows, which share the heights,
+ * where these still give each CU three and so fill a second round half
+ * (3840 x 2160: 149 us instead of 164, with a camera on the ground 93 instead of
+ * 107; 2900 x 1500, 2.2 per CU: 108 instead of 105). */
+template <int HBITS, bool HP2>
+static int launch_render2(const Render2Args &a, hipStream_t s)
+{
+    const uint32_t tiles = (uint32_t)(a.cols + 63) / 64;
+    const int64_t low = (int64_t)tiles * ((a.rows + 31) / 32);
+    const int64_t tall = (int64_t)tiles * ((a.rows + 127) / 128);
+    const int rows = tall >= 3 * cu_count() ? 128 : 32;
+    void (*kern)(Render2Args) = low <= cu_count() ? k_render2<HBITS, HP2, 32, 4, false>
+                                : rows == 32 ? k_render2<HBITS, HP2, 32, 8, true>
+                                             : k_render2<HBITS, HP2, 128, 8, true>;
+    hipLaunchKernelGGL(kern, dim3(tiles, (a.rows + rows - 1) / rows), dim3(1024), 0, s, a);
+    return hipGetLastError();
+}
+
 extern "C" {
 
 int fsk_device_init(void)
@@ -3521,12 +3568,10 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
     a.n = n;
     a.rows = f->rows;
     a.cols = f->cols;
-    dim3 grid((f->cols + 63) / 64, (f->rows + kR2Rows - 1) / kR2Rows);
     const bool p2 = pow2(m->hrows) && pow2(m->hcols);
-    void (*kern)(Render2Args) = m->hbits == 8 ? (p2 ? k_render2<8, true> : k_render2<8, false>)
-                                              : (p2 ? k_render2<16, true> : k_render2<16, false>);
-    hipLaunchKernelGGL(kern, grid, dim3(1024), 0, s, a);
-    return hipGetLastError();
+    if (m->hbits == 8)
+        return p2 ? launch_render2<8, true>(a, s) : launch_render2<8, false>(a, s);
+    return p2 ? launch_render2<16, true>(a, s) : launch_render2<16, false>(a, s);
 }
 
 float fsk_wrap_recip(int32_t m)

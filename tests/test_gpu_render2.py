@@ -92,3 +92,28 @@ def test_render2_steps_and_tiles(ctx, distance, h, w, horizon, bits):
         got = ctx.render2(m, v)
         bad = int(np.count_nonzero(got != want))
         assert bad == 0, f"{bad} of {got.size} pixels differ"
+
+
+@pytest.mark.parametrize("h,w,distance,bits,cols", [
+    (40, 70, 252.0, 8, 128), (40, 70, 256.0, 16, 96), (33, 65, 700.0, 8, 96),   # a workgroup per CU
+    (35, 16640, 20.0, 8, 96), (3, 16640, 280.0, 16, 128),                       # two per CU
+    (3, 49200, 260.0, 8, 128), (129, 24640, 24.0, 16, 96),                      # 128 rows
+])
+def test_render2_of_low_cameras(ctx, h, w, distance, bits, cols):
+    """Cameras in, on and little above the ground, level and steep, whose hits
+    lie before, in and after the short first chunk, in each of the kernel's
+    shapes."""
+    top = 255 if bits == 8 else 900
+    hts = scene.heightmap(33, 128, 0.6, top)
+    col = scene.colormap(33, hts, top)[:, :cols].copy()
+    hts = np.ascontiguousarray(hts[:, :cols])
+    m = ctx.map(col, hts, height_bits=bits)
+    alt = np.asarray(hts, np.int32) & (255 if bits == 8 else 0xFFFF)
+    cases = [(-5.0, 3.0), (0.5, 60.0), (9.0, 20.0), (30.0, 4.0)]
+    for above, horizon in cases if h * w < 1 << 20 else cases[1:2]:
+        v = View(x=40.2, y=77.9, height=float(hts[77, 40] + above), angle=2.2, horizon=horizon,
+                 distance=distance, h=h, w=w)
+        want = O.render2(v, col, alt)
+        got = ctx.render2(m, v)
+        bad = int(np.count_nonzero(got != want))
+        assert bad == 0, f"{above} {horizon}: {bad} of {got.size} pixels differ"
