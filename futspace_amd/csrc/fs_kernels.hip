@@ -1615,7 +1615,7 @@ __global__ void k_color_quads(const uint32_t *__restrict__ c, int32_t rows, int3
  * non-decreasing in t for a fixed probe, also in f32, so once it is at least
  * -0.5 against the map's largest height no later step can count, and the
  * wave leaves when that holds for its lowest texel (at sun height 0.1
- * after at most 64 of the 255 steps on an 8-bit map).  Measured, sun height
+ * after at most 65 of the 255 steps on an 8-bit map).  Measured, sun height
  * 0.1: 1024^2 grid 338 -> 25 us; 4096^2 grid, heights to 1024 (nearly every
  * step) 4.79 -> 0.64 ms, where the vector instructions bound it; before,
  * one texel per thread took every step with two general floor-mods. */
@@ -1655,7 +1655,8 @@ __device__ __forceinline__ int32_t wrap_map(int32_t v, int32_t m, float rm)
 }
 
 /* WRAP kWrapX86 is for sun vectors that are not finite, whose probes take
- * the x86 cast's INT_MIN; a finite sun's offsets are at most 1020. */
+ * the x86 cast's INT_MIN (a finite sun's offsets are at most 1020), and for
+ * map sides or grids above 2^16. */
 template <int WRAP, bool FACTOR>
 __global__ __launch_bounds__(256) void k_shade(ShadeArgs a)
 {
@@ -3577,7 +3578,8 @@ int fsk_render2(const fsk_map *m, const fsk_frame *f, const float *d_cs, const f
 float fsk_wrap_recip(int32_t m)
 {
     /* at most (1 - 2^-24) / m, so that its product with v, rounded, is not
-     * above v / m, and at least (1 - 2^-22) / m */
+     * above v / m, and at least (1 - 2^-21.6) / m (the least over the sides up
+     * to 2^20 is (1 - 2^-21.68) / m, at 1047899) */
     const float r = 1.0f / (float)m;
     return nextafterf(nextafterf(r, 0.0f), 0.0f);
 }
