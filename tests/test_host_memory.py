@@ -95,6 +95,8 @@ def test_buffers_read_elsewhere_are_freed_and_not_reused(lib, contexts, call, wh
     stream alone reads is kept for the next load."""
     a, b = contexts
     m = a.map()
+    if where == "graph":
+        assert lib.fsx_context_stream(a.ptr)      # as who captures it has to
     _set(lib, "stub_capturing", int(where == "graph"), ctypes.c_int)
     assert _readers(lib, b if where == "other" else a, m)[call]() == 0
     _set(lib, "stub_capturing", 0, ctypes.c_int)
@@ -103,6 +105,21 @@ def test_buffers_read_elsewhere_are_freed_and_not_reused(lib, contexts, call, wh
     freed = _get(lib, "stub_frees") - frees
     # only render reads the shade's two buffers as well
     assert freed == (0 if where == "own" else MAP_BUFFERS if call == "render" else 3)
+
+
+def test_buffers_read_on_a_callers_stream_under_capture_are_freed(lib, contexts):
+    """A context moved onto a caller's stream, which the caller captures."""
+    a = contexts[0]
+    m = a.map()
+    own = ctypes.create_string_buffer(8)
+    assert lib.fsx_context_set_stream(a.ptr, ctypes.addressof(own)) == 0
+    _set(lib, "stub_capturing", 1, ctypes.c_int)
+    assert _readers(lib, a, m)["render"]() == 0
+    _set(lib, "stub_capturing", 0, ctypes.c_int)
+    assert lib.fsx_context_set_stream(a.ptr, None) == 0
+    frees = _get(lib, "stub_frees")
+    a.free(m)
+    assert _get(lib, "stub_frees") - frees == MAP_BUFFERS
 
 
 def test_a_map_freed_through_another_context_leaves_no_pool(lib, contexts):
@@ -145,6 +162,7 @@ def test_a_shade_that_a_captured_graph_writes_is_freed_and_not_reused(lib, conte
     assert lib.futhark_entry_update_map(a.ptr, ctypes.byref(loaded), ctypes.c_void_p(col),
                                         ctypes.c_void_p(hts), init) == 0
     assert lib.futhark_entry_key(a.ptr, ctypes.byref(keyed), 0, ord("u"), loaded) == 0
+    assert lib.fsx_context_stream(a.ptr)
     _set(lib, "stub_capturing", 1, ctypes.c_int)
     assert lib.futhark_entry_step(a.ptr, ctypes.byref(stepped), 0.016, keyed) == 0
     _set(lib, "stub_capturing", 0, ctypes.c_int)
