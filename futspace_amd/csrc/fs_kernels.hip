@@ -2754,7 +2754,7 @@ __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval 
  * cancels), likewise for the other texels, 0 where px == 0.  A wave loops over
  * its lanes' runs, every lane at its next one wherever that starts: row by
  * row, a wave evaluated and inserted on each row where any lane began a run
- * (0.94 of a 4K view's rows; now 0.66 evaluations per row, 54 M instead of
+ * (0.94 of a 4K view's rows; now 0.66 evaluations per row, 51 M instead of
  * 70 M vector instructions).  The texel terms are summed in two stages before
  * any global atomic: lanes of a wave whose runs hit the same texels (adjacent
  * columns magnifying one near texel) are merged by a segmented reduction
@@ -2766,7 +2766,7 @@ __device__ __forceinline__ void sample_grad(const DiffArgs &a, const SampleEval 
  * added into the global f32 gradient with one atomic per channel.
  *
  * What bounds it: in large frames the vector instructions (3840 x 2160 fitting
- * view 127 -> 92 us); in small ones the inserts and the flush's atomics, with
+ * view 127 -> 89 us); in small ones the inserts and the flush's atomics, with
  * the latency of a block's chain behind them (1280 x 720: 51 -> 46 us, 24
  * without inserts; 800 x 600 vjp 32 -> 26 us).
  *

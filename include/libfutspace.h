@@ -190,7 +190,9 @@ int fsx_render_batch(struct futhark_context *ctx, const struct fsx_map *const *m
  * number of times.  fsx_batch_run enqueues it on the context stream;
  * fsx_batch_capture records that launch into a HIP graph once and
  * fsx_batch_replay relaunches the graph.  The batch holds references to
- * its maps; the output buffer must outlive it. */
+ * its maps; the output buffer must outlive it.  Launches of one batch that
+ * overlap on several streams share its work: every view is rendered when all
+ * of them have ended. */
 struct fsx_batch;
 int fsx_batch_new(struct futhark_context *ctx, const struct fsx_map *const *maps, int32_t n_maps,
                   const struct fsx_view *views, int32_t n_views, uint32_t *dev_out,
