@@ -2132,10 +2132,13 @@ struct BatchArgs {
  * Launches of one batch that overlap (two contexts, or an eager launch beside
  * a replay) share the counters: between them they hand out every item, some
  * of them twice, with the same pixels.  The ended workgroups are counted over
- * all of them and the count is lowered by a launch's worth, not cleared, so
- * that none is lost; the last of all to end finds a whole number of launches
- * and leaves the counters reset.  Atomic stores, since a plain one would
- * reach memory when its launch ends, maybe over another's claims. */
+ * all of them by an atomic that wraps at a launch's worth, so that none is
+ * lost; the last of all to end finds a whole number of launches and leaves the
+ * counters reset.  A reset that reaches memory late, when its launch ends, over
+ * the claims of another only has items handed out again, and that one's own end
+ * resets the counters after it.  Resets by agent-scope stores, with the count
+ * lowered by a second atomic, kept a launch's last workgroup and so the next
+ * launch waiting: 0.3 to 1 us of a batch of 13 to 40 us. */
 __host__ __device__ constexpr uint32_t batch_first_claim(uint32_t grid, uint32_t q, uint32_t nq)
 {
     return (grid + nq - 1u - q) / nq;      /* workgroups that start on queue q */
@@ -2201,12 +2204,9 @@ __global__ __launch_bounds__(NT, WPE) void k_render_batch(BatchArgs b)
     }
     if (threadIdx.x == 0) {
         uint32_t *ended = b.counters + nq * FSK_COUNTER_STRIDE;
-        if (atomicAdd(ended, 1u) % gridDim.x == gridDim.x - 1u) {
+        if (atomicInc(ended, gridDim.x - 1u) == gridDim.x - 1u) {
             for (uint32_t i = 0; i < nq; i++)
-                __hip_atomic_store(b.counters + i * FSK_COUNTER_STRIDE,
-                                   batch_first_claim(gridDim.x, i, nq), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            atomicSub(ended, gridDim.x);
+                b.counters[i * FSK_COUNTER_STRIDE] = batch_first_claim(gridDim.x, i, nq);
         }
     }
 }
